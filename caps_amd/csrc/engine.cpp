@@ -23,6 +23,7 @@
 #include "engine.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 
 #include "crt.h"
@@ -707,7 +708,9 @@ MergeKey merge_key(const Plan &plan, const Step &st) {
     case STEP_EW: k = {STEP_MULTI_EW, st.op, st.vec2}; break;
     case STEP_REW: k = {STEP_MULTI_REW, st.op, st.vec2}; break;
     case STEP_GEMM_F64:
-      k = {STEP_MULTI_GEMM, dgemm_block_tile((int)st.n, st.levels, st.tile), 0};
+      // the block tile of a launch that fills the device (emit_merged looks
+      // at the tiles there are)
+      k = {STEP_MULTI_GEMM, dgemm_block_tile((int)st.n, st.levels, st.tile, 1LL << 24), 0};
       break;
     case STEP_OZ_GEMM: {
       // INT8 products that would take the 128 x 128 kernel alone; those on
@@ -791,6 +794,24 @@ void emit_merged(Plan &plan, const MergeKey &k, const std::vector<const Step *> 
     }
     return;
   }
+  // FP64 products: a smaller block tile where all heads together leave the
+  // device idle
+  int bt = k.a;
+  if (k.kind == STEP_MULTI_GEMM && heads[0]->tile == 0) {
+    double cost = INFINITY;
+    for (int b = k.a; b >= 32; b /= 2) {
+      double tiles = 0;
+      for (const Step *st : heads) {
+        const double t = (double)((st->n + b - 1) / b);
+        tiles += t * t * st->count;
+      }
+      const double c = dgemm_tile_cost(b, tiles);
+      if (c < cost) {
+        bt = b;
+        cost = c;
+      }
+    }
+  }
   std::vector<VSeg> segs;
   long long total = 0;
   for (const Step *st : heads) {
@@ -804,7 +825,7 @@ void emit_merged(Plan &plan, const MergeKey &k, const std::vector<const Step *> 
       rew_grid(st->count, st->n, moduli, st->vec2 != 0, v.gx, v.gy);
       v.aux = moduli;
     } else if (k.kind == STEP_MULTI_GEMM) {
-      const int m = (int)st->n, bt = k.a;
+      const int m = (int)st->n;
       v.gx = (m + bt - 1) / bt;
       v.gy = st->count;
       v.aux = st->levels | (((m >> st->levels) % bt != 0) << 8);
@@ -823,7 +844,7 @@ void emit_merged(Plan &plan, const MergeKey &k, const std::vector<const Step *> 
   const size_t off = push_segs(plan, segs);
   // op: the Winograd op of an add step; flag: 16/4-byte accesses (adds) or
   // the FP64 block tile
-  plan.steps.push_back(multi_step(k.kind, k.a, k.kind == STEP_MULTI_GEMM ? k.a : k.b, segs,
+  plan.steps.push_back(multi_step(k.kind, k.a, k.kind == STEP_MULTI_GEMM ? bt : k.b, segs,
                                   total, off));
 }
 

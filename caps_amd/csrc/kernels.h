@@ -62,9 +62,15 @@ struct GemmPtrs {
 // quadtrees of `levels` quadrant levels over column-major leaves of size
 // m >> levels (levels = 0: plain column-major; levels > 0 needs leaves that
 // are multiples of 128).  One persistent launch over all tiles of all problems.
-// tile: 0 = 128 x 128 block tiles, 1 = 64 x 64.
+// tile: 0 = the block tile of dgemm_block_tile, 1 = 64 x 64.
 hipError_t launch_dgemm_batched(const GemmPtrs *d_tab, int count, int m, int levels, int tile,
                                 hipStream_t s);
+
+// The block tile (128, 64 or 32) of `count` products of order m: the one that
+// keeps the device busiest.  dgemm_tile_cost is its estimate for a launch of
+// `tiles` tiles.
+int dgemm_block_tile(int m, int levels, int tile, long long count);
+double dgemm_tile_cost(int bt, double tiles);
 
 int device_cu_count();
 
@@ -93,8 +99,7 @@ __device__ __forceinline__ int vseg_find(const VSeg *__restrict__ segs, int nseg
 // FP64 leaf GEMMs over segments of different sizes, one persistent launch:
 // segment args are GemmPtrs tables, n = order, gx = tiles per dimension, gy =
 // problems, blk0 = first global tile, aux = quadtree levels | edge checks <<
-// 8.  bt: block tile (dgemm_block_tile).
-int dgemm_block_tile(int m, int levels, int tile);
+// 8.  bt: block tile.
 hipError_t launch_dgemm_multi(int bt, const char *d_tables, const VSeg *d_segs, int nseg,
                               int total_tiles, hipStream_t s);
 
