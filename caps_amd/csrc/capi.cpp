@@ -27,7 +27,14 @@
 // on holds its own copy from module load until the process ends.  Host code
 // never uses this name as an address: the per-device address comes from
 // hipGetSymbolAddress (State::scratch).
-static __device__ __align__(256) char scratch[(size_t)CAPS_NOALLOC_SCRATCH_MIB << 20];
+//
+// CAPS_NOALLOC_SCRATCH_MIB limits a plan's tables and workspace counted
+// without the padding of residue leaves to a 16-byte pitch.  From leaves of 17
+// up the pitch adds at most 15 / 17, so twice the limit holds every plan that
+// passes; smaller leaves (orders up to 1920 with at most 7 levels) that do not
+// fit with it run fewer levels batched.
+constexpr size_t SCRATCH_BYTES = (size_t)(2 * CAPS_NOALLOC_SCRATCH_MIB) << 20;
+static __device__ __align__(256) char scratch[SCRATCH_BYTES];
 
 namespace caps {
 
@@ -477,16 +484,33 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
   if (!p) {
     auto plan = std::make_unique<Plan>();
     plan->key = key;
-    if (build_plan(*plan, dA, dB, dC, *desc, pat, mode, moduli, cutoff, nullptr, fuse, tile) !=
-        CAPS_OK)
+    auto size_of = [&](const std::string &p, bool pad, size_t &tables, size_t &total) {
+      int r = build_plan(*plan, dA, dB, dC, *desc, p, mode, moduli, cutoff, nullptr, fuse, tile,
+                         pad);
+      tables = (plan->host_tables.size() + 255) / 256 * 256;
+      total = tables + plan->work_bytes;
+      return r;
+    };
+    size_t toff = 0, need = 0;
+    if (size_of(pat, false, toff, need) != CAPS_OK)
       return fail(CAPS_EINVAL, "internal: plan layout check failed");
-    const size_t toff = (plan->host_tables.size() + 255) / 256 * 256;
-    if (toff + plan->work_bytes > cap)
+    if (need > cap)
       return fail(CAPS_ENOMEM,
                   "plan needs %.1f MiB of tables and workspace; caps_multiply_device_noalloc "
                   "has %d MiB of scratch",
-                  (toff + plan->work_bytes) / 1048576.0, CAPS_NOALLOC_SCRATCH_MIB);
-    if (build_plan(*plan, dA, dB, dC, *desc, pat, mode, moduli, cutoff, base + toff, fuse,
+                  need / 1048576.0, CAPS_NOALLOC_SCRATCH_MIB);
+    // with the residue pitch: where that does not fit, levels run recursively
+    // from the bottom up (the same bits)
+    std::string run = pat;
+    for (size_t l = pat.size();; l--) {
+      if (size_of(run, true, toff, need) != CAPS_OK)
+        return fail(CAPS_EINVAL, "internal: plan layout check failed");
+      if (need <= SCRATCH_BYTES) break;
+      if (l == 0)
+        return fail(CAPS_ENOMEM, "plan needs %.1f MiB of padded workspace", need / 1048576.0);
+      run[l - 1] = 'd';
+    }
+    if (build_plan(*plan, dA, dB, dC, *desc, run, mode, moduli, cutoff, base + toff, fuse,
                    tile) != CAPS_OK ||
         (plan->host_tables.size() + 255) / 256 * 256 != toff)
       return fail(CAPS_EINVAL, "internal: plan layout check failed");

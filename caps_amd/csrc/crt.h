@@ -28,9 +28,10 @@ struct CrtMats {
   const double *A;  // n x n CAPS layout (nrec, bs)
   const double *B;
   double *C;
-  int8_t *ra;  // residues of A': nmod planes of n*n bytes, leaves row-major
+  int8_t *ra;  // residues of A': nmod planes of `plane` bytes, leaves row-major
   int8_t *rb;  // residues of B': leaves column-major
   int8_t *rc;  // residues of C': leaves column-major
+  long long plane;  // 4^nrec leaves of residue_area(m) bytes
   int *sa;     // n row exponents of A
   int *sb;     // n column exponents of B
   double *pa;  // row partials (e, s) of A: [2^nrec * chunks][n] pairs
@@ -67,7 +68,7 @@ enum CrtKernel : int {
   CRT_RECON = 5
 };
 // the grid kernel k has for one item alone (gx x gy) and its template flag
-// (column-major leaves / aligned sizes); items merged in one launch share it
+// (column-major leaves); items merged in one launch share it
 bool crt_grid(int k, const CrtMats &h, int &gx, int &gy);
 hipError_t launch_crt_multi(int k, bool flag, int np, const char *d_tables, const VSeg *d_segs,
                             int nseg, int blocks, const OzakiConsts *d_consts, hipStream_t s);

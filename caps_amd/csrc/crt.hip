@@ -123,98 +123,72 @@ __global__ __launch_bounds__(T) void crt_finalize_kernel(const CrtMats *__restri
 }
 
 // ------------------------------------------------------------------ split
-// A leaf L -> row-major residue leaves, transposed through LDS.
-// FAST (m % 64 == 0 and the leaf column-major, bs == 1 or bs == m): tiles of
-// 32 rows x 128 k; the column-major side moves as 256-byte column pieces, the
-// row-major side as 128-byte row pieces (8 lanes x 16 residues), K chunks past
-// m (m % 128 == 64) skipped.  Column c of the tile in T2[c], row r at slot r ^
-// tswz(c); the transposed read has lanes on 8 rows and 8 column groups, the
-// swizzle puts 4 of the groups 8 slots apart (the other 4 pairs share a
-// slot: a 64-lane 8-byte read spans at least two 256-byte passes anyway).
-// Otherwise 64 x 64 tiles with checked, element-wise accesses.
+// A leaf L -> row-major residue leaves, transposed through LDS: tiles of 32
+// rows x 128 k.  PLAIN (the leaf column-major, bs == 1 or bs == m): the
+// column-major side moves as 256-byte column pieces; the row-major side moves
+// as 128-byte row pieces (8 lanes x 16 residues).  Elements past m are zero,
+// 16-byte chunks past the pitch skipped.  Column c of the tile in T2[c], row r
+// at slot r ^ tswz(c); the transposed read has lanes on 8 rows and 8 column
+// groups, the swizzle puts 4 of the groups 8 slots apart (the other 4 pairs
+// share a slot: a 64-lane 8-byte read spans at least two 256-byte passes
+// anyway).
+constexpr int SPLIT_R = 32, SPLIT_K = 128;
 __device__ __forceinline__ int tswz(int c) { return ((c >> 4) & 3) << 3; }
 
-template <bool FAST>
+template <bool PLAIN>
 __device__ __forceinline__ void split_a_body(const CrtMats *__restrict__ M,
                                              const OzakiConsts *__restrict__ kc, int bx, int by,
-                                             double (&Ts)[64][64]) {
+                                             double (&T2)[SPLIT_K][SPLIT_R]) {
   const int m = M->m, nmod = M->nmod, bs = M->bs;
   const int L = by;
   int bi, bj;
   leaf_coords(L, M->nrec, bi, bj);
-  const long long lbase = (long long)L * m * m;
-  const long long plane = (long long)M->n * M->n;
-  if (FAST) {
-    double(*T2)[32] = reinterpret_cast<double(*)[32]>(&Ts[0][0]);  // [128 k][32 rows]
-    const int tk = (m + 127) / 128;
-    const int r0 = (bx / tk) * 32, k0 = (bx % tk) * 128;
-    for (int idx = threadIdx.x; idx < 32 * 128; idx += T) {
-      const int r = idx & 31, c = idx >> 5;
-      const int lj = k0 + c;
-      T2[c][r ^ tswz(c)] = lj < m ? M->A[lbase + r0 + r + (long long)lj * m] : 0.0;
-    }
-    __syncthreads();
-    const int r = threadIdx.x >> 3, kq = (threadIdx.x & 7) * 16;
-    if (k0 + kq >= m) return;  // m % 16 == 0: the chunk is wholly past the leaf
-    const int li = r0 + r;
-    const int sa = M->sa[bi * m + li];
-    double x[16];
-#pragma unroll
-    for (int c = 0; c < 16; c++) x[c] = trunc(ldexp(T2[kq + c][r ^ tswz(kq)], sa));
-    int8_t *dst = M->ra + lbase + (long long)li * m + k0 + kq;
-    for (int l = 0; l < nmod; l++) {
-      const int mi = kc->m[l];
-      const double inv = kc->inv_m[l];
-      const int c22 = kc->c22[l];
-      unsigned w[4];
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-        w[q] = pack4_lo(sym_residue(x[4 * q], mi, inv, c22),
-                        sym_residue(x[4 * q + 1], mi, inv, c22),
-                        sym_residue(x[4 * q + 2], mi, inv, c22),
-                        sym_residue(x[4 * q + 3], mi, inv, c22));
-      *reinterpret_cast<uint4 *>(dst + l * plane) = make_uint4(w[0], w[1], w[2], w[3]);
-    }
-    return;
-  }
-  const int tiles = (m + 63) / 64;
-  const int r0 = (bx % tiles) * 64, k0 = (bx / tiles) * 64;
-  for (int idx = threadIdx.x; idx < 64 * 64; idx += T) {
-    const int r = idx & 63, c = idx >> 6;
+  const double *A = M->A + (long long)L * m * m;
+  const long long plane = M->plane;
+  const int tk = (m + SPLIT_K - 1) / SPLIT_K;
+  const int r0 = (bx / tk) * SPLIT_R, k0 = (bx % tk) * SPLIT_K;
+  for (int idx = threadIdx.x; idx < SPLIT_R * SPLIT_K; idx += T) {
+    const int r = idx & 31, c = idx >> 5;
     const int li = r0 + r, lj = k0 + c;
     double v = 0.0;
-    if (li < m && lj < m) v = M->A[lbase + leaf_elem_offset(m, bs, li, lj)];
-    Ts[c][r ^ tswz(c)] = v;
+    if (li < m && lj < m)
+      v = A[PLAIN ? li + (long long)lj * m : leaf_elem_offset(m, bs, li, lj)];
+    T2[c][r ^ tswz(c)] = v;
   }
   __syncthreads();
-  const int r = threadIdx.x >> 2, kq = (threadIdx.x & 3) * 16;
+  const int r = threadIdx.x >> 3, kq = (threadIdx.x & 7) * 16;
   const int li = r0 + r;
-  if (li >= m) return;
+  if (li >= m || k0 + kq >= m) return;
   const int sa = M->sa[bi * m + li];
   double x[16];
 #pragma unroll
-  for (int c = 0; c < 16; c++) x[c] = trunc(ldexp(Ts[kq + c][r ^ tswz(kq)], sa));
-  int8_t *dst = M->ra + lbase + (long long)li * m + k0 + kq;
+  for (int c = 0; c < 16; c++) x[c] = trunc(ldexp(T2[kq + c][r ^ tswz(kq)], sa));
+  int8_t *dst = M->ra + L * residue_area(m) + (long long)li * residue_pitch(m) + k0 + kq;
   for (int l = 0; l < nmod; l++) {
     const int mi = kc->m[l];
     const double inv = kc->inv_m[l];
     const int c22 = kc->c22[l];
+    unsigned w[4];
 #pragma unroll
-    for (int c = 0; c < 16; c++)
-      if (k0 + kq + c < m) dst[l * plane + c] = (int8_t)sym_residue(x[c], mi, inv, c22);
+    for (int q = 0; q < 4; q++)
+      w[q] = pack4_lo(sym_residue(x[4 * q], mi, inv, c22),
+                      sym_residue(x[4 * q + 1], mi, inv, c22),
+                      sym_residue(x[4 * q + 2], mi, inv, c22),
+                      sym_residue(x[4 * q + 3], mi, inv, c22));
+    *reinterpret_cast<uint4 *>(dst + l * plane) = make_uint4(w[0], w[1], w[2], w[3]);
   }
 }
 
-template <bool FAST>
+template <bool PLAIN>
 __global__ __launch_bounds__(T) void crt_split_a_kernel(const CrtMats *__restrict__ M,
                                                         const OzakiConsts *__restrict__ kc) {
-  __shared__ double Ts[64][64];  // [col][swizzled row]
-  split_a_body<FAST>(M, kc, blockIdx.x, blockIdx.y, Ts);
+  __shared__ double Ts[SPLIT_K][SPLIT_R];  // [col][swizzled row]
+  split_a_body<PLAIN>(M, kc, blockIdx.x, blockIdx.y, Ts);
 }
 
-// B leaf L -> column-major residue leaves; thread per 16 consecutive rows.
-// FAST: m % 16 == 0 and the leaf is column-major.
-template <bool FAST>
+// B leaf L -> column-major residue leaves; thread per 16 consecutive rows of a
+// column (rows past m are zero).  PLAIN: the leaf is column-major.
+template <bool PLAIN>
 __device__ __forceinline__ void split_b_body(const CrtMats *__restrict__ M,
                                              const OzakiConsts *__restrict__ kc, int bx, int by,
                                              int gx) {
@@ -222,57 +196,52 @@ __device__ __forceinline__ void split_b_body(const CrtMats *__restrict__ M,
   const int L = by;
   int bi, bj;
   leaf_coords(L, M->nrec, bi, bj);
-  const long long lbase = (long long)L * m * m;
-  const long long mm = (long long)m * m;
-  const long long plane = (long long)M->n * M->n;
-  const long long units = FAST ? mm / 16 : mm;
+  const double *B = M->B + (long long)L * m * m;
+  int8_t *rb = M->rb + L * residue_area(m);
+  const long long plane = M->plane;
+  const int c16 = residue_pitch(m) / 16;
+  const long long units = (long long)m * c16;
   for (long long u = (long long)bx * T + threadIdx.x; u < units; u += (long long)gx * T) {
-    if (FAST) {
-      const long long e0 = u * 16;
-      const int lj = (int)(e0 / m);
-      const int s = M->sb[bj * m + lj];
-      double x[16];
-#pragma unroll
-      for (int c = 0; c < 16; c += 2) {
-        double2 v = *reinterpret_cast<const double2 *>(M->B + lbase + e0 + c);
-        x[c] = trunc(ldexp(v.x, s));
-        x[c + 1] = trunc(ldexp(v.y, s));
-      }
-      for (int l = 0; l < nmod; l++) {
-        const int mi = kc->m[l];
-        const double inv = kc->inv_m[l];
-        const int c22 = kc->c22[l];
-        unsigned w[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          unsigned v = 0;
-#pragma unroll
-          for (int b = 0; b < 4; b++)
-            v |= (unsigned)(sym_residue(x[4 * q + b], mi, inv, c22) & 0xff) << (8 * b);
-          w[q] = v;
-        }
-        *reinterpret_cast<uint4 *>(M->rb + l * plane + lbase + e0) =
-            make_uint4(w[0], w[1], w[2], w[3]);
-      }
+    const int lj = (int)(u / c16), li = (int)(u - (long long)lj * c16) * 16;
+    const int s = M->sb[bj * m + lj];
+    double x[16];
+    if (PLAIN) {
+      load_rows16(B + (long long)lj * m + li, m - li, x);
     } else {
-      const int li = (int)(u % m), lj = (int)(u / m);
-      const double x = trunc(ldexp(M->B[lbase + leaf_elem_offset(m, bs, li, lj)],
-                                   M->sb[bj * m + lj]));
-      for (int l = 0; l < nmod; l++)
-        M->rb[l * plane + lbase + u] = (int8_t)sym_residue(x, kc->m[l], kc->inv_m[l], kc->c22[l]);
+#pragma unroll
+      for (int c = 0; c < 16; c++)
+        x[c] = li + c < m ? B[leaf_elem_offset(m, bs, li + c, lj)] : 0.0;
+    }
+#pragma unroll
+    for (int c = 0; c < 16; c++) x[c] = trunc(ldexp(x[c], s));
+    for (int l = 0; l < nmod; l++) {
+      const int mi = kc->m[l];
+      const double inv = kc->inv_m[l];
+      const int c22 = kc->c22[l];
+      unsigned w[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        unsigned v = 0;
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+          v |= (unsigned)(sym_residue(x[4 * q + b], mi, inv, c22) & 0xff) << (8 * b);
+        w[q] = v;
+      }
+      *reinterpret_cast<uint4 *>(rb + l * plane + 16 * u) = make_uint4(w[0], w[1], w[2], w[3]);
     }
   }
 }
 
-template <bool FAST>
+template <bool PLAIN>
 __global__ __launch_bounds__(T) void crt_split_b_kernel(const CrtMats *__restrict__ M,
                                                         const OzakiConsts *__restrict__ kc) {
-  split_b_body<FAST>(M, kc, blockIdx.x, blockIdx.y, gridDim.x);
+  split_b_body<PLAIN>(M, kc, blockIdx.x, blockIdx.y, gridDim.x);
 }
 
 // ------------------------------------------------------------------ reconstruct
-// C' residues (column-major leaves) -> C (CAPS layout, bs blocks)
-template <int NP, bool FAST>
+// C' residues (column-major leaves) -> C (CAPS layout, bs blocks); thread: 4
+// consecutive rows of a column.  PLAIN: the leaf of C is column-major.
+template <int NP, bool PLAIN>
 __device__ __forceinline__ void recon_body(const CrtMats *__restrict__ M,
                                            const OzakiConsts *__restrict__ kc, int bx, int by,
                                            int gx) {
@@ -280,48 +249,47 @@ __device__ __forceinline__ void recon_body(const CrtMats *__restrict__ M,
   const int L = by;
   int bi, bj;
   leaf_coords(L, M->nrec, bi, bj);
-  const long long lbase = (long long)L * m * m;
-  const long long mm = (long long)m * m;
-  const long long plane = (long long)M->n * M->n;
-  const int per = FAST ? 4 : 1;
-  const long long units = mm / per;
+  double *C = M->C + (long long)L * m * m;
+  const int8_t *rc = M->rc + L * residue_area(m);
+  const long long plane = M->plane;
+  const int ld = residue_pitch(m), w4 = (m + 3) / 4;  // words of a column with rows below m
+  const long long units = (long long)m * w4;
   for (long long u = (long long)bx * T + threadIdx.x; u < units; u += (long long)gx * T) {
-    const long long e0 = u * per;
-    const int li = (int)(e0 % m), lj = (int)(e0 / m);
+    const int lj = (int)(u / w4), li = (int)(u - (long long)lj * w4) * 4;
     const int sb = M->sb[bj * m + lj];
-    if (FAST) {
-      double S[4][NP];
+    const int *sa = M->sa + bi * m + li;
+    double S[4][NP];
 #pragma unroll
-      for (int q = 0; q < 4; q++)
+    for (int q = 0; q < 4; q++)
 #pragma unroll
-        for (int p = 0; p < NP; p++) S[q][p] = 0.0;
-      for (int l = 0; l < nmod; l++) {
-        const unsigned w = *reinterpret_cast<const unsigned *>(M->rc + l * plane + lbase + e0);
+      for (int p = 0; p < NP; p++) S[q][p] = 0.0;
+    for (int l = 0; l < nmod; l++) {
+      const unsigned w =
+          *reinterpret_cast<const unsigned *>(rc + l * plane + (long long)lj * ld + li);
 #pragma unroll
-        for (int q = 0; q < 4; q++) crt_acc<NP>(S[q], (int)(int8_t)((w >> (8 * q)) & 0xff), l, kc);
-      }
+      for (int q = 0; q < 4; q++) crt_acc<NP>(S[q], (int)(int8_t)((w >> (8 * q)) & 0xff), l, kc);
+    }
+    if (PLAIN && m % 4 == 0) {
       double out[4];
 #pragma unroll
-      for (int q = 0; q < 4; q++)
-        out[q] = ldexp(crt_finish<NP>(S[q], kc), -(M->sa[bi * m + li + q] + sb));
-      double2 *dst = reinterpret_cast<double2 *>(M->C + lbase + e0);
+      for (int q = 0; q < 4; q++) out[q] = ldexp(crt_finish<NP>(S[q], kc), -(sa[q] + sb));
+      double2 *dst = reinterpret_cast<double2 *>(C + (long long)lj * m + li);
       dst[0] = make_double2(out[0], out[1]);
       dst[1] = make_double2(out[2], out[3]);
     } else {
-      double S[NP];
 #pragma unroll
-      for (int p = 0; p < NP; p++) S[p] = 0.0;
-      for (int l = 0; l < nmod; l++) crt_acc<NP>(S, (int)M->rc[l * plane + lbase + e0], l, kc);
-      M->C[lbase + leaf_elem_offset(m, bs, li, lj)] =
-          ldexp(crt_finish<NP>(S, kc), -(M->sa[bi * m + li] + sb));
+      for (int q = 0; q < 4; q++)
+        if (li + q < m)
+          C[PLAIN ? (long long)lj * m + li + q : leaf_elem_offset(m, bs, li + q, lj)] =
+              ldexp(crt_finish<NP>(S[q], kc), -(sa[q] + sb));
     }
   }
 }
 
-template <int NP, bool FAST>
+template <int NP, bool PLAIN>
 __global__ __launch_bounds__(T) void crt_recon_kernel(const CrtMats *__restrict__ M,
                                                       const OzakiConsts *__restrict__ kc) {
-  recon_body<NP, FAST>(M, kc, blockIdx.x, blockIdx.y, gridDim.x);
+  recon_body<NP, PLAIN>(M, kc, blockIdx.x, blockIdx.y, gridDim.x);
 }
 
 // ------------------------------------------------------------------ segmented CRT steps
@@ -331,7 +299,7 @@ template <int K, bool F, int NP>
 __global__ __launch_bounds__(T) void crt_multi_kernel(const char *__restrict__ base,
                                                       const VSeg *__restrict__ segs, int nseg,
                                                       const OzakiConsts *__restrict__ kc) {
-  __shared__ double Ts[K == CRT_SPLIT_A ? 64 : 1][K == CRT_SPLIT_A ? 64 : 1];
+  __shared__ double Ts[K == CRT_SPLIT_A ? SPLIT_K : 1][K == CRT_SPLIT_A ? SPLIT_R : 1];
   const VSeg &S = segs[vseg_find(segs, nseg, blockIdx.x)];
   const int l = blockIdx.x - S.blk0;
   const int bx = l % S.gx, by = l / S.gx;
@@ -494,7 +462,6 @@ bool crt_grid(int k, const CrtMats &h, int &gx, int &gy) {
   const int leaves = 1 << (2 * h.nrec);
   const int nblk = 1 << h.nrec;
   const bool plain = (h.bs == 1 || h.bs == h.m);
-  const long long mm = (long long)h.m * h.m;
   gy = 1;
   switch (k) {
     case CRT_ROWPART:
@@ -507,26 +474,18 @@ bool crt_grid(int k, const CrtMats &h, int &gx, int &gy) {
     case CRT_FINALIZE:
       gx = (h.n + T - 1) / T;
       return false;
-    case CRT_SPLIT_A: {
-      const bool fast = plain && h.m % 64 == 0;
-      const int tiles = (h.m + 63) / 64;
-      // fast: 32-row x 128-k tiles; else 64 x 64
-      gx = fast ? (h.m / 32) * ((h.m + 127) / 128) : tiles * tiles;
+    case CRT_SPLIT_A:
+      gx = ((h.m + SPLIT_R - 1) / SPLIT_R) * ((h.m + SPLIT_K - 1) / SPLIT_K);
       gy = leaves;
-      return fast;
-    }
-    case CRT_SPLIT_B: {
-      const bool fb = plain && h.m % 16 == 0;
-      gx = (int)capped_blocks(fb ? mm / 16 : mm, leaves);
+      return plain;
+    case CRT_SPLIT_B:
+      gx = (int)capped_blocks(residue_area(h.m) / 16, leaves);
       gy = leaves;
-      return fb;
-    }
-    case CRT_RECON: {
-      const bool fast = (h.m % 4 == 0) && plain;
-      gx = (int)capped_blocks(fast ? mm / 4 : mm, leaves);
+      return plain;
+    case CRT_RECON:
+      gx = (int)capped_blocks((long long)h.m * ((h.m + 3) / 4), leaves);
       gy = leaves;
-      return fast;
-    }
+      return plain;
   }
   gx = 0;
   return false;

@@ -54,6 +54,8 @@ struct Builder {
   bool fuse = true;      // fuse two leading 'b' levels when the sizes allow
   int tile = 0;          // leaf-GEMM block tile (0 default, 1 smaller)
   bool residue = false;  // matrices are nmod INT8 planes
+  int m0 = 1;            // residue mode: the layout's leaf size
+  bool pad = true;       // residue leaves at residue_pitch (false: sizes only)
   int es = 8;            // bytes per element: 8 (FP64) or 1 (residue)
   int planes = 1;        // 1 or nmod
   bool broken = false;   // an internal layout invariant failed (plan unusable)
@@ -76,6 +78,13 @@ struct Builder {
     return {base + off, (long long)per_plane};
   }
   Mat at(Mat M, long long elems) const { return {M.p + elems * es, M.ps}; }
+  // elements of an s x s matrix: residue leaves have the pitch residue_pitch,
+  // and every Winograd step is position-wise, so the padding (zeros) carries
+  // through all levels
+  long long area(int s) const {
+    const long long leaves = (long long)(s / m0) * (s / m0);
+    return residue && pad ? leaves * residue_area(m0) : (long long)s * s;
+  }
 
   size_t add_table(const void *data, size_t bytes) {
     auto &t = plan.host_tables;
@@ -112,9 +121,11 @@ struct Builder {
     steps().push_back(st);
   }
 
-  // one Winograd add step over the batch: ins[p][k], outs[p][k]
+  // one Winograd add step over the batch: ins[p][k], outs[p][k], matrices of
+  // order h
   void ew(int op, const std::vector<std::vector<Mat>> &ins,
-          const std::vector<std::vector<Mat>> &outs, long long q) {
+          const std::vector<std::vector<Mat>> &outs, int h) {
+    const long long q = area(h), elems = (long long)h * h;
     const int count = (int)ins.size();
     if (!residue) {
       std::vector<EwPtrs> t(ins.size());
@@ -153,7 +164,7 @@ struct Builder {
       }
       push(STEP_REW, op, count, q, 0, add_table(t.data(), t.size() * sizeof(RPtrs)), aligned);
     }
-    plan.additions += (long long)ew_additions(op) * q * (long long)ins.size();
+    plan.additions += (long long)ew_additions(op) * elems * (long long)ins.size();
   }
 
   void level_tag(int depth, char c) {
@@ -235,7 +246,7 @@ struct Builder {
   void ozaki_leaf_steps(const std::vector<Prob> &work, int m) {
     const int nmod = moduli;
     const size_t nb = work.size();
-    const size_t plane = (size_t)m * m;  // bytes per INT8 plane
+    const size_t plane = (size_t)residue_area(m);  // bytes per INT8 plane
     ensure_consts();
     const size_t ex_bytes = (size_t)m * sizeof(int);
     const size_t pa_bytes = (size_t)OZ_CHUNKS * m * 2 * sizeof(double);
@@ -272,7 +283,7 @@ struct Builder {
 
   void bfs(const std::vector<Prob> &batch, int s, int nrec, int depth) {
     const int h = s / 2;
-    const long long q = (long long)h * h;
+    const long long q = area(h);
     const size_t mark = top;
     const size_t nb = batch.size();
     Mat LF = alloc_mats(4 * nb, q), RF = alloc_mats(4 * nb, q), P = alloc_mats(7 * nb, q);
@@ -293,15 +304,15 @@ struct Builder {
       for (int i = 0; i < 7; i++) post_in[p].push_back(at(pp, i * q));
       for (int k = 0; k < 4; k++) post_out[p].push_back(at(C, k * q));  // C11 C21 C12 C22
     }
-    ew(EW_BFS_PRE, pre_in, pre_out, q);
+    ew(EW_BFS_PRE, pre_in, pre_out, h);
     rec(next, h, nrec - 1, depth + 1);
-    ew(EW_BFS_POST, post_in, post_out, q);
+    ew(EW_BFS_POST, post_in, post_out, h);
     top = mark;
   }
 
   void dfs(const std::vector<Prob> &batch, int s, int nrec, int depth) {
     const int h = s / 2;
-    const long long q = (long long)h * h;
+    const long long q = area(h);
     const size_t mark = top;
     const size_t nb = batch.size();
     Mat R2o = alloc_mats(nb, q), R5o = alloc_mats(nb, q);
@@ -324,7 +335,7 @@ struct Builder {
         ins[p] = pick_in(r[p]);
         outs[p] = pick_out(r[p]);
       }
-      ew(op, ins, outs, q);
+      ew(op, ins, outs, h);
     };
     auto sub = [&](Prob (*pick)(const Regs &)) {
       std::vector<Prob> b(nb);
@@ -365,7 +376,7 @@ struct Builder {
     if (!fuse || batch != 1 || nrec - cutoff < 2) return false;
     if (!(pattern[depth] == 'b' || pattern[depth] == 'B')) return false;
     if (!(pattern[depth + 1] == 'b' || pattern[depth + 1] == 'B')) return false;
-    const long long q = (long long)(s / 4) * (s / 4);
+    const long long q = area(s / 4);
     return residue ? (q % 4 == 0) : (q % 2 == 0);
   }
 
@@ -373,12 +384,13 @@ struct Builder {
   // the top, `crt` carries the reconstruction target and the combinations are
   // fused with it.
   void bfs2(const Prob &pb, int s, int nrec, int depth, const CrtMats *crt) {
-    const int h = s / 2, sub = s / 4;
-    const long long q = (long long)sub * sub;
+    const int sub = s / 4;
+    const long long q = area(sub);
+    const long long e2 = (long long)sub * sub;  // elements of a depth-2 sub-block
     const size_t mark = top;
     level_tag(depth, pattern[depth]);
     level_tag(depth + 1, pattern[depth + 1]);
-    plan.additions += 15LL * h * h + 7LL * 15 * q;
+    plan.additions += 15LL * 4 * e2 + 7LL * 15 * e2;
     // plain sub-blocks passed by pointer: level-1 / level-2 operand -> quadrant
     const int quadA[7] = {0, 2, -1, -1, -1, -1, 3};  // T1 = A11, T2 = A12, T7 = A22
     const int quadB[7] = {0, 1, -1, -1, -1, 3, -1};  // S1 = B11, S2 = B21, S6 = B22
@@ -438,7 +450,7 @@ struct Builder {
       sp.sub = sub;
       sp.m0 = crt->m;
       sp.nrec2 = crt->nrec - 2;
-      push(STEP_BB_SPLIT_B, 1, 1, q, 0, add_table(&sp, sizeof(sp)));
+      push(STEP_BB_SPLIT_B, 1, 1, q, crt->m, add_table(&sp, sizeof(sp)));
     }
     if (fused_a) {
       BBSplitA sp{};
@@ -498,17 +510,17 @@ struct Builder {
   void crt_group(const std::vector<const BatchItem *> &items) {
     const caps_desc &d = items[0]->desc;
     const int n = d.lda, m = n >> d.nrec;
-    const long long n2 = (long long)n * n;
+    const long long n2 = area(n);
     ensure_consts();
     std::vector<Prob> top_batch;
     std::vector<size_t> mats;
     // two fused 'b' levels at the top: the reconstruction is fused with the
-    // combinations; with an even leaf size B's split is fused with its
-    // pre-additions too, and with leaves a multiple of 128 A's split as well
-    // (no residue planes of C, B and A).  Otherwise A's split is a pass of
-    // its own, which transposes its leaves to row-major on the way.
+    // combinations and B's split with its pre-additions; with leaves a
+    // multiple of 128 A's split is fused too (no residue planes of C, B and
+    // A).  Otherwise A's split is a pass of its own, which transposes its
+    // leaves to row-major on the way.
     const bool top2 = items.size() == 1 && fusable(1, n, d.nrec, 0) && (d.bs == 1 || d.bs == m);
-    const bool fused_b = top2 && m % 2 == 0;
+    const bool fused_b = top2 && (pad || m % 2 == 0);
     const bool fused_a = fused_b && m % 128 == 0;
     for (const BatchItem *it : items) {
       CrtMats M{};
@@ -519,6 +531,7 @@ struct Builder {
       M.nrec = d.nrec;
       M.bs = d.bs;
       M.m = m;
+      M.plane = n2;
       M.nmod = moduli;
       M.chunks = crt_row_chunks(m);
       const int nblk = 1 << d.nrec;
@@ -594,7 +607,8 @@ hipError_t run_one(const Plan &plan, const Step &st, hipStream_t s) {
       return launch_bb_pre(reinterpret_cast<const BBPre *>(tb + st.table), st.n, st.op != 0,
                            plan.oz_moduli, kc, s, st.vec2 != 0);
     case STEP_BB_SPLIT_B:
-      return launch_bb_split_b(reinterpret_cast<const BBSplitB *>(tb + st.table), st.n, kc, s);
+      return launch_bb_split_b(reinterpret_cast<const BBSplitB *>(tb + st.table), st.n, st.bs,
+                               kc, s);
     case STEP_BB_SPLIT_A:
       return launch_bb_split_a(reinterpret_cast<const BBSplitA *>(tb + st.table), st.n, st.bs,
                                kc, s);
@@ -659,7 +673,7 @@ int timer_of(const Step &st) {
 
 int build_plan(Plan &plan, const double *A, const double *B, double *C, const caps_desc &d,
                const std::string &pattern, int mode, int moduli, int cutoff, void *work_base,
-               bool fuse, int tile) {
+               bool fuse, int tile, bool pad) {
   plan.steps.clear();
   plan.host_tables.clear();
   plan.additions = plan.multiplications = plan.leaves = 0;
@@ -677,6 +691,8 @@ int build_plan(Plan &plan, const double *A, const double *B, double *C, const ca
   b.residue = residue_mode(mode);
   b.es = b.residue ? 1 : 8;
   b.planes = b.residue ? moduli : 1;
+  b.m0 = d.lda >> d.nrec;
+  b.pad = pad;
   if (b.residue) {
     BatchItem it{A, B, C, d, pattern, cutoff};
     b.crt_group({&it});
@@ -721,8 +737,7 @@ MergeKey merge_key(const Plan &plan, const Step &st) {
           (long long)((m + 255) / 256) * ((m + 255) / 256) * st.count * st.op;  // op: moduli
       const bool big = (st.tile == 0 && m0 % 256 == 0 && (long long)m * m < (1LL << 31)) ||
                        (big_edge_gemm(m, st.levels, st.tile) && t256 >= 256);
-      if (st.bs == 0 && !big && residue_gemm_check(m, st.levels) >= 0)
-        k = {STEP_MULTI_RGEMM, 0, 0};
+      if (st.bs == 0 && !big) k = {STEP_MULTI_RGEMM, 0, 0};
       break;
     }
     case STEP_CRT_SCALE:
@@ -833,7 +848,7 @@ void emit_merged(Plan &plan, const MergeKey &k, const std::vector<const Step *> 
       const int m = (int)st->n;
       v.gx = (m + 127) / 128;
       v.gy = st->count * moduli;
-      v.aux = st->levels | (residue_gemm_check(m, st->levels) << 8);
+      v.aux = st->levels | (((m >> st->levels) % 128 != 0) << 8);
     }
     // elementwise segments count blocks (gx x gy), GEMM segments tiles
     // (gx x gx per problem, gy problems)
@@ -933,6 +948,7 @@ int build_batch_plan(Plan &plan, const std::vector<BatchItem> &items, int mode, 
     b.residue = residue_mode(mode);
     b.es = b.residue ? 1 : 8;
     b.planes = b.residue ? moduli : 1;
+    b.m0 = g[0]->desc.lda >> g[0]->desc.nrec;
     b.fuse = true;
     b.tile = tile;
     if (b.residue) {

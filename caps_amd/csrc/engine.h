@@ -46,7 +46,7 @@ enum StepKind : int {
   STEP_CRT_RECON = 10, // residue mode: C residues -> C
   STEP_BB_PRE = 11,    // two 'b' levels of pre-additions in one pass (op = residue)
   STEP_BB_POST = 12,   // two 'b' levels of combinations (residue: + reconstruction)
-  STEP_BB_SPLIT_B = 13,  // residue mode: B's split fused with its two top 'b' levels
+  STEP_BB_SPLIT_B = 13,  // residue mode: B's split fused with its two top 'b' levels, bs = m0
   // segmented launches (kernels.h VSeg) merging one step of several
   // problems of an uneven batch: table = segment array, count = segments,
   // n = flat blocks (or tiles) of the launch
@@ -117,10 +117,11 @@ struct BatchItem {
 };
 
 // Build a plan: pattern must already be resolved to one char per level.
-// work_base = nullptr computes sizes only.
+// work_base = nullptr computes sizes only; pad = false then gives the sizes
+// without the residue leaves' pitch (the measure of the fixed scratch's limit).
 int build_plan(Plan &plan, const double *A, const double *B, double *C,
                const caps_desc &d, const std::string &pattern, int mode, int moduli,
-               int cutoff, void *work_base, bool fuse = true, int tile = 0);
+               int cutoff, void *work_base, bool fuse = true, int tile = 0, bool pad = true);
 
 // Build one plan for independent multiplies of possibly different shapes:
 // items with the same (descriptor, pattern, cutoff) form a group that shares

@@ -40,7 +40,7 @@ struct BBPost {
   double *out_c;
   const int *sa, *sb;     // scale exponents of the global rows / columns
   int sub;                // depth-2 sub-block size (n / 4)
-  int m0;                 // leaf size of the layout
+  int m0;                 // leaf size of the layout (products: pitch residue_pitch(m0))
   int nrec2;              // quadrant levels inside a depth-2 sub-block (nrec - 2)
   int bs;
 };
@@ -49,12 +49,12 @@ struct BBPost {
 // fused with B's split.  FP64 B (column-major leaves) in, the residues of
 // all 49 depth-2 operands out (the plain ones too).
 struct BBSplitB {
-  const double *B;        // 16 depth-2 sub-blocks of q elements, (a, b) at element (4a + b) * q
+  const double *B;        // 16 depth-2 sub-blocks, (a, b) at element (4a + b) * sub^2
   int8_t *out;            // operand (i, j) of modulus l at out + l * sout + (7 i + j) * q
   long long sout;         // plane stride (bytes)
   const int *sb;          // scale exponents of B's global columns
   int sub;                // depth-2 sub-block size (n / 4)
-  int m0;                 // leaf size (even)
+  int m0;                 // leaf size (operands: pitch residue_pitch(m0))
   int nrec2;              // quadrant levels inside a depth-2 sub-block
 };
 
@@ -72,13 +72,14 @@ struct BBSplitA {
   int nrec2;              // quadrant levels inside a depth-2 sub-block
 };
 
+// q: positions of a depth-2 sub-block (residue mode: with the leaves' pitch).
 // FP64: q % 2 == 0; residue: q % 4 == 0.  a_only (residue): side B is
 // produced by launch_bb_split_b instead.
 hipError_t launch_bb_pre(const BBPre *d_P, long long q, bool residue, int nmod,
                          const OzakiConsts *d_consts, hipStream_t s, bool a_only = false);
-// q % 4 == 0, q < 2^31, m0 even
-hipError_t launch_bb_split_b(const BBSplitB *d_P, long long q, const OzakiConsts *d_consts,
-                             hipStream_t s);
+// m0: host copy of the table's leaf size; q < 2^31
+hipError_t launch_bb_split_b(const BBSplitB *d_P, long long q, int m0,
+                             const OzakiConsts *d_consts, hipStream_t s);
 // m0 % 128 == 0 (host copy of the table's m0), q < 2^31
 hipError_t launch_bb_split_a(const BBSplitA *d_P, long long q, int m0,
                              const OzakiConsts *d_consts, hipStream_t s);

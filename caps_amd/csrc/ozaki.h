@@ -48,22 +48,32 @@ struct OzakiConsts {
   double log2M;
 };
 
+// Residue planes store a leaf of order m0 with rows (A side) or columns (B and
+// C side) of residue_pitch(m0) bytes, the bytes past m0 zero: 16-byte chunks
+// are aligned and wholly inside or outside the pitch for every leaf size, so
+// no kernel reads residues byte by byte, and zero k positions add nothing to
+// a product.
+__host__ __device__ constexpr int residue_pitch(int m0) { return (m0 + 15) & ~15; }
+__host__ __device__ constexpr long long residue_area(int m0) {
+  return (long long)m0 * residue_pitch(m0);
+}
+
 struct OzLeaf {
   const double *A;  // m x m column-major
   const double *B;
   double *C;
   int *ea;          // m row exponents of A
   int *eb;          // m column exponents of B
-  int8_t *ra;       // nmod planes, m x m row-major
-  int8_t *rb;       // nmod planes, m x m column-major
-  int8_t *rc;       // nmod planes, m x m column-major (product residues)
+  int8_t *ra;       // nmod planes of residue_area(m), row-major
+  int8_t *rb;       // nmod planes, column-major
+  int8_t *rc;       // nmod planes, column-major (product residues)
   double *pa;       // OZ_CHUNKS x m partial row sums of squares (A)
   double *pb;       // m column sums of squares (B)
 };
 
 // One leaf product of the INT8 GEMM step: nmod residue planes per operand,
-// plane l of an operand at base + l * stride (bytes).  a: row-major m x m
-// (k contiguous), b and c: column-major m x m.  Element e of C's plane l sits
+// plane l of an operand at base + l * stride (bytes).  a: row-major leaves
+// (k contiguous), b and c: column-major, all of residue_pitch.  Element e of C's plane l sits
 // at c + l * sc + (e >> 7) * cseg + (e & 127): cseg = 128 is the plain plane;
 // a larger cseg interleaves the 128-byte segments of several products (the
 // 256-tile kernels only: residue_gemm_segmented says which launches take them).
@@ -98,11 +108,10 @@ hipError_t launch_residue_gemm_bf16(const RGemm *d_tab, int count, int m, int le
                                     const OzakiConsts *d_consts, hipStream_t s);
 // The 128 x 128 residue products over segments of different sizes in one
 // persistent launch (kernels.h VSeg: args are RGemm tables, n = order, gx =
-// tiles per dimension, gy = leaves x moduli, aux = quadtree levels | check
-// mode << 8, the mode residue_gemm_check gives; -1: not supported).
-int residue_gemm_check(int m, int levels);
+// tiles per dimension, gy = leaves x moduli, aux = quadtree levels | edge
+// checks << 8).
 // launch_residue_gemm takes the large tiles with partial edges for this
-// (plain leaves, m % 16 == 0, little padding)
+// (plain leaves, little padding)
 bool big_edge_gemm(int m, int levels, int tile);
 // launch_residue_gemm (INT8) / launch_residue_gemm_bf16 (bf16) runs these
 // leaves on the 256-tile kernel for whole tiles, which honours RGemm::cseg

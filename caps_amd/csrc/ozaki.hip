@@ -76,6 +76,7 @@ __global__ __launch_bounds__(T256) void oz_finalize_kernel(const OzLeaf *__restr
 
 // ------------------------------------------------------------------ split
 // A (column-major) -> nmod row-major INT8 planes; 64 x 64 tiles through LDS.
+// CHECK: m % 64 != 0; elements past m are zero, chunks past the pitch skipped.
 template <bool CHECK>
 __global__ __launch_bounds__(T256) void oz_split_a_kernel(const OzLeaf *__restrict__ tab, int m,
                                                           int nmod,
@@ -95,18 +96,51 @@ __global__ __launch_bounds__(T256) void oz_split_a_kernel(const OzLeaf *__restri
   // each thread: one row, 16 consecutive k
   const int r = threadIdx.x >> 2, kq = (threadIdx.x & 3) * 16;
   const int gr = r0 + r;
-  if (CHECK && gr >= m) return;
+  if (CHECK && (gr >= m || k0 + kq >= m)) return;
   const int sa = L.ea[gr];
   double x[16];
 #pragma unroll
   for (int c = 0; c < 16; c++) x[c] = trunc(ldexp(T[kq + c][r], sa));
-  int8_t *base = L.ra + (long long)gr * m + k0 + kq;
-  const long long plane = (long long)m * m;
+  int8_t *base = L.ra + (long long)gr * residue_pitch(m) + k0 + kq;
+  const long long plane = residue_area(m);
   for (int l = 0; l < nmod; l++) {
     const int mi = kc->m[l];
     const double inv = kc->inv_m[l];
     const int c22 = kc->c22[l];
-    if (!CHECK) {
+    unsigned w[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      unsigned v = 0;
+#pragma unroll
+      for (int b = 0; b < 4; b++)
+        v |= (unsigned)(sym_residue(x[4 * q + b], mi, inv, c22) & 0xff) << (8 * b);
+      w[q] = v;
+    }
+    *reinterpret_cast<uint4 *>(base + l * plane) = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+}
+
+// B (column-major) -> nmod column-major INT8 planes; thread per 16 rows of a
+// column (rows past m are zero)
+__global__ __launch_bounds__(T256) void oz_split_b_kernel(const OzLeaf *__restrict__ tab, int m,
+                                                          int nmod,
+                                                          const OzakiConsts *__restrict__ kc) {
+  const OzLeaf &L = tab[blockIdx.y];
+  const int c16 = residue_pitch(m) / 16;
+  const long long total16 = (long long)m * c16;
+  const long long plane = residue_area(m);
+  for (long long u = (long long)blockIdx.x * T256 + threadIdx.x; u < total16;
+       u += (long long)gridDim.x * T256) {
+    const int j = (int)(u / c16), i0 = (int)(u - (long long)j * c16) * 16;
+    const int s = L.eb[j];
+    double x[16];
+    load_rows16(L.B + (long long)j * m + i0, m - i0, x);
+#pragma unroll
+    for (int c = 0; c < 16; c++) x[c] = trunc(ldexp(x[c], s));
+    for (int l = 0; l < nmod; l++) {
+      const int mi = kc->m[l];
+      const double inv = kc->inv_m[l];
+      const int c22 = kc->c22[l];
       unsigned w[4];
 #pragma unroll
       for (int q = 0; q < 4; q++) {
@@ -116,68 +150,7 @@ __global__ __launch_bounds__(T256) void oz_split_a_kernel(const OzLeaf *__restri
           v |= (unsigned)(sym_residue(x[4 * q + b], mi, inv, c22) & 0xff) << (8 * b);
         w[q] = v;
       }
-      *reinterpret_cast<uint4 *>(base + l * plane) = make_uint4(w[0], w[1], w[2], w[3]);
-    } else {
-#pragma unroll
-      for (int c = 0; c < 16; c++)
-        if (k0 + kq + c < m) base[l * plane + c] = (int8_t)sym_residue(x[c], mi, inv, c22);
-    }
-  }
-}
-
-// B (column-major) -> nmod column-major INT8 planes; thread per 16 rows of a column
-template <bool CHECK>
-__global__ __launch_bounds__(T256) void oz_split_b_kernel(const OzLeaf *__restrict__ tab, int m,
-                                                          int nmod,
-                                                          const OzakiConsts *__restrict__ kc) {
-  const OzLeaf &L = tab[blockIdx.y];
-  const long long total16 = ((long long)m * m + 15) / 16;
-  const long long plane = (long long)m * m;
-  for (long long u = (long long)blockIdx.x * T256 + threadIdx.x; u < total16;
-       u += (long long)gridDim.x * T256) {
-    const long long e0 = u * 16;
-    double x[16];
-    int sb[16];
-    if (!CHECK) {
-      // m % 16 == 0: the 16 elements share a column
-      const int j = (int)(e0 / m);
-      const int s = L.eb[j];
-#pragma unroll
-      for (int c = 0; c < 16; c += 2) {
-        double2 v = *reinterpret_cast<const double2 *>(L.B + e0 + c);
-        x[c] = trunc(ldexp(v.x, s));
-        x[c + 1] = trunc(ldexp(v.y, s));
-      }
-      for (int l = 0; l < nmod; l++) {
-        const int mi = kc->m[l];
-        const double inv = kc->inv_m[l];
-        const int c22 = kc->c22[l];
-        unsigned w[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          unsigned v = 0;
-#pragma unroll
-          for (int b = 0; b < 4; b++)
-            v |= (unsigned)(sym_residue(x[4 * q + b], mi, inv, c22) & 0xff) << (8 * b);
-          w[q] = v;
-        }
-        *reinterpret_cast<uint4 *>(L.rb + l * plane + e0) = make_uint4(w[0], w[1], w[2], w[3]);
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < 16; c++) {
-        const long long e = e0 + c;
-        sb[c] = e < plane ? L.eb[(int)(e / m)] : 0;
-        x[c] = e < plane ? trunc(ldexp(L.B[e], sb[c])) : 0.0;
-      }
-      for (int l = 0; l < nmod; l++) {
-        const int mi = kc->m[l];
-        const double inv = kc->inv_m[l];
-        const int c22 = kc->c22[l];
-#pragma unroll
-        for (int c = 0; c < 16; c++)
-          if (e0 + c < plane) L.rb[l * plane + e0 + c] = (int8_t)sym_residue(x[c], mi, inv, c22);
-      }
+      *reinterpret_cast<uint4 *>(L.rb + l * plane + 16 * u) = make_uint4(w[0], w[1], w[2], w[3]);
     }
   }
 }
@@ -191,57 +164,26 @@ constexpr int ISTR = IBK + 16;  // LDS row stride (bytes): b128 reads of 16 lane
 
 // global -> registers: 128 rows of A (k contiguous) and 128 columns of B
 // (k contiguous), 64 k each, 16 bytes per access.  Ab / Bb point at the
-// slice's first element, ld is the row (A) / column (B) stride.  CHECK 0:
-// none; 1: every byte against m; 2: rows / columns against m (m % 64 == 0,
-// so K slices are whole); 3: rows / columns and 16-byte K chunks against m
-// (m % 16 == 0, so a chunk is wholly inside or outside).  Checks use the
-// slice origin; plain operands only.
+// slice's first element, ld is the row (A) / column (B) stride.  CHECK: rows /
+// columns against m, 16-byte K chunks against ld; checks use the slice origin,
+// plain operands only.
 typedef __attribute__((address_space(1))) unsigned gu32;  // stores as global_*, not flat_*
 typedef __attribute__((address_space(1))) v4i gv4i;
 typedef const __attribute__((address_space(1))) v4u gv4u;
 
-template <int CHECK>
+template <bool CHECK>
 __device__ __forceinline__ void gload_i8(const int8_t *__restrict__ Ab,
-                                         const int8_t *__restrict__ Bb, long long ld, int m,
-                                         int row0, int col0, int k0, int tid, v4u (&ga)[2],
-                                         v4u (&gb)[2]) {
+                                         const int8_t *__restrict__ Bb, int ld, int m, int row0,
+                                         int col0, int k0, int tid, v4u (&ga)[2], v4u (&gb)[2]) {
 #pragma unroll
   for (int it = 0; it < 2; it++) {
     const int idx = tid + T256 * it;
     const int r = idx >> 2, kq = (idx & 3) * 16;
-    if (CHECK == 0) {
-      ga[it] = *reinterpret_cast<const v4u *>(Ab + r * ld + kq);
-      gb[it] = *reinterpret_cast<const v4u *>(Bb + r * ld + kq);
-    } else if (CHECK == 2) {
-      // the K slice is whole; rows of A / columns of B beyond m read as zero
-      const v4u z = {0u, 0u, 0u, 0u};
-      ga[it] = row0 + r < m ? *reinterpret_cast<const v4u *>(Ab + r * ld + kq) : z;
-      gb[it] = col0 + r < m ? *reinterpret_cast<const v4u *>(Bb + r * ld + kq) : z;
-    } else if (CHECK == 3) {
-      // 16-byte chunks beyond K, rows of A / columns of B beyond m read as zero
-      const v4u z = {0u, 0u, 0u, 0u};
-      const bool kin = k0 + kq < m;
-      ga[it] = kin && row0 + r < m ? *reinterpret_cast<const v4u *>(Ab + r * ld + kq) : z;
-      gb[it] = kin && col0 + r < m ? *reinterpret_cast<const v4u *>(Bb + r * ld + kq) : z;
-    } else {
-      unsigned wa[4], wb[4];
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        unsigned va = 0, vb = 0;
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-          const int k = k0 + kq + 4 * q + b;
-          if (k < m && row0 + r < m)
-            va |= (unsigned)(uint8_t)Ab[r * ld + kq + 4 * q + b] << (8 * b);
-          if (k < m && col0 + r < m)
-            vb |= (unsigned)(uint8_t)Bb[r * ld + kq + 4 * q + b] << (8 * b);
-        }
-        wa[q] = va;
-        wb[q] = vb;
-      }
-      ga[it] = v4u{wa[0], wa[1], wa[2], wa[3]};
-      gb[it] = v4u{wb[0], wb[1], wb[2], wb[3]};
-    }
+    const v4u z = {0u, 0u, 0u, 0u};
+    const bool kin = !CHECK || k0 + kq < ld;
+    const long long off = (long long)r * ld + kq;
+    ga[it] = kin && (!CHECK || row0 + r < m) ? *reinterpret_cast<const v4u *>(Ab + off) : z;
+    gb[it] = kin && (!CHECK || col0 + r < m) ? *reinterpret_cast<const v4u *>(Bb + off) : z;
   }
 }
 
@@ -259,16 +201,16 @@ __device__ __forceinline__ void lstore_i8(int8_t *As, int8_t *Bs, int tid, const
 // One 128 x 128 tile (ti, tj) of problem p = leaf * nmod + l: C_l = A_l *
 // B_l (mod m_l).  Operands are m x m quadtrees of d levels over leaves of size
 // m0 = m >> d in CAPS quadrant order: A leaves row-major, B and C leaves
-// column-major (d = 0: plain matrices).  The fast path needs m0 % 128 == 0.
-template <int CHECK>
+// column-major, of pitch ld (d = 0: one leaf).  Without CHECK m0 % 128 == 0.
+template <bool CHECK>
 __device__ __forceinline__ void oz_tile(const RGemm *__restrict__ tab, int m, int nmod,
-                                        const OzakiConsts *__restrict__ kc, int m0, int d,
+                                        const OzakiConsts *__restrict__ kc, int m0, int ld, int d,
                                         int prob, int ti, int tj, int8_t (*As)[IBM * ISTR],
                                         int8_t (*Bs)[IBN * ISTR]) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   const int l16 = lane & 15, lk = lane >> 4;
-  const int nk = (m + IBK - 1) / IBK;
+  const int K = CHECK ? ld : m, nk = (K + IBK - 1) / IBK;
   const int leaf = prob / nmod, l = prob - leaf * nmod;
   const int8_t *__restrict__ Ap = tab[leaf].a + l * tab[leaf].sa;  // row-major
   const int8_t *__restrict__ Bp = tab[leaf].b + l * tab[leaf].sb;  // column-major
@@ -287,20 +229,20 @@ __device__ __forceinline__ void oz_tile(const RGemm *__restrict__ tab, int m, in
     for (int c = 0; c < 4; c++) acc[r][c] = v4i{bias, bias, bias, bias};
 
   v4u ga[2], gb[2];
-  const long long mm0 = (long long)m0 * m0;
+  const long long mm0 = (long long)m0 * ld;
   auto a_at = [&](int k0) {  // A slice origin (row0, k0), row-major leaf
-    return Ap + quad_leaf(row0 / m0, k0 / m0, d) * mm0 + (long long)(row0 % m0) * m0 + (k0 % m0);
+    return Ap + quad_leaf(row0 / m0, k0 / m0, d) * mm0 + (long long)(row0 % m0) * ld + (k0 % m0);
   };
   auto b_at = [&](int k0) {  // B slice origin (k0, col0), column-major leaf
-    return Bp + quad_leaf(k0 / m0, col0 / m0, d) * mm0 + (k0 % m0) + (long long)(col0 % m0) * m0;
+    return Bp + quad_leaf(k0 / m0, col0 / m0, d) * mm0 + (k0 % m0) + (long long)(col0 % m0) * ld;
   };
-  gload_i8<CHECK>(a_at(0), b_at(0), m0, m, row0, col0, 0, tid, ga, gb);
+  gload_i8<CHECK>(a_at(0), b_at(0), ld, m, row0, col0, 0, tid, ga, gb);
   lstore_i8(As[0], Bs[0], tid, ga, gb);
   __syncthreads();
   for (int kt = 0; kt < nk; kt++) {
     const int buf = kt & 1;
     if (kt + 1 < nk)
-      gload_i8<CHECK>(a_at((kt + 1) * IBK), b_at((kt + 1) * IBK), m0, m, row0, col0,
+      gload_i8<CHECK>(a_at((kt + 1) * IBK), b_at((kt + 1) * IBK), ld, m, row0, col0,
                       (kt + 1) * IBK, tid, ga, gb);
     v4i a[4], b[4];
     // lane group lk supplies k = 16*lk .. 16*lk+15 for both operands
@@ -326,8 +268,8 @@ __device__ __forceinline__ void oz_tile(const RGemm *__restrict__ tab, int m, in
     for (int c = 0; c < 4; c++) {
       const int row = row0 + wm * 64 + r * 16 + 4 * lk;
       const int col = col0 + wn * 64 + c * 16 + l16;
-      int8_t *dst = Cp + quad_leaf(row0 / m0, col0 / m0, d) * mm0 + (long long)(col % m0) * m0 +
-                    (row % m0);
+      int8_t *dst = Cp + quad_leaf(row0 / m0, col0 / m0, d) * mm0 +
+                    (long long)(col0 % m0 + col - col0) * ld + (row0 % m0 + row - row0);
       unsigned v = 0;
       if (small_k) {
         const int c14m = kc->c14[l] - 16384;
@@ -339,24 +281,16 @@ __device__ __forceinline__ void oz_tile(const RGemm *__restrict__ tab, int m, in
 #pragma unroll
         for (int q = 0; q < 4; q++) v |= (unsigned)(mod_i32(acc[r][c][q], mi, invf) & 0xff) << (8 * q);
       }
-      if (CHECK == 0) {
-        *(gu32 *)dst = v;
-      } else if (CHECK >= 2) {
-        // m % 16 == 0: the 4 rows of the word are all inside or all outside
-        if (col < m && row < m) *(gu32 *)dst = v;
-      } else if (col < m) {
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (row + q < m) dst[q] = (int8_t)(v >> (8 * q));
-      }
+      // ld % 16 == 0: the 4 rows of the word are all inside or all outside
+      if (!CHECK || (col < m && row < ld)) *(gu32 *)dst = v;
     }
 }
 
-template <int CHECK>
+template <bool CHECK>
 __global__ __launch_bounds__(T256) void oz_igemm_kernel(const RGemm *__restrict__ tab, int m,
                                                         int nmod,
                                                         const OzakiConsts *__restrict__ kc,
-                                                        TileMap map, int m0, int d) {
+                                                        TileMap map, int m0, int ld, int d) {
   __shared__ __attribute__((aligned(16))) int8_t As[2][IBM * ISTR];
   __shared__ __attribute__((aligned(16))) int8_t Bs[2][IBN * ISTR];
   const int G = gridDim.x;
@@ -365,13 +299,13 @@ __global__ __launch_bounds__(T256) void oz_igemm_kernel(const RGemm *__restrict_
     if (tile >= map.total) break;
     int prob, ti, tj;
     tile_coords(map, tile, prob, ti, tj);
-    oz_tile<CHECK>(tab, m, nmod, kc, m0, d, prob, ti, tj, As, Bs);
+    oz_tile<CHECK>(tab, m, nmod, kc, m0, ld, d, prob, ti, tj, As, Bs);
   }
 }
 
 // The residue products of several sizes in one persistent launch: segment
 // args are RGemm tables, n = order, gx = tiles per dimension, gy = problems
-// (leaves x moduli), aux = quadtree levels | check mode << 8.
+// (leaves x moduli), aux = quadtree levels | edge checks << 8.
 __global__ __launch_bounds__(T256) void oz_igemm_multi_kernel(const char *__restrict__ base,
                                                               const VSeg *__restrict__ segs,
                                                               int nseg, int total, int nmod,
@@ -388,12 +322,11 @@ __global__ __launch_bounds__(T256) void oz_igemm_multi_kernel(const char *__rest
     const int prob = local / per, r = local - prob * per;
     const int ti = r % S.gx, tj = r / S.gx;
     const RGemm *tab = reinterpret_cast<const RGemm *>(base + S.arg);
-    switch (check) {
-      case 0: oz_tile<0>(tab, m, nmod, kc, m >> d, d, prob, ti, tj, As, Bs); break;
-      case 2: oz_tile<2>(tab, m, nmod, kc, m >> d, d, prob, ti, tj, As, Bs); break;
-      case 3: oz_tile<3>(tab, m, nmod, kc, m >> d, d, prob, ti, tj, As, Bs); break;
-      default: oz_tile<1>(tab, m, nmod, kc, m >> d, d, prob, ti, tj, As, Bs); break;
-    }
+    const int m0 = m >> d, ld = residue_pitch(m0);
+    if (check)
+      oz_tile<true>(tab, m, nmod, kc, m0, ld, d, prob, ti, tj, As, Bs);
+    else
+      oz_tile<false>(tab, m, nmod, kc, m0, ld, d, prob, ti, tj, As, Bs);
   }
 }
 
@@ -404,7 +337,7 @@ __global__ __launch_bounds__(T256) void oz_igemm_multi_kernel(const char *__rest
 // wave's LDS base + 16 * lane), double-buffered, so no registers hold the
 // next stage.  Per MAC this reads 3/4 of the LDS bytes and half the L2 bytes
 // of the 128 x 128 kernel above.  Leaves of m0 % 256 == 0, or (EDGE) plain
-// leaves of m % 16 == 0 with partial last tiles.
+// leaves of any size with partial last tiles.
 //
 // LDS stage layout per operand: 256 rows x 8 chunks of 16 bytes (k), no
 // padding; chunk c of row r sits in slot c ^ swz(r), swz(r) = (r >> 1) & 7.
@@ -464,24 +397,24 @@ __device__ __forceinline__ void stage_load(__amdgpu_buffer_rsrc_t ra, __amdgpu_b
   }
 }
 
-// stage_load for plain m x m operands (d = 0) of any m % 16 == 0: rows /
-// columns at or beyond m and 16-byte K chunks at or beyond m read as zero
+// stage_load for plain operands (d = 0) of any order m, pitch ld: rows /
+// columns at or beyond m and 16-byte K chunks at or beyond ld read as zero
 // (their buffer offset is the plane size, past num_records: the buffer range
 // check returns zeros without a memory access)
 __device__ __forceinline__ void stage_load_edge(__amdgpu_buffer_rsrc_t ra,
                                                 __amdgpu_buffer_rsrc_t rb, int row0, int col0,
-                                                int k, int m, int8_t *As, int8_t *Bs, int wave,
-                                                int lane) {
+                                                int k, int m, int ld, int8_t *As, int8_t *Bs,
+                                                int wave, int lane) {
   const int rl = lane >> 3;
   const int c = (lane & 7) ^ (((wave & 1) << 2) | (rl >> 1));
-  const int oob = m * m;
-  const bool kin = k + c * 16 < m;
+  const int oob = m * ld;
+  const bool kin = k + c * 16 < ld;
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int r = j * 64 + wave * 8 + rl;
     const int slot0 = (j * 8 + wave) * 64;
-    const int ao = (kin && row0 + r < m) ? (row0 + r) * m + k + c * 16 : oob;
-    const int bo = (kin && col0 + r < m) ? (col0 + r) * m + k + c * 16 : oob;
+    const int ao = (kin && row0 + r < m) ? (row0 + r) * ld + k + c * 16 : oob;
+    const int bo = (kin && col0 + r < m) ? (col0 + r) * ld + k + c * 16 : oob;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr)(As + slot0 * 16), 16, ao, 0, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr)(Bs + slot0 * 16), 16, bo, 0, 0, 0);
   }
@@ -544,13 +477,13 @@ __device__ __forceinline__ BigTile big_tile(const RGemm *__restrict__ tab, const
 // SMALL_K: K = m <= 16384, so |sums| <= m 2^14 < 2^28 and the one-pass
 // exact reduction res_byte128 applies (sums start at 128); larger K takes the
 // general one
-// EDGE: plain operands (d = 0) whose size m is a multiple of 16 but not of
-// 256: the last tile row / column and K-step are partial, their missing
-// elements read as zero and the stores beyond m are skipped.
+// EDGE: plain operands (d = 0) whose size m is not a multiple of 256: the last
+// tile row / column and K-step are partial, their missing elements read as
+// zero and the stores beyond m (rows: beyond ld) are skipped.
 template <bool SMALL_K, bool EDGE>
 __global__ __launch_bounds__(JT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
-                    const OzakiConsts *__restrict__ kc, TileMap map, int m0, int d) {
+                    const OzakiConsts *__restrict__ kc, TileMap map, int m0, int pitch, int d) {
   __shared__ __attribute__((aligned(1024))) int8_t A0[JSTAGE];
   __shared__ __attribute__((aligned(1024))) int8_t A1[JSTAGE];
   __shared__ __attribute__((aligned(1024))) int8_t B0[JSTAGE];
@@ -560,15 +493,16 @@ oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
   const int wm = wave & 1, wn = wave >> 1;  // 2 x 4 waves: rows wm * 128, columns wn * 64
   const int l16 = lane & 15, lk = lane >> 4;
   const int G = gridDim.x;
-  const int nk = (m + JBK - 1) / JBK;
+  const int ld = EDGE ? pitch : m0;
+  const int nk = ((EDGE ? ld : m) + JBK - 1) / JBK;
   constexpr int bias = SMALL_K ? 128 : 0;
   // read offsets (bytes) of this lane's row l16, chunk lk (kh = 0) and lk + 4 (kh = 1)
   const int s16 = jswz(l16);
   const int rd0 = l16 * JBK + ((lk ^ s16) << 4);
   const int rd1 = l16 * JBK + (((lk + 4) ^ s16) << 4);
   const int aoff = wm * 128 * JBK, boff = wn * 64 * JBK;
-  const long long mm0 = (long long)m0 * m0;
-  const long long opb = (long long)m * m;  // bytes of one operand quadtree
+  const long long mm0 = (long long)m0 * ld;
+  const long long opb = (long long)m * (EDGE ? ld : m);  // bytes of one operand quadtree
   // the prefetch needs the 8 x 4 patch order of tile_coords
   const bool pf_wave = map.patch && wave < 2;
 
@@ -578,12 +512,12 @@ oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
   // offsets of row `row` / column `col` at k in the quadtree operands; plain
   // operands (d == 0) need no division by the leaf size
   auto a_off = [&](int row, int k) -> long long {
-    return d == 0 ? (long long)row * m0 + k
-                  : quad_leaf(row / m0, k / m0, d) * mm0 + (long long)(row % m0) * m0 + (k % m0);
+    return d == 0 ? (long long)row * ld + k
+                  : quad_leaf(row / m0, k / m0, d) * mm0 + (long long)(row % m0) * ld + (k % m0);
   };
   auto b_off = [&](int col, int k) -> long long {
-    return d == 0 ? (long long)col * m0 + k
-                  : quad_leaf(k / m0, col / m0, d) * mm0 + (long long)(col % m0) * m0 + (k % m0);
+    return d == 0 ? (long long)col * ld + k
+                  : quad_leaf(k / m0, col / m0, d) * mm0 + (long long)(col % m0) * ld + (k % m0);
   };
   // waves 0 and 1: this block's 1/32 share of the patch's A / B slab at k
   auto prefetch = [&](const BigTile &c, int k) {
@@ -598,9 +532,9 @@ oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
   };
   auto load = [&](const BigTile &c, int k, int8_t *As, int8_t *Bs) {
     if (EDGE)
-      stage_load_edge(c.ra, c.rb, c.row0, c.col0, k, m, As, Bs, wave, lane);
+      stage_load_edge(c.ra, c.rb, c.row0, c.col0, k, m, ld, As, Bs, wave, lane);
     else
-      stage_load(c.ra, c.rb, (int)a_off(c.row0, k), (int)b_off(c.col0, k), m0, As, Bs, wave, lane);
+      stage_load(c.ra, c.rb, (int)a_off(c.row0, k), (int)b_off(c.col0, k), ld, As, Bs, wave, lane);
   };
   load(t, 0, A0, B0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -714,20 +648,20 @@ oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
     stage_barrier();
     // lane: 16 bytes (chunk j16) of tile column pass * 32 + (tid >> 4)
     // element e of the C plane at (e >> 7) cseg + (e & 127); a 16-byte chunk
-    // (e % 16 == 0) stays in one segment, and a pass moves 32 m0 elements, a
-    // multiple of 128 (m0 % 16 == 0)
+    // (e % 16 == 0) stays in one segment, and a pass moves 32 ld elements, a
+    // multiple of 128 (ld % 16 == 0)
     const int j16 = tid & 15;
     const long long e0 = quad_leaf(t.row0 / m0, t.col0 / m0, d) * mm0 +
-                         (long long)(t.col0 % m0 + (tid >> 4)) * m0 + (t.row0 % m0) + 16 * j16;
+                         (long long)(t.col0 % m0 + (tid >> 4)) * ld + (t.row0 % m0) + 16 * j16;
     int8_t *Cl = t.Cp + (e0 >> 7) * t.cseg + (e0 & 127);
-    const long long pstep = (long long)(m0 >> 2) * t.cseg;
+    const long long pstep = (long long)(ld >> 2) * t.cseg;
 #pragma unroll
     for (int pass = 0; pass < 8; pass++) {
       const int ccl = (pass * 32 + (tid >> 4)) & 127;  // pass < 4: A1, else B1
       const unsigned *Cs = reinterpret_cast<const unsigned *>(pass < 4 ? A1 : B1);
       const v4i v = *reinterpret_cast<const v4i *>(Cs + ccl * 64 + ((4 * j16) ^ (4 * (ccl & 15))));
-      // EDGE: m % 16 == 0, so a 16-row chunk is wholly inside or outside
-      if (!EDGE || (t.col0 + pass * 32 + (tid >> 4) < m && t.row0 + 16 * j16 < m))
+      // EDGE: ld % 16 == 0, so a 16-row chunk is wholly inside or outside
+      if (!EDGE || (t.col0 + pass * 32 + (tid >> 4) < m && t.row0 + 16 * j16 < ld))
         *(gv4i *)(Cl + pass * pstep) = v;
     }
     if (!has_next) break;
@@ -783,18 +717,18 @@ __device__ __forceinline__ float fold_f32(float x, float mf, float inv) {
   return fmaf(-rintf(x * inv), mf, x);
 }
 
-template <int CHECK>
+template <bool CHECK>
 __global__ __launch_bounds__(T256) void oz_bgemm_kernel(const RGemm *__restrict__ tab, int m,
                                                         int nmod,
                                                         const OzakiConsts *__restrict__ kc,
-                                                        TileMap map, int m0, int d) {
+                                                        TileMap map, int m0, int ld, int d) {
   __shared__ __attribute__((aligned(16))) int8_t As[2][IBM * BSTR];
   __shared__ __attribute__((aligned(16))) int8_t Bs[2][IBN * BSTR];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   const int l16 = lane & 15, lk = lane >> 4;
   const int G = gridDim.x;
-  const int nk = (m + IBK - 1) / IBK;
+  const int K = CHECK ? ld : m, nk = (K + IBK - 1) / IBK;
   const int fold_every = BFOLD / IBK;
 
   for (int round = 0; round * G < map.total; round++) {
@@ -817,20 +751,20 @@ __global__ __launch_bounds__(T256) void oz_bgemm_kernel(const RGemm *__restrict_
       for (int c = 0; c < 4; c++) acc[r][c] = v4f{0.f, 0.f, 0.f, 0.f};
 
     v4u ga[2], gb[2];
-    const long long mm0 = (long long)m0 * m0;
+    const long long mm0 = (long long)m0 * ld;
     auto a_at = [&](int k0) {
-      return Ap + quad_leaf(row0 / m0, k0 / m0, d) * mm0 + (long long)(row0 % m0) * m0 + (k0 % m0);
+      return Ap + quad_leaf(row0 / m0, k0 / m0, d) * mm0 + (long long)(row0 % m0) * ld + (k0 % m0);
     };
     auto b_at = [&](int k0) {
-      return Bp + quad_leaf(k0 / m0, col0 / m0, d) * mm0 + (k0 % m0) + (long long)(col0 % m0) * m0;
+      return Bp + quad_leaf(k0 / m0, col0 / m0, d) * mm0 + (k0 % m0) + (long long)(col0 % m0) * ld;
     };
-    gload_i8<CHECK>(a_at(0), b_at(0), m0, m, row0, col0, 0, tid, ga, gb);
+    gload_i8<CHECK>(a_at(0), b_at(0), ld, m, row0, col0, 0, tid, ga, gb);
     lstore_bf(As[0], Bs[0], tid, ga, gb);
     __syncthreads();
     for (int kt = 0; kt < nk; kt++) {
       const int buf = kt & 1;
       if (kt + 1 < nk)
-        gload_i8<CHECK>(a_at((kt + 1) * IBK), b_at((kt + 1) * IBK), m0, m, row0, col0,
+        gload_i8<CHECK>(a_at((kt + 1) * IBK), b_at((kt + 1) * IBK), ld, m, row0, col0,
                         (kt + 1) * IBK, tid, ga, gb);
 #pragma unroll
       for (int kh = 0; kh < 2; kh++) {
@@ -872,28 +806,17 @@ __global__ __launch_bounds__(T256) void oz_bgemm_kernel(const RGemm *__restrict_
         const int row = row0 + wm * 64 + r * 16 + 4 * lk;
         const int col = col0 + wn * 64 + c * 16 + l16;
         int8_t *dst = Cp + quad_leaf(row0 / m0, col0 / m0, d) * mm0 +
-                      (long long)(col % m0) * m0 + (row % m0);
+                    (long long)(col0 % m0 + col - col0) * ld + (row0 % m0 + row - row0);
         int res[4];
 #pragma unroll
         for (int q = 0; q < 4; q++)
           res[q] = mod_k((int)fold_f32(acc[r][c][q], mf, invf), kc->c22[l], mi);  // |.| <= 1.5 m
-        if (CHECK == 0) {
+        // ld % 16 == 0: the 4 rows of the word are all inside or all outside
+        if (!CHECK || (col < m && row < ld)) {
           unsigned v = 0;
 #pragma unroll
           for (int q = 0; q < 4; q++) v |= (unsigned)(res[q] & 0xff) << (8 * q);
-          *reinterpret_cast<unsigned *>(dst) = v;
-        } else if (CHECK >= 2) {
-          // m % 16 == 0: the 4 rows of the word are all inside or all outside
-          if (col < m && row < m) {
-            unsigned v = 0;
-#pragma unroll
-            for (int q = 0; q < 4; q++) v |= (unsigned)(res[q] & 0xff) << (8 * q);
-            *(gu32 *)dst = v;
-          }
-        } else if (col < m) {
-#pragma unroll
-          for (int q = 0; q < 4; q++)
-            if (row + q < m) dst[q] = (int8_t)res[q];
+          *(gu32 *)dst = v;
         }
       }
   }
@@ -1091,41 +1014,40 @@ oz_bgemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
 }
 
 // ------------------------------------------------------------------ reconstruct
-template <int NP, bool VEC>
+// thread: 4 consecutive rows of a column (one word per plane)
+template <int NP>
 __global__ __launch_bounds__(T256) void oz_recon_kernel(const OzLeaf *__restrict__ tab, int m,
                                                         int nmod,
                                                         const OzakiConsts *__restrict__ kc) {
   const OzLeaf &L = tab[blockIdx.y];
-  const long long plane = (long long)m * m;
-  const int per = VEC ? 4 : 1;
-  const long long units = plane / per;
+  const int ld = residue_pitch(m), w4 = (m + 3) / 4;  // words of a column with rows below m
+  const long long plane = residue_area(m), units = (long long)m * w4;
   for (long long u = (long long)blockIdx.x * T256 + threadIdx.x; u < units;
        u += (long long)gridDim.x * T256) {
-    const long long e0 = u * per;
-    const int j = (int)(e0 / m), i0 = (int)(e0 - (long long)j * m);
+    const int j = (int)(u / w4), i0 = (int)(u - (long long)j * w4) * 4;
     const int sb = L.eb[j];
-    if (VEC) {
-      double S[4][NP];
+    const int8_t *rc = L.rc + (long long)j * ld + i0;
+    double S[4][NP];
 #pragma unroll
-      for (int q = 0; q < 4; q++)
+    for (int q = 0; q < 4; q++)
 #pragma unroll
-        for (int p = 0; p < NP; p++) S[q][p] = 0.0;
-      for (int l = 0; l < nmod; l++) {
-        const unsigned w = *reinterpret_cast<const unsigned *>(L.rc + l * plane + e0);
+      for (int p = 0; p < NP; p++) S[q][p] = 0.0;
+    for (int l = 0; l < nmod; l++) {
+      const unsigned w = *reinterpret_cast<const unsigned *>(rc + l * plane);
 #pragma unroll
-        for (int q = 0; q < 4; q++) crt_acc<NP>(S[q], (int)(int8_t)((w >> (8 * q)) & 0xff), l, kc);
-      }
+      for (int q = 0; q < 4; q++) crt_acc<NP>(S[q], (int)(int8_t)((w >> (8 * q)) & 0xff), l, kc);
+    }
+    double *dst = L.C + (long long)j * m + i0;
+    if (m % 4 == 0) {
       double out[4];
 #pragma unroll
       for (int q = 0; q < 4; q++) out[q] = ldexp(crt_finish<NP>(S[q], kc), -(L.ea[i0 + q] + sb));
-      reinterpret_cast<double2 *>(L.C + e0)[0] = make_double2(out[0], out[1]);
-      reinterpret_cast<double2 *>(L.C + e0)[1] = make_double2(out[2], out[3]);
+      reinterpret_cast<double2 *>(dst)[0] = make_double2(out[0], out[1]);
+      reinterpret_cast<double2 *>(dst)[1] = make_double2(out[2], out[3]);
     } else {
-      double S[NP];
 #pragma unroll
-      for (int p = 0; p < NP; p++) S[p] = 0.0;
-      for (int l = 0; l < nmod; l++) crt_acc<NP>(S, (int)L.rc[l * plane + e0], l, kc);
-      L.C[e0] = ldexp(crt_finish<NP>(S, kc), -(L.ea[i0] + sb));
+      for (int q = 0; q < 4; q++)
+        if (i0 + q < m) dst[q] = ldexp(crt_finish<NP>(S[q], kc), -(L.ea[i0 + q] + sb));
     }
   }
 }
@@ -1133,20 +1055,15 @@ __global__ __launch_bounds__(T256) void oz_recon_kernel(const OzLeaf *__restrict
 template <int NP>
 hipError_t launch_recon(const OzLeaf *tab, int count, int m, int nmod, const OzakiConsts *kc,
                         hipStream_t s) {
-  const bool vec = (m % 4 == 0);
-  const long long units = (long long)m * m / (vec ? 4 : 1);
+  const long long units = (long long)m * ((m + 3) / 4);
   long long blocks = (units + T256 - 1) / T256;
   long long cap = (long long)device_cu_count() * 8 / count;
   if (cap < 1) cap = 1;
   if (blocks > cap) blocks = cap;
   dim3 grid((unsigned)blocks, (unsigned)count);
-  if (vec)
-    hipLaunchKernelGGL((oz_recon_kernel<NP, true>), grid, dim3(T256), 0, s, tab, m, nmod, kc);
-  else
-    hipLaunchKernelGGL((oz_recon_kernel<NP, false>), grid, dim3(T256), 0, s, tab, m, nmod, kc);
+  hipLaunchKernelGGL((oz_recon_kernel<NP>), grid, dim3(T256), 0, s, tab, m, nmod, kc);
   return hipGetLastError();
 }
-
 
 }  // namespace
 
@@ -1171,27 +1088,21 @@ hipError_t launch_residue_gemm_bf16(const RGemm *tab, int count, int m, int leve
   const int G = persistent_grid(2, device_cu_count(), map.total);
   const bool fast = (m0 % IBM == 0);
   if (!fast && levels > 0) return hipErrorInvalidValue;
+  const int ld = residue_pitch(m0);
   if (fast)
-    hipLaunchKernelGGL((oz_bgemm_kernel<0>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
-                       m0, levels);
-  else if (m % IBK == 0)
-    hipLaunchKernelGGL((oz_bgemm_kernel<2>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
-                       m0, levels);
-  else if (m % 16 == 0)
-    hipLaunchKernelGGL((oz_bgemm_kernel<3>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
-                       m0, levels);
+    hipLaunchKernelGGL((oz_bgemm_kernel<false>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
+                       m0, ld, levels);
   else
-    hipLaunchKernelGGL((oz_bgemm_kernel<1>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
-                       m0, levels);
+    hipLaunchKernelGGL((oz_bgemm_kernel<true>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
+                       m0, ld, levels);
   return hipGetLastError();
 }
 
 // the large-tile kernel with partial edges for plain leaves (levels = 0) of
-// m % 16 == 0, m <= 16384, when the padding to 256 x 256 tiles adds at most
-// half the area (m >= 512 at worst): at 0.4 of peak it beats the 128 x 128
-// kernel there
+// m <= 16384, when the padding to 256 x 256 tiles adds at most half the area
+// (m >= 512 at worst): at 0.4 of peak it beats the 128 x 128 kernel there
 bool big_edge_gemm(int m, int levels, int tile) {
-  if (tile != 0 || levels != 0 || m % 16 != 0 || m % JBM == 0 || m > 16384 || m < 512)
+  if (tile != 0 || levels != 0 || m % JBM == 0 || residue_pitch(m) > 16384 || m < 512)
     return false;
   const long long padded = (long long)((m + JBM - 1) / JBM) * JBM;
   return 2 * padded * padded <= 3LL * m * m;
@@ -1222,49 +1133,34 @@ hipError_t launch_residue_gemm(const RGemm *tab, int count, int m, int levels, i
     const int G = persistent_grid(1, device_cu_count(), map.total);
     if (m <= 16384)
       hipLaunchKernelGGL((oz_igemm_big_kernel<true, false>), dim3(G), dim3(JT), 0, s, tab, m,
-                         nmod, kc, map, m0, levels);
+                         nmod, kc, map, m0, m0, levels);
     else
       hipLaunchKernelGGL((oz_igemm_big_kernel<false, false>), dim3(G), dim3(JT), 0, s, tab, m,
-                         nmod, kc, map, m0, levels);
+                         nmod, kc, map, m0, m0, levels);
     return hipGetLastError();
   }
   if (big_edge_gemm(m, levels, tile)) {
-    // plain operands of any m % 16 == 0 on the large tiles, partial edges
+    // plain operands of any order on the large tiles, partial edges
     TileMap map = make_tilemap(m, JBM, (long long)count * nmod, ok);
     if (!ok) return hipErrorInvalidValue;
     const int G = persistent_grid(1, device_cu_count(), map.total);
     hipLaunchKernelGGL((oz_igemm_big_kernel<true, true>), dim3(G), dim3(JT), 0, s, tab, m, nmod,
-                       kc, map, m0, levels);
+                       kc, map, m0, residue_pitch(m0), levels);
     return hipGetLastError();
   }
   TileMap map = make_tilemap(m, IBM, (long long)count * nmod, ok);
   if (!ok) return hipErrorInvalidValue;
   const int G = persistent_grid(2, device_cu_count(), map.total);
-  // the fast path reads 16-byte rows: leaves of a multiple of 128; with m %
-  // 64 == 0 the K slices are whole and only edge rows / columns are checked;
-  // with m % 16 == 0 whole 16-byte K chunks are checked too; else every byte
   const bool fast = (m0 % IBM == 0);
-  if (!fast && levels > 0) return hipErrorInvalidValue;
+  if (!fast && levels > 0) return hipErrorInvalidValue;  // quadtree operands need whole tiles
+  const int ld = residue_pitch(m0);
   if (fast)
-    hipLaunchKernelGGL((oz_igemm_kernel<0>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
-                       m0, levels);
-  else if (m % IBK == 0)
-    hipLaunchKernelGGL((oz_igemm_kernel<2>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
-                       m0, levels);
-  else if (m % 16 == 0)
-    hipLaunchKernelGGL((oz_igemm_kernel<3>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
-                       m0, levels);
+    hipLaunchKernelGGL((oz_igemm_kernel<false>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
+                       m0, ld, levels);
   else
-    hipLaunchKernelGGL((oz_igemm_kernel<1>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
-                       m0, levels);
+    hipLaunchKernelGGL((oz_igemm_kernel<true>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
+                       m0, ld, levels);
   return hipGetLastError();
-}
-
-int residue_gemm_check(int m, int levels) {
-  const int m0 = m >> levels;
-  if (m0 % IBM == 0) return 0;
-  if (levels > 0) return -1;  // quadtree operands need whole tiles
-  return m % IBK == 0 ? 2 : (m % 16 == 0 ? 3 : 1);
 }
 
 hipError_t launch_residue_gemm_multi(const char *base, const VSeg *segs, int nseg, int total,
@@ -1299,16 +1195,13 @@ hipError_t launch_ozaki_step(int step, const OzLeaf *tab, int count, int m, int 
         hipLaunchKernelGGL((oz_split_a_kernel<false>), ga, dim3(T256), 0, s, tab, m, nmod, kc);
       else
         hipLaunchKernelGGL((oz_split_a_kernel<true>), ga, dim3(T256), 0, s, tab, m, nmod, kc);
-      const long long u16 = ((long long)m * m + 15) / 16;
+      const long long u16 = residue_area(m) / 16;
       long long blocks = (u16 + T256 - 1) / T256;
       long long cap = (long long)device_cu_count() * 8 / count;
       if (cap < 1) cap = 1;
       if (blocks > cap) blocks = cap;
       dim3 gb((unsigned)blocks, count);
-      if (m % 16 == 0)
-        hipLaunchKernelGGL((oz_split_b_kernel<false>), gb, dim3(T256), 0, s, tab, m, nmod, kc);
-      else
-        hipLaunchKernelGGL((oz_split_b_kernel<true>), gb, dim3(T256), 0, s, tab, m, nmod, kc);
+      hipLaunchKernelGGL(oz_split_b_kernel, gb, dim3(T256), 0, s, tab, m, nmod, kc);
       return hipGetLastError();
     }
     case 3: {

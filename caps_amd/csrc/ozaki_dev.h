@@ -220,6 +220,24 @@ __device__ __forceinline__ double crt_finish(const double (&S)[NP],
   }
 }
 
+// 16 rows of a column from p on, zeros from row `left` on (left: rows to the
+// column's end).  Loads of 16 bytes at any 8-byte alignment.
+__device__ __forceinline__ void load_rows16(const double *__restrict__ p, int left,
+                                            double (&x)[16]) {
+  typedef double v2d __attribute__((ext_vector_type(2), aligned(8)));
+  if (left >= 16) {
+#pragma unroll
+    for (int c = 0; c < 16; c += 2) {
+      const v2d v = *reinterpret_cast<const v2d *>(p + c);
+      x[c] = v.x;
+      x[c + 1] = v.y;
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < 16; c++) x[c] = c < left ? p[c] : 0.0;
+  }
+}
+
 // offset of element (i, j) of an n x n matrix in the CAPS layout (nproc = 1):
 // nrec quadrant levels in the order 11, 21, 12, 22, then bs x bs blocks
 // column-major between and within blocks (matrix.h:20-44)

@@ -142,10 +142,11 @@ int caps_multiply_device(const double *dA, const double *dB, double *dC,
 /* Same as caps_multiply_device, for callers that cannot allocate device
  * memory (code under stream capture, tight serving loops): it calls no
  * hipMalloc / hipFree.  No counterpart in the reference.  The pointer tables
- * and workspace live in a scratch array of CAPS_NOALLOC_SCRATCH_MIB MiB that
- * every device the library runs on holds from module load until the process
- * ends; a call whose plan does not fit returns CAPS_ENOMEM (e.g. FP64 n = 2048
- * 'bd' fits, residue mode n = 1024 'bb' fits).  No graph: the steps are
+ * and workspace live in a scratch array of twice CAPS_NOALLOC_SCRATCH_MIB MiB
+ * that every device the library runs on holds from module load until the
+ * process ends; a call whose plan needs more than CAPS_NOALLOC_SCRATCH_MIB MiB,
+ * not counting the padding of residue leaves to 16 bytes, returns CAPS_ENOMEM
+ * (e.g. FP64 n = 2048 'bd' fits, residue mode n = 1024 'bb' fits).  No graph: the steps are
  * enqueued one by one on `stream`.  CAPS_MODE_AUTO is not accepted.  All calls
  * on one device share its scratch (it keeps the last call's contents; no step
  * reads scratch it has not written in the same call): calls that overlap on
