@@ -212,6 +212,11 @@ int check_cutoff(const caps_desc &d, int mode, int cutoff) {
   return CAPS_OK;
 }
 
+// the workspace limit of batch_levels: the caller's budget when one is set
+size_t batch_limit_bytes(const State &s) {
+  return s.budget_set ? (size_t)s.available_doubles * sizeof(double) : ~(size_t)0;
+}
+
 // allocate, build and upload a plan whose builder is `build(plan, work)`
 template <typename F>
 int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out) {
@@ -257,19 +262,27 @@ int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out) {
 int get_plan_locked(State &s, const double *A, const double *B, double *C, const caps_desc &d,
                     const std::string &pat, int mode, int moduli, int cutoff, bool fuse,
                     hipStream_t stream, int tile, Plan *&out) {
-  PlanKey key{A, B, C, d, pat, mode, moduli, cutoff, fuse, std::string(), stream, tile};
-  for (auto &p : s.plans)
-    if (p->key == key) {
-      out = p.get();
-      p->last_use = ++s.clock;
-      return CAPS_OK;
-    }
-  return make_plan_locked(
-      s, key,
-      [&](Plan &pl, void *work) {
-        return build_plan(pl, A, B, C, d, pat, mode, moduli, cutoff, work, fuse, tile);
-      },
-      out);
+  PlanKey key{A,  B,    C,             d,      pat,  mode, moduli, cutoff,
+              fuse, std::string(), stream, tile,
+              batch_levels(d, pat, mode, moduli, cutoff, batch_limit_bytes(s))};
+  for (;;) {
+    for (auto &p : s.plans)
+      if (p->key == key) {
+        out = p.get();
+        p->last_use = ++s.clock;
+        return CAPS_OK;
+      }
+    int rc = make_plan_locked(
+        s, key,
+        [&](Plan &pl, void *work) {
+          return build_plan(pl, A, B, C, d, pat, mode, moduli, cutoff, work, fuse, tile, true,
+                            key.run);
+        },
+        out);
+    // no memory for more batched levels than asked for: exactly those
+    if (rc != CAPS_ENOMEM || key.run == pat) return rc;
+    key.run = pat;
+  }
 }
 
 int capture_graph(Plan &p) {
@@ -474,7 +487,8 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
   // host-only plans, one per (buffers, shape, options, device): their tables
   // hold this device's scratch addresses
   PlanKey key{dA, dB, dC, *desc, pat, mode, moduli, cutoff, fuse,
-              "scratch of device " + std::to_string(s.device), nullptr, tile};
+              "scratch of device " + std::to_string(s.device), nullptr, tile,
+              batch_levels(*desc, pat, mode, moduli, cutoff, batch_limit_bytes(s))};
   Plan *p = nullptr;
   for (auto &hp : s.host_plans)
     if (hp->key == key) {
@@ -485,8 +499,8 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
     auto plan = std::make_unique<Plan>();
     plan->key = key;
     auto size_of = [&](const std::string &p, bool pad, size_t &tables, size_t &total) {
-      int r = build_plan(*plan, dA, dB, dC, *desc, p, mode, moduli, cutoff, nullptr, fuse, tile,
-                         pad);
+      int r = build_plan(*plan, dA, dB, dC, *desc, pat, mode, moduli, cutoff, nullptr, fuse, tile,
+                         pad, p);
       tables = (plan->host_tables.size() + 255) / 256 * 256;
       total = tables + plan->work_bytes;
       return r;
@@ -499,19 +513,22 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
                   "plan needs %.1f MiB of tables and workspace; caps_multiply_device_noalloc "
                   "has %d MiB of scratch",
                   need / 1048576.0, CAPS_NOALLOC_SCRATCH_MIB);
-    // with the residue pitch: where that does not fit, levels run recursively
-    // from the bottom up (the same bits)
-    std::string run = pat;
-    for (size_t l = pat.size();; l--) {
+    // as run, with the residue pitch: where that does not fit, the requested
+    // levels, then levels recursively from the bottom up (the same bits)
+    std::string run = key.run;
+    for (size_t l = pat.size() + 1;; l--) {
       if (size_of(run, true, toff, need) != CAPS_OK)
         return fail(CAPS_EINVAL, "internal: plan layout check failed");
       if (need <= SCRATCH_BYTES) break;
       if (l == 0)
         return fail(CAPS_ENOMEM, "plan needs %.1f MiB of padded workspace", need / 1048576.0);
-      run[l - 1] = 'd';
+      if (l > pat.size())
+        run = pat;
+      else
+        run[l - 1] = 'd';
     }
-    if (build_plan(*plan, dA, dB, dC, *desc, run, mode, moduli, cutoff, base + toff, fuse,
-                   tile) != CAPS_OK ||
+    if (build_plan(*plan, dA, dB, dC, *desc, pat, mode, moduli, cutoff, base + toff, fuse, tile,
+                   true, run) != CAPS_OK ||
         (plan->host_tables.size() + 255) / 256 * 256 != toff)
       return fail(CAPS_EINVAL, "internal: plan layout check failed");
     plan->d_tables = base;
@@ -718,6 +735,10 @@ int caps_multiply_batch_device(int count, const double *const *dA, const double 
     rc = resolve_pattern(descs[i], patterns ? patterns[i] : nullptr, &o, items[i].pattern, mode,
                          moduli, share > 0 ? share : 1, true);
     if (rc) return rc;
+    // recursive levels run batched within the item's share of the budget (the
+    // key holds the pattern as run)
+    items[i].pattern = batch_levels(descs[i], items[i].pattern, mode, moduli, cutoff,
+                                    (size_t)share * sizeof(double), count);
     char buf[176];
     snprintf(buf, sizeof(buf), "%p %p %p %d %d %d %d %s;", (const void *)dA[i],
              (const void *)dB[i], (void *)dC[i], descs[i].lda, descs[i].nrec, descs[i].bs, cutoff,
@@ -730,7 +751,7 @@ int caps_multiply_batch_device(int count, const double *const *dA, const double 
   const bool merge = !(opts && (opts[0].flags & CAPS_FLAG_NO_FUSION));
   const size_t merge_budget = merge ? planner_budget_bytes(s.available_doubles, s.budget_set) : 0;
   PlanKey pk{nullptr, nullptr, nullptr, descs[0], std::string(), mode, moduli, 0, merge, key,
-             stream, tile};
+             stream, tile, std::string()};
   Plan *plan = nullptr;
   for (auto &p : s.plans)
     if (p->key == pk) {

@@ -35,7 +35,8 @@ namespace caps {
 bool PlanKey::operator==(const PlanKey &o) const {
   return A == o.A && B == o.B && C == o.C && memcmp(&desc, &o.desc, sizeof(desc)) == 0 &&
          pattern == o.pattern && mode == o.mode && moduli == o.moduli && cutoff == o.cutoff &&
-         fuse == o.fuse && batch == o.batch && stream == o.stream && tile == o.tile;
+         fuse == o.fuse && batch == o.batch && stream == o.stream && tile == o.tile &&
+         run == o.run;
 }
 
 namespace {
@@ -51,6 +52,7 @@ struct Builder {
   int moduli = 0;
   int cutoff = 0;  // layout levels below the Strassen recursion
   std::string pattern;
+  std::string tags;      // the requested pattern (reported), when pattern differs
   bool fuse = true;      // fuse two leading 'b' levels when the sizes allow
   int tile = 0;          // leaf-GEMM block tile (0 default, 1 smaller)
   bool residue = false;  // matrices are nmod INT8 planes
@@ -167,7 +169,8 @@ struct Builder {
     plan.additions += (long long)ew_additions(op) * elems * (long long)ins.size();
   }
 
-  void level_tag(int depth, char c) {
+  void level_tag(int depth) {
+    const char c = tags.empty() ? pattern[depth] : tags[depth];
     const char *t = (c == 'b' || c == 'B') ? "BFS" : (c == 'h' || c == 'H') ? "HYB" : "DFS";
     // setExecutionType (counters.cpp:49-59): one 4-char field per level
     size_t want = (size_t)(depth + 1) * 4;
@@ -388,8 +391,8 @@ struct Builder {
     const long long q = area(sub);
     const long long e2 = (long long)sub * sub;  // elements of a depth-2 sub-block
     const size_t mark = top;
-    level_tag(depth, pattern[depth]);
-    level_tag(depth + 1, pattern[depth + 1]);
+    level_tag(depth);
+    level_tag(depth + 1);
     plan.additions += 15LL * 4 * e2 + 7LL * 15 * e2;
     // plain sub-blocks passed by pointer: level-1 / level-2 operand -> quadrant
     const int quadA[7] = {0, 2, -1, -1, -1, -1, 3};  // T1 = A11, T2 = A12, T7 = A22
@@ -498,7 +501,7 @@ struct Builder {
       return;
     }
     char c = pattern[depth];
-    level_tag(depth, c);
+    level_tag(depth);
     if (c == 'b' || c == 'B')
       bfs(batch, s, nrec, depth);
     else
@@ -673,7 +676,7 @@ int timer_of(const Step &st) {
 
 int build_plan(Plan &plan, const double *A, const double *B, double *C, const caps_desc &d,
                const std::string &pattern, int mode, int moduli, int cutoff, void *work_base,
-               bool fuse, int tile, bool pad) {
+               bool fuse, int tile, bool pad, const std::string &run) {
   plan.steps.clear();
   plan.host_tables.clear();
   plan.additions = plan.multiplications = plan.leaves = 0;
@@ -687,14 +690,15 @@ int build_plan(Plan &plan, const double *A, const double *B, double *C, const ca
   b.cutoff = cutoff;
   b.fuse = fuse;
   b.tile = tile;
-  b.pattern = pattern;
+  b.pattern = run.empty() ? pattern : run;
+  b.tags = pattern;
   b.residue = residue_mode(mode);
   b.es = b.residue ? 1 : 8;
   b.planes = b.residue ? moduli : 1;
   b.m0 = d.lda >> d.nrec;
   b.pad = pad;
   if (b.residue) {
-    BatchItem it{A, B, C, d, pattern, cutoff};
+    BatchItem it{A, B, C, d, b.pattern, cutoff};
     b.crt_group({&it});
   } else {
     std::vector<Prob> top{{{reinterpret_cast<char *>(const_cast<double *>(A)), 0},

@@ -83,6 +83,7 @@ struct PlanKey {
   std::string batch;  // batched plans: every item's pointers, descriptor and pattern
   const void *stream;
   int tile;           // leaf-GEMM block tile: 0 default, 1 the smaller one
+  std::string run;    // the pattern the plan runs (batch_levels of `pattern`)
   bool operator==(const PlanKey &o) const;
 };
 
@@ -112,16 +113,19 @@ struct BatchItem {
   const double *A, *B;
   double *C;
   caps_desc desc;
-  std::string pattern;  // resolved, one char per recursed level
+  std::string pattern;  // as run (batch_levels), one char per recursed level
   int cutoff = 0;       // layout levels multiplied classically
 };
 
-// Build a plan: pattern must already be resolved to one char per level.
+// Build a plan: pattern must already be resolved to one char per level; the
+// plan runs `run` (empty: pattern itself), its execution pattern is reported
+// as `pattern`.
 // work_base = nullptr computes sizes only; pad = false then gives the sizes
 // without the residue leaves' pitch (the measure of the fixed scratch's limit).
 int build_plan(Plan &plan, const double *A, const double *B, double *C,
                const caps_desc &d, const std::string &pattern, int mode, int moduli,
-               int cutoff, void *work_base, bool fuse = true, int tile = 0, bool pad = true);
+               int cutoff, void *work_base, bool fuse = true, int tile = 0, bool pad = true,
+               const std::string &run = std::string());
 
 // Build one plan for independent multiplies of possibly different shapes:
 // items with the same (descriptor, pattern, cutoff) form a group that shares

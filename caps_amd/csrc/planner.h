@@ -16,6 +16,13 @@ size_t planner_budget_bytes(long long budget_doubles, bool budget_set);
 std::string choose_pattern(const caps_desc &d, int mode, int moduli, long long budget_doubles,
                            bool budget_set);
 
+// The pattern a plan runs for the requested one: recursive levels run batched,
+// the deepest first, while they add at most the operands' own bytes (or 64 MiB)
+// to the requested pattern's workspace, within limit_bytes.  The results do not
+// depend on it.  items: problems of the same shape planned together.
+std::string batch_levels(const caps_desc &d, const std::string &pattern, int mode, int moduli,
+                         int cutoff, size_t limit_bytes, int items = 1);
+
 // Leaf arithmetic when the caller asks for CAPS_MODE_AUTO.
 int choose_mode(const caps_desc &d);
 
