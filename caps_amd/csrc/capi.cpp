@@ -29,11 +29,11 @@
 // hipGetSymbolAddress (State::scratch).
 //
 // CAPS_NOALLOC_SCRATCH_MIB limits a plan's tables and workspace counted
-// without the padding of residue leaves to a 16-byte pitch.  From leaves of 17
-// up the pitch adds at most 15 / 17, so twice the limit holds every plan that
-// passes; smaller leaves (orders up to 1920 with at most 7 levels) that do not
-// fit with it run fewer levels batched.
-constexpr size_t SCRATCH_BYTES = (size_t)(2 * CAPS_NOALLOC_SCRATCH_MIB) << 20;
+// without the padding of residue leaves to a 16-byte pitch.  A plan that passes
+// and does not fit with it runs fewer levels batched; recursive at every level,
+// the largest padded plan is 344 MiB (order 2176, 6 levels, 13 moduli).  Module
+// load clears the array (0.38 ms per MiB), so it is no larger than that needs.
+constexpr size_t SCRATCH_BYTES = (size_t)(CAPS_NOALLOC_SCRATCH_MIB + 96) << 20;
 static __device__ __align__(256) char scratch[SCRATCH_BYTES];
 
 namespace caps {

@@ -188,7 +188,8 @@ struct Builder {
       // residue leaves are already row-major (A) / column-major (B, C)
       ensure_consts();
       std::vector<RGemm> g(batch.size());
-      const bool segmented = residue_gemm_segmented(m, cutoff, tile, mode == CAPS_MODE_CRT_BF16);
+      const bool segmented = residue_gemm_segmented(m, cutoff, tile, mode == CAPS_MODE_CRT_BF16,
+                                                    (long long)batch.size() * moduli);
       for (size_t p = 0; p < batch.size(); p++) {
         g[p] = {reinterpret_cast<const int8_t *>(batch[p].A.p),
                 reinterpret_cast<const int8_t *>(batch[p].B.p),
@@ -405,7 +406,8 @@ struct Builder {
     // segments, so that the post-combination reads one contiguous 49 x 128
     // bytes per modulus for 128 positions
     const bool seg = residue && nrec - 2 == cutoff && q % 128 == 0 &&
-                     residue_gemm_segmented(sub, cutoff, tile, mode == CAPS_MODE_CRT_BF16);
+                     residue_gemm_segmented(sub, cutoff, tile, mode == CAPS_MODE_CRT_BF16,
+                                          49LL * moduli);
     const long long pstep = seg ? 128 : q * es, cseg = seg ? 49 * 128 : 128;
     // the kernels address the 40 written operands of a side as out + k * step
     // (k counts the non-plain (i, j) in order) and product (i, j) as
@@ -635,7 +637,7 @@ hipError_t run_one(const Plan &plan, const Step &st, hipStream_t s) {
       return launch_dgemm_multi(st.bs, tb, reinterpret_cast<const VSeg *>(tb + st.table),
                                 st.count, (int)st.n, s);
     case STEP_MULTI_RGEMM:
-      return launch_residue_gemm_multi(tb, reinterpret_cast<const VSeg *>(tb + st.table),
+      return launch_residue_gemm_multi(st.bs, tb, reinterpret_cast<const VSeg *>(tb + st.table),
                                        st.count, (int)st.n, plan.oz_moduli, kc, s);
     case STEP_MULTI_CRT:
       return launch_crt_multi(st.op, st.vec2 != 0, ozaki_npieces(plan.oz_moduli), tb,
@@ -733,15 +735,10 @@ MergeKey merge_key(const Plan &plan, const Step &st) {
       k = {STEP_MULTI_GEMM, dgemm_block_tile((int)st.n, st.levels, st.tile, 1LL << 24), 0};
       break;
     case STEP_OZ_GEMM: {
-      // INT8 products that would take the 128 x 128 kernel alone; those on
-      // 256-tile leaves keep their own launch, and so do those that take the
-      // 256 tiles with partial edges when they fill the device (256 tiles)
-      const int m = (int)st.n, m0 = m >> st.levels;
-      const long long t256 =
-          (long long)((m + 255) / 256) * ((m + 255) / 256) * st.count * st.op;  // op: moduli
-      const bool big = (st.tile == 0 && m0 % 256 == 0 && (long long)m * m < (1LL << 31)) ||
-                       (big_edge_gemm(m, st.levels, st.tile) && t256 >= 256);
-      if (st.bs == 0 && !big) k = {STEP_MULTI_RGEMM, 0, 0};
+      // INT8 products below the 256 tiles share a launch by block tile (that
+      // of a launch which fills the device); those on 256 tiles keep their own
+      const int bt = residue_block_tile((int)st.n, st.levels, st.tile, 1LL << 24);
+      if (st.bs == 0 && bt < 256) k = {STEP_MULTI_RGEMM, bt, 0};
       break;
     }
     case STEP_CRT_SCALE:
@@ -816,6 +813,7 @@ void emit_merged(Plan &plan, const MergeKey &k, const std::vector<const Step *> 
   // FP64 products: a smaller block tile where all heads together leave the
   // device idle
   int bt = k.a;
+  const bool gemm_step = k.kind == STEP_MULTI_GEMM || k.kind == STEP_MULTI_RGEMM;
   if (k.kind == STEP_MULTI_GEMM && heads[0]->tile == 0) {
     double cost = INFINITY;
     for (int b = k.a; b >= 32; b /= 2) {
@@ -849,22 +847,19 @@ void emit_merged(Plan &plan, const MergeKey &k, const std::vector<const Step *> 
       v.gy = st->count;
       v.aux = st->levels | (((m >> st->levels) % bt != 0) << 8);
     } else {  // STEP_MULTI_RGEMM
-      const int m = (int)st->n;
-      v.gx = (m + 127) / 128;
+      v.gx = ((int)st->n + bt - 1) / bt;
       v.gy = st->count * moduli;
-      v.aux = st->levels | (((m >> st->levels) % 128 != 0) << 8);
+      v.aux = st->levels;
     }
     // elementwise segments count blocks (gx x gy), GEMM segments tiles
     // (gx x gx per problem, gy problems)
-    const bool gemm = k.kind == STEP_MULTI_GEMM || k.kind == STEP_MULTI_RGEMM;
-    total += gemm ? (long long)v.gx * v.gx * v.gy : (long long)v.gx * v.gy;
+    total += gemm_step ? (long long)v.gx * v.gx * v.gy : (long long)v.gx * v.gy;
     segs.push_back(v);
   }
   const size_t off = push_segs(plan, segs);
   // op: the Winograd op of an add step; flag: 16/4-byte accesses (adds) or
-  // the FP64 block tile
-  plan.steps.push_back(multi_step(k.kind, k.a, k.kind == STEP_MULTI_GEMM ? bt : k.b, segs,
-                                  total, off));
+  // the block tile
+  plan.steps.push_back(multi_step(k.kind, k.a, gemm_step ? bt : k.b, segs, total, off));
 }
 
 // Interleave the groups' step lists: repeatedly take the key shared by the

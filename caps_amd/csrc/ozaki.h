@@ -106,20 +106,21 @@ hipError_t launch_ozaki_step(int step, const OzLeaf *d_tab, int count, int m, in
 // the same products on BF16 MFMA with FP32 accumulation (bit-identical results)
 hipError_t launch_residue_gemm_bf16(const RGemm *d_tab, int count, int m, int levels, int nmod,
                                     const OzakiConsts *d_consts, hipStream_t s);
-// The 128 x 128 residue products over segments of different sizes in one
-// persistent launch (kernels.h VSeg: args are RGemm tables, n = order, gx =
-// tiles per dimension, gy = leaves x moduli, aux = quadtree levels | edge
-// checks << 8).
-// launch_residue_gemm takes the large tiles with partial edges for this
-// (plain leaves, little padding)
-bool big_edge_gemm(int m, int levels, int tile);
+// The block tile of `problems` INT8 products (leaves x moduli) of order m: 256
+// (the large-tile kernel) or 64..192, by residue_tile_cost's estimate of a
+// launch of `tiles` tiles over K.
+int residue_block_tile(int m, int levels, int tile, long long problems);
+double residue_tile_cost(int bt, double tiles, int K);
 // launch_residue_gemm (INT8) / launch_residue_gemm_bf16 (bf16) runs these
 // leaves on the 256-tile kernel for whole tiles, which honours RGemm::cseg
-bool residue_gemm_segmented(int m, int levels, int tile, bool bf16);
-hipError_t launch_residue_gemm_multi(const char *d_tables, const VSeg *d_segs, int nseg,
+bool residue_gemm_segmented(int m, int levels, int tile, bool bf16, long long problems);
+// INT8 products over segments of different sizes in one persistent launch
+// (kernels.h VSeg: args are RGemm tables, n = order, gx = tiles per dimension,
+// gy = leaves x moduli, aux = quadtree levels), block tile bt < 256
+hipError_t launch_residue_gemm_multi(int bt, const char *d_tables, const VSeg *d_segs, int nseg,
                                      int total_tiles, int nmod, const OzakiConsts *d_consts,
                                      hipStream_t s);
-// tile: 0 = 256 x 256 block tiles where the leaves allow, 1 = 128 x 128
+// tile: 0 = the block tile of residue_block_tile, 1 = the same below 256
 hipError_t launch_residue_gemm(const RGemm *d_tab, int count, int m, int levels, int nmod,
                                const OzakiConsts *d_consts, hipStream_t s, int tile = 0);
 

@@ -9,7 +9,7 @@
 //   igemm  : INT8 planes -> INT32 products on v_mfma_i32_16x16x64_i8, mod m_l
 //            in the epilogue, INT8 residue planes out.            MFMA-bound
 //   recon  : CRT in FP64 from the residue planes, unscale.        HBM-bound
-#include <climits>
+#include <math.h>
 
 #include "kernels.h"
 #include "ozaki.h"
@@ -159,121 +159,162 @@ __global__ __launch_bounds__(T256) void oz_split_b_kernel(const OzLeaf *__restri
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
-constexpr int IBM = 128, IBN = 128, IBK = 64;
-constexpr int ISTR = IBK + 16;  // LDS row stride (bytes): b128 reads of 16 lanes hit 64 banks
-
-// global -> registers: 128 rows of A (k contiguous) and 128 columns of B
-// (k contiguous), 64 k each, 16 bytes per access.  Ab / Bb point at the
-// slice's first element, ld is the row (A) / column (B) stride.  CHECK: rows /
-// columns against m, 16-byte K chunks against ld; checks use the slice origin,
-// plain operands only.
 typedef __attribute__((address_space(1))) unsigned gu32;  // stores as global_*, not flat_*
 typedef __attribute__((address_space(1))) v4i gv4i;
 typedef const __attribute__((address_space(1))) v4u gv4u;
+typedef __attribute__((address_space(3))) void *lds_ptr;
 
-template <bool CHECK>
-__device__ __forceinline__ void gload_i8(const int8_t *__restrict__ Ab,
-                                         const int8_t *__restrict__ Bb, int ld, int m, int row0,
-                                         int col0, int k0, int tid, v4u (&ga)[2], v4u (&gb)[2]) {
-#pragma unroll
-  for (int it = 0; it < 2; it++) {
-    const int idx = tid + T256 * it;
-    const int r = idx >> 2, kq = (idx & 3) * 16;
-    const v4u z = {0u, 0u, 0u, 0u};
-    const bool kin = !CHECK || k0 + kq < ld;
-    const long long off = (long long)r * ld + kq;
-    ga[it] = kin && (!CHECK || row0 + r < m) ? *reinterpret_cast<const v4u *>(Ab + off) : z;
-    gb[it] = kin && (!CHECK || col0 + r < m) ? *reinterpret_cast<const v4u *>(Bb + off) : z;
-  }
+// block barrier for LDS stages filled by this wave's own loads: the caller
+// has waited for them (vmcnt) and consumed every LDS read of the stage it
+// leaves; the empty asm statements keep memory operations on their side
+__device__ __forceinline__ void stage_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 }
 
-__device__ __forceinline__ void lstore_i8(int8_t *As, int8_t *Bs, int tid, const v4u (&ga)[2],
-                                          const v4u (&gb)[2]) {
-#pragma unroll
-  for (int it = 0; it < 2; it++) {
-    const int idx = tid + T256 * it;
-    const int r = idx >> 2, kq = (idx & 3) * 16;
-    *reinterpret_cast<v4u *>(&As[r * ISTR + kq]) = ga[it];
-    *reinterpret_cast<v4u *>(&Bs[r * ISTR + kq]) = gb[it];
-  }
+// a raw buffer of `bytes` (< 2^31) from p on
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const int8_t *p, long long bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(p), 0, (int)bytes, 0x00020000);
 }
 
-// One 128 x 128 tile (ti, tj) of problem p = leaf * nmod + l: C_l = A_l *
-// B_l (mod m_l).  Operands are m x m quadtrees of d levels over leaves of size
-// m0 = m >> d in CAPS quadrant order: A leaves row-major, B and C leaves
-// column-major, of pitch ld (d = 0: one leaf).  Without CHECK m0 % 128 == 0.
-template <bool CHECK>
-__device__ __forceinline__ void oz_tile(const RGemm *__restrict__ tab, int m, int nmod,
-                                        const OzakiConsts *__restrict__ kc, int m0, int ld, int d,
-                                        int prob, int ti, int tj, int8_t (*As)[IBM * ISTR],
-                                        int8_t (*Bs)[IBN * ISTR]) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// Block tile BT x BT (64, 96, 128, 160 or 192), 4 waves in a 2 x 2 grid of
+// (BT / 2)^2 wave tiles, K slices of 64 on v_mfma_i32_16x16x64_i8.
+//
+// For the leaves the 256 tiles would mostly pad, and launches they would leave
+// the device idle in.  Several blocks share a CU (2 to 8), so one block's
+// epilogue, barriers and load latency run under the others' MFMAs.  Operands
+// go global -> LDS by buffer loads that write LDS directly, double-buffered;
+// rows past the leaf and 16-byte chunks past its pitch get an offset past the
+// buffer (the range check returns zeros).  LDS rows are 64 bytes; chunk c of
+// row r sits in slot c ^ ((r >> 2) & 3), so the 16 rows of one ds_read_b128
+// cycle cover the 64 banks once.  C leaves through LDS (columns of BT / 4 + 4
+// words: 16 columns start 4 odd multiples of 4 banks apart) as 16-byte pieces
+// of BT-byte columns.
+constexpr int MBK = 64;
+template <int BT>
+struct Mid {
+  static constexpr int WT = BT / 2;       // wave tile
+  static constexpr int MT = WT / 16;      // MFMA tiles per wave dimension
+  static constexpr int STAGE = BT * MBK;  // bytes of one operand's stage
+  static constexpr int CP = BT / 4 + 4;   // words of a staged C column
+  static constexpr int OCC = BT == 64 ? 8 : (BT == 96 ? 5 : (BT == 128 ? 4 : (BT == 160 ? 3 : 2)));
+  static_assert(BT * CP * 4 <= 4 * STAGE, "C is staged in the operands' LDS");
+};
+
+// 64 lanes x 16 bytes at lane offset v of r to 1 KB of LDS
+__device__ __forceinline__ void dma_1k(__amdgpu_buffer_rsrc_t r, int8_t *lds, int v) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)lds, 16, v, 0, 0, 0);
+}
+
+// One tile (ti, tj) of problem p = leaf * nmod + l: C_l = A_l * B_l (mod m_l).
+// Operands are m x m quadtrees of d levels over leaves of size m0 = m >> d in
+// CAPS quadrant order, A leaves row-major, B and C leaves column-major, of
+// pitch ld (d = 0: one leaf; d > 0 needs m0 % BT == 0 and ld == m0).
+template <int BT>
+__device__ __forceinline__ void mid_tile(const RGemm *__restrict__ tab, int m, int nmod,
+                                         const OzakiConsts *__restrict__ kc, int d, int prob,
+                                         int ti, int tj, int8_t *S) {
+  using P = Mid<BT>;
+  constexpr int WT = P::WT, MT = P::MT, ST = P::STAGE;
+  constexpr int NUM_RECORDS = 0x40000000, OOB = 0x7fffff00;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
   const int l16 = lane & 15, lk = lane >> 4;
-  const int K = CHECK ? ld : m, nk = (K + IBK - 1) / IBK;
+  const int m0 = m >> d, ld = residue_pitch(m0);
+  const int K = d == 0 ? ld : m, nk = (K + MBK - 1) / MBK;
   const int leaf = prob / nmod, l = prob - leaf * nmod;
-  const int8_t *__restrict__ Ap = tab[leaf].a + l * tab[leaf].sa;  // row-major
-  const int8_t *__restrict__ Bp = tab[leaf].b + l * tab[leaf].sb;  // column-major
-  int8_t *__restrict__ Cp = tab[leaf].c + l * tab[leaf].sc;
+  const int8_t *Ap = tab[leaf].a + l * tab[leaf].sa;  // row-major
+  const int8_t *Bp = tab[leaf].b + l * tab[leaf].sb;  // column-major
+  int8_t *Cp = tab[leaf].c + l * tab[leaf].sc;
   const int mi = kc->m[l];
   const float mf = (float)mi, invf = 1.0f / mf;
-  const int row0 = ti * IBM, col0 = tj * IBN;
+  const int row0 = ti * BT, col0 = tj * BT;
+  const long long mm0 = (long long)m0 * ld;
+
+  // load i of a slice (i = 4 it + wave): 16 rows of A (i < BT / 16) or of B
+  int off[MT];
+  const int c16 = ((lane & 3) ^ (lane >> 4)) * 16;  // this lane's chunk of its row
+#pragma unroll
+  for (int it = 0; it < MT; it++) {
+    const int i = 4 * it + wave, j = i < BT / 16 ? i : i - BT / 16;
+    const int r = 16 * j + (lane >> 2);
+    off[it] = (i < BT / 16 ? row0 : col0) + r < m ? r * ld + c16 : OOB;
+  }
+  // the next slice of A and B, moved along K; the next leaf of the quadtree
+  // after m0
+  auto a_at = [&](int k) {
+    return Ap + quad_leaf(row0 / m0, k / m0, d) * mm0 + (long long)(row0 % m0) * ld;
+  };
+  auto b_at = [&](int k) {
+    return Bp + quad_leaf(k / m0, col0 / m0, d) * mm0 + (long long)(col0 % m0) * ld;
+  };
+  const int8_t *pa = d == 0 ? Ap + (long long)row0 * ld : a_at(0);
+  const int8_t *pb = d == 0 ? Bp + (long long)col0 * ld : b_at(0);
+  int knext = 0, kleft = m0;
+  auto stage = [&](int8_t *buf) {
+    const __amdgpu_buffer_rsrc_t ra = plane_rsrc(pa, NUM_RECORDS), rb = plane_rsrc(pb, NUM_RECORDS);
+    const bool in = c16 < K - knext;  // chunks past K (K % 16 == 0)
+#pragma unroll
+    for (int it = 0; it < MT; it++) {
+      const int i = 4 * it + wave;
+      const int v = in ? off[it] : OOB;
+      if (i < BT / 16)
+        dma_1k(ra, buf + i * 1024, v);
+      else
+        dma_1k(rb, buf + i * 1024, v);
+    }
+    pa += MBK;
+    pb += MBK;
+    knext += MBK;
+    kleft -= MBK;
+    if (d > 0 && kleft == 0 && knext < m) {
+      pa = a_at(knext);
+      pb = b_at(knext);
+      kleft = m0;
+    }
+  };
 
   // small K: the sums start at 128 for the one-pass reduction res_byte128
-  const bool small_k = m <= 16384;
+  const bool small_k = K <= 16384;
   const int bias = small_k ? 128 : 0;
-  v4i acc[4][4];
+  v4i acc[MT][MT];
 #pragma unroll
-  for (int r = 0; r < 4; r++)
+  for (int r = 0; r < MT; r++)
 #pragma unroll
-    for (int c = 0; c < 4; c++) acc[r][c] = v4i{bias, bias, bias, bias};
-
-  v4u ga[2], gb[2];
-  const long long mm0 = (long long)m0 * ld;
-  auto a_at = [&](int k0) {  // A slice origin (row0, k0), row-major leaf
-    return Ap + quad_leaf(row0 / m0, k0 / m0, d) * mm0 + (long long)(row0 % m0) * ld + (k0 % m0);
-  };
-  auto b_at = [&](int k0) {  // B slice origin (k0, col0), column-major leaf
-    return Bp + quad_leaf(k0 / m0, col0 / m0, d) * mm0 + (k0 % m0) + (long long)(col0 % m0) * ld;
-  };
-  gload_i8<CHECK>(a_at(0), b_at(0), ld, m, row0, col0, 0, tid, ga, gb);
-  lstore_i8(As[0], Bs[0], tid, ga, gb);
-  __syncthreads();
+    for (int c = 0; c < MT; c++) acc[r][c] = v4i{bias, bias, bias, bias};
+  const int rd = l16 * MBK + ((lk ^ (l16 >> 2)) << 4);
+  stage(S);
   for (int kt = 0; kt < nk; kt++) {
-    const int buf = kt & 1;
-    if (kt + 1 < nk)
-      gload_i8<CHECK>(a_at((kt + 1) * IBK), b_at((kt + 1) * IBK), ld, m, row0, col0,
-                      (kt + 1) * IBK, tid, ga, gb);
-    v4i a[4], b[4];
-    // lane group lk supplies k = 16*lk .. 16*lk+15 for both operands
+    int8_t *cur = S + (kt & 1) * 2 * ST, *oth = S + ((kt & 1) ^ 1) * 2 * ST;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    stage_barrier();
+    if (kt + 1 < nk) stage(oth);
+    v4i a[MT], b[MT];
 #pragma unroll
-    for (int r = 0; r < 4; r++)
-      a[r] = *reinterpret_cast<const v4i *>(&As[buf][(wm * 64 + r * 16 + l16) * ISTR + 16 * lk]);
+    for (int c = 0; c < MT; c++)
+      b[c] = *reinterpret_cast<const v4i *>(cur + ST + (wn * WT + c * 16) * MBK + rd);
 #pragma unroll
-    for (int c = 0; c < 4; c++)
-      b[c] = *reinterpret_cast<const v4i *>(&Bs[buf][(wn * 64 + c * 16 + l16) * ISTR + 16 * lk]);
+    for (int r = 0; r < MT; r++)
+      a[r] = *reinterpret_cast<const v4i *>(cur + (wm * WT + r * 16) * MBK + rd);
 #pragma unroll
-    for (int r = 0; r < 4; r++)
+    for (int r = 0; r < MT; r++)
 #pragma unroll
-      for (int c = 0; c < 4; c++)
+      for (int c = 0; c < MT; c++)
         acc[r][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[r], b[c], acc[r][c], 0, 0, 0);
-    if (kt + 1 < nk) lstore_i8(As[buf ^ 1], Bs[buf ^ 1], tid, ga, gb);
-    __syncthreads();
   }
+  stage_barrier();  // every wave has read its last fragments: the stages are free
 
   // D layout: lane holds column (lane % 16), rows 4 * (lane / 16) + v
+  unsigned *Cw = reinterpret_cast<unsigned *>(S);
+  const int c14m = kc->c14[l] - 16384;
+  const float cl = 0.5f - 128.0f * invf;
 #pragma unroll
-  for (int r = 0; r < 4; r++)
+  for (int r = 0; r < MT; r++)
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-      const int row = row0 + wm * 64 + r * 16 + 4 * lk;
-      const int col = col0 + wn * 64 + c * 16 + l16;
-      int8_t *dst = Cp + quad_leaf(row0 / m0, col0 / m0, d) * mm0 +
-                    (long long)(col0 % m0 + col - col0) * ld + (row0 % m0 + row - row0);
+    for (int c = 0; c < MT; c++) {
       unsigned v = 0;
       if (small_k) {
-        const int c14m = kc->c14[l] - 16384;
-        const float cl = 0.5f - 128.0f * invf;
 #pragma unroll
         for (int q = 0; q < 4; q++) v = res_byte128(acc[r][c][q], c14m, mf, invf, cl, q, v);
         v ^= 0x80808080u;
@@ -281,52 +322,55 @@ __device__ __forceinline__ void oz_tile(const RGemm *__restrict__ tab, int m, in
 #pragma unroll
         for (int q = 0; q < 4; q++) v |= (unsigned)(mod_i32(acc[r][c][q], mi, invf) & 0xff) << (8 * q);
       }
-      // ld % 16 == 0: the 4 rows of the word are all inside or all outside
-      if (!CHECK || (col < m && row < ld)) *(gu32 *)dst = v;
+      Cw[(wn * WT + c * 16 + l16) * P::CP + wm * (WT / 4) + r * 4 + lk] = v;
     }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  stage_barrier();
+  int8_t *Ct = Cp + (d == 0 ? (long long)col0 * ld + row0
+                            : quad_leaf(row0 / m0, col0 / m0, d) * mm0 +
+                                  (long long)(col0 % m0) * ld + row0 % m0);
+  const int clim = m - col0, rlim = K - row0;  // rows: to the pitch (d = 0)
+  for (int idx = tid; idx < BT * (BT / 16); idx += T256) {
+    const int col = idx / (BT / 16), j = idx % (BT / 16);
+    const v4i v = *reinterpret_cast<const v4i *>(Cw + col * P::CP + 4 * j);
+    if (col < clim && 16 * j < rlim) *(gv4i *)(Ct + (long long)col * ld + 16 * j) = v;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  stage_barrier();  // the next tile's first stage overwrites the staged C
 }
 
-template <bool CHECK>
-__global__ __launch_bounds__(T256) void oz_igemm_kernel(const RGemm *__restrict__ tab, int m,
-                                                        int nmod,
-                                                        const OzakiConsts *__restrict__ kc,
-                                                        TileMap map, int m0, int ld, int d) {
-  __shared__ __attribute__((aligned(16))) int8_t As[2][IBM * ISTR];
-  __shared__ __attribute__((aligned(16))) int8_t Bs[2][IBN * ISTR];
+template <int BT>
+__global__ __launch_bounds__(T256) __attribute__((amdgpu_waves_per_eu(Mid<BT>::OCC))) void
+oz_igemm_mid_kernel(const RGemm *__restrict__ tab, int m, int nmod,
+                    const OzakiConsts *__restrict__ kc, TileMap map, int d) {
+  __shared__ __attribute__((aligned(1024))) int8_t S[4 * Mid<BT>::STAGE];
   const int G = gridDim.x;
   for (int round = 0; round * G < map.total; round++) {
     const int tile = round * G + xcd_tile(blockIdx.x, G);
     if (tile >= map.total) break;
     int prob, ti, tj;
     tile_coords(map, tile, prob, ti, tj);
-    oz_tile<CHECK>(tab, m, nmod, kc, m0, ld, d, prob, ti, tj, As, Bs);
+    mid_tile<BT>(tab, m, nmod, kc, d, prob, ti, tj, S);
   }
 }
 
 // The residue products of several sizes in one persistent launch: segment
 // args are RGemm tables, n = order, gx = tiles per dimension, gy = problems
-// (leaves x moduli), aux = quadtree levels | edge checks << 8.
-__global__ __launch_bounds__(T256) void oz_igemm_multi_kernel(const char *__restrict__ base,
-                                                              const VSeg *__restrict__ segs,
-                                                              int nseg, int total, int nmod,
-                                                              const OzakiConsts *__restrict__ kc) {
-  __shared__ __attribute__((aligned(16))) int8_t As[2][IBM * ISTR];
-  __shared__ __attribute__((aligned(16))) int8_t Bs[2][IBN * ISTR];
+// (leaves x moduli), aux = quadtree levels.
+template <int BT>
+__global__ __launch_bounds__(T256) __attribute__((amdgpu_waves_per_eu(Mid<BT>::OCC))) void
+oz_igemm_multi_kernel(const char *__restrict__ base, const VSeg *__restrict__ segs, int nseg,
+                      int total, int nmod, const OzakiConsts *__restrict__ kc) {
+  __shared__ __attribute__((aligned(1024))) int8_t S[4 * Mid<BT>::STAGE];
   const int G = gridDim.x;
   for (int round = 0; round * G < total; round++) {
     const int tile = round * G + xcd_tile(blockIdx.x, G);
     if (tile >= total) break;
-    const VSeg &S = segs[vseg_find(segs, nseg, tile)];
-    const int m = (int)S.n, d = S.aux & 255, check = S.aux >> 8;
-    const int local = tile - S.blk0, per = S.gx * S.gx;
+    const VSeg &V = segs[vseg_find(segs, nseg, tile)];
+    const int local = tile - V.blk0, per = V.gx * V.gx;
     const int prob = local / per, r = local - prob * per;
-    const int ti = r % S.gx, tj = r / S.gx;
-    const RGemm *tab = reinterpret_cast<const RGemm *>(base + S.arg);
-    const int m0 = m >> d, ld = residue_pitch(m0);
-    if (check)
-      oz_tile<true>(tab, m, nmod, kc, m0, ld, d, prob, ti, tj, As, Bs);
-    else
-      oz_tile<false>(tab, m, nmod, kc, m0, ld, d, prob, ti, tj, As, Bs);
+    const RGemm *tab = reinterpret_cast<const RGemm *>(base + V.arg);
+    mid_tile<BT>(tab, (int)V.n, nmod, kc, V.aux, prob, r % V.gx, r / V.gx, S);
   }
 }
 
@@ -336,7 +380,7 @@ __global__ __launch_bounds__(T256) void oz_igemm_multi_kernel(const char *__rest
 // directly (MUBUF buffer_load ... lds: each lane's 16 bytes land at the
 // wave's LDS base + 16 * lane), double-buffered, so no registers hold the
 // next stage.  Per MAC this reads 3/4 of the LDS bytes and half the L2 bytes
-// of the 128 x 128 kernel above.  Leaves of m0 % 256 == 0, or (EDGE) plain
+// of 128 x 128 tiles.  Leaves of m0 % 256 == 0, or (EDGE) plain
 // leaves of any size with partial last tiles.
 //
 // LDS stage layout per operand: 256 rows x 8 chunks of 16 bytes (k), no
@@ -369,13 +413,6 @@ constexpr int JSTAGE = JBM * JBK;  // 32 KB per operand per stage
 constexpr int JPF = 2;             // prefetch distance, K-steps
 
 __device__ __forceinline__ int jswz(int r) { return (r >> 1) & 7; }
-
-typedef __attribute__((address_space(3))) void *lds_ptr;
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const int8_t *p, long long bytes) {
-  // raw buffer over one operand's quadtree (bytes < 2^31 for m <= 46340)
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(p), 0, (int)bytes, 0x00020000);
-}
 
 // one stage: wave w loads rows 8 (8 j + w) .. + 7 of A and of B, 8 lanes per
 // 128-byte row; for those rows swz(r) = ((w & 1) << 2) | (rl >> 1).
@@ -418,15 +455,6 @@ __device__ __forceinline__ void stage_load_edge(__amdgpu_buffer_rsrc_t ra,
     __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr)(As + slot0 * 16), 16, ao, 0, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr)(Bs + slot0 * 16), 16, bo, 0, 0, 0);
   }
-}
-
-// block barrier for LDS stages filled by this wave's own loads: the caller
-// has waited for them (vmcnt) and consumed every LDS read of the stage it
-// leaves; the empty asm statements keep memory operations on their side
-__device__ __forceinline__ void stage_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 }
 
 struct BigTile {
@@ -681,6 +709,30 @@ oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
 // INT8 kernel's bit for bit.  128 x 128 tiles, 4 waves of 64 x 64, BK = 64.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+constexpr int IBM = 128, IBN = 128, IBK = 64;
+
+// global -> registers: 128 rows of A (k contiguous) and 128 columns of B
+// (k contiguous), 64 k each, 16 bytes per access.  Ab / Bb point at the
+// slice's first element, ld is the row (A) / column (B) stride.  CHECK: rows /
+// columns against m, 16-byte K chunks against ld; checks use the slice origin,
+// plain operands only.
+
+template <bool CHECK>
+__device__ __forceinline__ void gload_i8(const int8_t *__restrict__ Ab,
+                                         const int8_t *__restrict__ Bb, int ld, int m, int row0,
+                                         int col0, int k0, int tid, v4u (&ga)[2], v4u (&gb)[2]) {
+#pragma unroll
+  for (int it = 0; it < 2; it++) {
+    const int idx = tid + T256 * it;
+    const int r = idx >> 2, kq = (idx & 3) * 16;
+    const v4u z = {0u, 0u, 0u, 0u};
+    const bool kin = !CHECK || k0 + kq < ld;
+    const long long off = (long long)r * ld + kq;
+    ga[it] = kin && (!CHECK || row0 + r < m) ? *reinterpret_cast<const v4u *>(Ab + off) : z;
+    gb[it] = kin && (!CHECK || col0 + r < m) ? *reinterpret_cast<const v4u *>(Bb + off) : z;
+  }
+}
+
 constexpr int BSTR = IBK * 2 + 16;  // LDS row stride (bytes) of BF16 rows
 constexpr int BFOLD = 512;          // K between folds
 
@@ -1098,27 +1150,83 @@ hipError_t launch_residue_gemm_bf16(const RGemm *tab, int count, int m, int leve
   return hipGetLastError();
 }
 
-// the large-tile kernel with partial edges for plain leaves (levels = 0) of
-// m <= 16384, when the padding to 256 x 256 tiles adds at most half the area
-// (m >= 512 at worst): at 0.4 of peak it beats the 128 x 128 kernel there
-bool big_edge_gemm(int m, int levels, int tile) {
-  if (tile != 0 || levels != 0 || m % JBM == 0 || residue_pitch(m) > 16384 || m < 512)
-    return false;
-  const long long padded = (long long)((m + JBM - 1) / JBM) * JBM;
-  return 2 * padded * padded <= 3LL * m * m;
-}
-
-// whole 256 x 256 tiles: one block (8 waves, 128 KB of LDS) per CU; buffer
-// offsets are 32-bit, so an operand quadtree stays below 2 GiB
+// whole 256 x 256 tiles: buffer offsets are 32-bit, so an operand quadtree
+// stays below 2 GiB
 static bool big_int8_gemm(int m, int levels, int tile) {
   const int m0 = m >> levels;
   return tile == 0 && m0 % JBM == 0 && (long long)m * m < (1LL << 31);
 }
 
-bool residue_gemm_segmented(int m, int levels, int tile, bool bf16) {
+bool residue_gemm_segmented(int m, int levels, int tile, bool bf16, long long problems) {
   if (m <= 0 || levels < 0 || ((m >> levels) << levels) != m) return false;
-  return bf16 ? (m >> levels) % JBM == 0 : big_int8_gemm(m, levels, tile);
+  if (bf16) return (m >> levels) % JBM == 0;
+  return big_int8_gemm(m, levels, tile) && residue_block_tile(m, levels, tile, problems) == 256;
 }
+
+// Cost of a launch: the busiest CU runs ceil(tiles / CUs) tiles of bt^2
+// outputs over K + epi, epi being the K that a tile's start and epilogue cost
+// as much as, at the tile's rate (POP/s over the device; the smaller tiles
+// load more operand bytes per product).  Both are fitted to launches of 686
+// products of orders 128 to 1000, in us with 256 / 192 / 160 / 128 / 96 / 64
+// tiles: order 128 26 25 18 14 24 19; 160 33 29 21 34 27 26; 320 120 88 67 77
+// 91 85; 384 127 107 123 97 120 135; 512 172 226 265 196 287 311; 640 421 475
+// 377 384 521 639; 750 572 676 708 769 936 1366; 1000 1177 1485 1608 1591 2359
+// 3097.  The 128 x 128 kernel these tiles replaced (registers between memory
+// and LDS, two blocks per CU) took 122 at 320 and 395 at 640.
+double residue_tile_cost(int bt, double tiles, int K) {
+  struct {
+    int bt;
+    double rate, epi;
+  } const t[] = {{256, 1.7, 230}, {192, 1.6, 390}, {160, 1.35, 250},
+                 {128, 1.1, 100}, {96, 1.0, 190},  {64, 0.57, 60}};
+  for (const auto &e : t)
+    if (e.bt == bt) return ceil(tiles / device_cu_count()) * bt * bt * (K + e.epi) / e.rate;
+  return INFINITY;
+}
+
+int residue_block_tile(int m, int levels, int tile, long long problems) {
+  const int m0 = m >> levels, K = levels > 0 ? m : residue_pitch(m);
+  // the one-pass reduction of partial 256 tiles needs K <= 16384
+  const bool big = tile == 0 && (m0 % JBM == 0 ? big_int8_gemm(m, levels, tile)
+                                               : levels == 0 && K <= 16384);
+  int best = 64;
+  double cost = INFINITY;
+  for (int bt : {256, 192, 160, 128, 96, 64}) {
+    if (bt == 256 ? !big : (levels > 0 && m0 % bt != 0)) continue;
+    const double t = (m + bt - 1) / bt;
+    const double c = residue_tile_cost(bt, t * t * (double)problems, K);
+    if (c < cost) {
+      best = bt;
+      cost = c;
+    }
+  }
+  return best;
+}
+
+namespace {
+
+template <int BT>
+hipError_t launch_mid(const RGemm *tab, int count, int m, int levels, int nmod,
+                      const OzakiConsts *kc, hipStream_t s) {
+  bool ok;
+  TileMap map = make_tilemap(m, BT, (long long)count * nmod, ok);
+  if (!ok) return hipErrorInvalidValue;
+  const int G = persistent_grid(Mid<BT>::OCC, device_cu_count(), map.total);
+  hipLaunchKernelGGL((oz_igemm_mid_kernel<BT>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
+                     levels);
+  return hipGetLastError();
+}
+
+template <int BT>
+hipError_t launch_mid_multi(const char *base, const VSeg *segs, int nseg, int total, int nmod,
+                            const OzakiConsts *kc, hipStream_t s) {
+  const int G = persistent_grid(Mid<BT>::OCC, device_cu_count(), total);
+  hipLaunchKernelGGL((oz_igemm_multi_kernel<BT>), dim3(G), dim3(T256), 0, s, base, segs, nseg,
+                     total, nmod, kc);
+  return hipGetLastError();
+}
+
+}  // namespace
 
 hipError_t launch_residue_gemm(const RGemm *tab, int count, int m, int levels, int nmod,
                                const OzakiConsts *kc, hipStream_t s, int tile) {
@@ -1126,51 +1234,44 @@ hipError_t launch_residue_gemm(const RGemm *tab, int count, int m, int levels, i
   if (nmod < 2 || nmod > OZ_MAX_MODULI) return hipErrorInvalidValue;
   const int m0 = m >> levels;
   if (levels < 0 || (m0 << levels) != m) return hipErrorInvalidValue;
-  bool ok;
-  if (big_int8_gemm(m, levels, tile)) {
-    TileMap map = make_tilemap(m, JBM, (long long)count * nmod, ok);
-    if (!ok) return hipErrorInvalidValue;
-    const int G = persistent_grid(1, device_cu_count(), map.total);
-    if (m <= 16384)
-      hipLaunchKernelGGL((oz_igemm_big_kernel<true, false>), dim3(G), dim3(JT), 0, s, tab, m,
-                         nmod, kc, map, m0, m0, levels);
-    else
-      hipLaunchKernelGGL((oz_igemm_big_kernel<false, false>), dim3(G), dim3(JT), 0, s, tab, m,
-                         nmod, kc, map, m0, m0, levels);
-    return hipGetLastError();
+  if (levels > 0 && m0 % 128 != 0) return hipErrorInvalidValue;  // quadtrees need whole tiles
+  switch (residue_block_tile(m, levels, tile, (long long)count * nmod)) {
+    case 64: return launch_mid<64>(tab, count, m, levels, nmod, kc, s);
+    case 96: return launch_mid<96>(tab, count, m, levels, nmod, kc, s);
+    case 128: return launch_mid<128>(tab, count, m, levels, nmod, kc, s);
+    case 160: return launch_mid<160>(tab, count, m, levels, nmod, kc, s);
+    case 192: return launch_mid<192>(tab, count, m, levels, nmod, kc, s);
   }
-  if (big_edge_gemm(m, levels, tile)) {
-    // plain operands of any order on the large tiles, partial edges
-    TileMap map = make_tilemap(m, JBM, (long long)count * nmod, ok);
-    if (!ok) return hipErrorInvalidValue;
-    const int G = persistent_grid(1, device_cu_count(), map.total);
+  // 256 x 256 tiles: one block (8 waves, 128 KB of LDS) per CU
+  bool ok;
+  TileMap map = make_tilemap(m, JBM, (long long)count * nmod, ok);
+  if (!ok) return hipErrorInvalidValue;
+  const int G = persistent_grid(1, device_cu_count(), map.total);
+  if (m0 % JBM != 0)
+    // plain operands of any order, partial edges
     hipLaunchKernelGGL((oz_igemm_big_kernel<true, true>), dim3(G), dim3(JT), 0, s, tab, m, nmod,
                        kc, map, m0, residue_pitch(m0), levels);
-    return hipGetLastError();
-  }
-  TileMap map = make_tilemap(m, IBM, (long long)count * nmod, ok);
-  if (!ok) return hipErrorInvalidValue;
-  const int G = persistent_grid(2, device_cu_count(), map.total);
-  const bool fast = (m0 % IBM == 0);
-  if (!fast && levels > 0) return hipErrorInvalidValue;  // quadtree operands need whole tiles
-  const int ld = residue_pitch(m0);
-  if (fast)
-    hipLaunchKernelGGL((oz_igemm_kernel<false>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
-                       m0, ld, levels);
+  else if (m <= 16384)
+    hipLaunchKernelGGL((oz_igemm_big_kernel<true, false>), dim3(G), dim3(JT), 0, s, tab, m, nmod,
+                       kc, map, m0, m0, levels);
   else
-    hipLaunchKernelGGL((oz_igemm_kernel<true>), dim3(G), dim3(T256), 0, s, tab, m, nmod, kc, map,
-                       m0, ld, levels);
+    hipLaunchKernelGGL((oz_igemm_big_kernel<false, false>), dim3(G), dim3(JT), 0, s, tab, m, nmod,
+                       kc, map, m0, m0, levels);
   return hipGetLastError();
 }
 
-hipError_t launch_residue_gemm_multi(const char *base, const VSeg *segs, int nseg, int total,
-                                     int nmod, const OzakiConsts *kc, hipStream_t s) {
+hipError_t launch_residue_gemm_multi(int bt, const char *base, const VSeg *segs, int nseg,
+                                     int total, int nmod, const OzakiConsts *kc, hipStream_t s) {
   if (nseg <= 0 || total <= 0) return hipSuccess;
   if (nmod < 2 || nmod > OZ_MAX_MODULI) return hipErrorInvalidValue;
-  const int G = persistent_grid(2, device_cu_count(), total);
-  hipLaunchKernelGGL(oz_igemm_multi_kernel, dim3(G), dim3(T256), 0, s, base, segs, nseg, total,
-                     nmod, kc);
-  return hipGetLastError();
+  switch (bt) {
+    case 64: return launch_mid_multi<64>(base, segs, nseg, total, nmod, kc, s);
+    case 96: return launch_mid_multi<96>(base, segs, nseg, total, nmod, kc, s);
+    case 128: return launch_mid_multi<128>(base, segs, nseg, total, nmod, kc, s);
+    case 160: return launch_mid_multi<160>(base, segs, nseg, total, nmod, kc, s);
+    case 192: return launch_mid_multi<192>(base, segs, nseg, total, nmod, kc, s);
+  }
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_ozaki_step(int step, const OzLeaf *tab, int count, int m, int nmod,

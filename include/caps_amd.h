@@ -104,8 +104,9 @@ typedef struct caps_opts {
 /* Run two leading 'b' levels as separate passes instead of the fused
  * two-level kernels (same results; for testing and timing comparisons). */
 #define CAPS_FLAG_NO_FUSION 8
-/* Leaf GEMMs on the smaller block tile: INT8 residue products 128 x 128
- * instead of 256 x 256, FP64 64 x 64 instead of 128 x 128 (same results; the
+/* Leaf GEMMs on a smaller block tile: INT8 residue products on the best of
+ * the tiles below 256 x 256, FP64 on 64 x 64 (same results; the default picks
+ * the tile by the leaf size and how well it fills the device; this is the
  * autotuner's tile dimension, caps_candidate.tile). */
 #define CAPS_FLAG_SMALL_TILE 16
 
@@ -145,10 +146,10 @@ int caps_multiply_device(const double *dA, const double *dB, double *dC,
 /* Same as caps_multiply_device, for callers that cannot allocate device
  * memory (code under stream capture, tight serving loops): it calls no
  * hipMalloc / hipFree.  No counterpart in the reference.  The pointer tables
- * and workspace live in a scratch array of twice CAPS_NOALLOC_SCRATCH_MIB MiB
- * that every device the library runs on holds from module load until the
- * process ends; a call whose plan needs more than CAPS_NOALLOC_SCRATCH_MIB MiB,
- * not counting the padding of residue leaves to 16 bytes, returns CAPS_ENOMEM
+ * and workspace live in a fixed scratch array that every device the library
+ * runs on holds from module load until the process ends; a call whose plan
+ * needs more than CAPS_NOALLOC_SCRATCH_MIB MiB, not counting the padding of
+ * residue leaves to 16 bytes (the array has room for it), returns CAPS_ENOMEM
  * (e.g. FP64 n = 2048 'bd' fits, residue mode n = 1024 'bb' fits).  No graph: the steps are
  * enqueued one by one on `stream`.  CAPS_MODE_AUTO is not accepted.  All calls
  * on one device share its scratch (it keeps the last call's contents; no step

@@ -76,6 +76,28 @@ def test_ragged_large_leaves_agree(m):
     assert np.array_equal(_run(A, B, n, 1, 1, "b", BF16), want)
 
 
+@pytest.mark.parametrize("m", [50, 64, 90, 96, 97, 126, 128, 150, 160, 161, 300, 320, 380, 384,
+                               570, 576, 640])
+def test_int8_tiles_equal_bf16(m):
+    """686 INT8 products on each of the block tiles 64, 96, 128, 160, 192 and
+    256, whole and partial, give the bits of the BF16 kernels (another tile,
+    another accumulation)."""
+    n = 4 * m
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m)
+    A, B = torch.rand((2, n * n), generator=g, device="cuda", dtype=torch.float64) * 2 - 1
+    d = caps_amd.MatDescriptor.one_device(n, 2, 1)
+    out = []
+    for mode, flags in ((BF16, 0), (INT8, 0), (INT8, caps_amd.FLAG_SMALL_TILE)):
+        print(f"[gpu] n={n} bb mode={mode} flags={flags}", flush=True)
+        C = torch.full_like(A, float("nan"))
+        caps_amd.multiply_device(A, B, C, d, "bb", mode=mode, flags=flags)
+        torch.cuda.synchronize()
+        out.append(C)
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    caps_amd.release()
+
+
 @pytest.mark.parametrize("m", [1, 15, 18, 49, 66])
 def test_leaf_split_ragged(m):
     n = 2 * m
