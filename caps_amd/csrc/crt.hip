@@ -127,7 +127,7 @@ __global__ __launch_bounds__(T) void crt_finalize_kernel(const CrtMats *__restri
 // rows x 128 k.  PLAIN (the leaf column-major, bs == 1 or bs == m): the
 // column-major side moves as 256-byte column pieces; the row-major side moves
 // as 128-byte row pieces (8 lanes x 16 residues).  Elements past m are zero,
-// 16-byte chunks past the pitch skipped.  Column c of the tile in T2[c], row r
+// 16-byte chunks past residue_k skipped.  Column c of the tile in T2[c], row r
 // at slot r ^ tswz(c); the transposed read has lanes on 8 rows and 8 column
 // groups, the swizzle puts 4 of the groups 8 slots apart (the other 4 pairs
 // share a slot: a 64-lane 8-byte read spans at least two 256-byte passes
@@ -199,7 +199,7 @@ __device__ __forceinline__ void split_b_body(const CrtMats *__restrict__ M,
   const double *B = M->B + (long long)L * m * m;
   int8_t *rb = M->rb + L * residue_area(m);
   const long long plane = M->plane;
-  const int c16 = residue_pitch(m) / 16;
+  const int ld = residue_pitch(m), c16 = residue_k(m) / 16;
   const long long units = (long long)m * c16;
   for (long long u = (long long)bx * T + threadIdx.x; u < units; u += (long long)gx * T) {
     const int lj = (int)(u / c16), li = (int)(u - (long long)lj * c16) * 16;
@@ -227,7 +227,8 @@ __device__ __forceinline__ void split_b_body(const CrtMats *__restrict__ M,
           v |= (unsigned)(sym_residue(x[4 * q + b], mi, inv, c22) & 0xff) << (8 * b);
         w[q] = v;
       }
-      *reinterpret_cast<uint4 *>(rb + l * plane + 16 * u) = make_uint4(w[0], w[1], w[2], w[3]);
+      *reinterpret_cast<uint4 *>(rb + l * plane + (long long)lj * ld + li) =
+          make_uint4(w[0], w[1], w[2], w[3]);
     }
   }
 }
@@ -479,7 +480,7 @@ bool crt_grid(int k, const CrtMats &h, int &gx, int &gy) {
       gy = leaves;
       return plain;
     case CRT_SPLIT_B:
-      gx = (int)capped_blocks(residue_area(h.m) / 16, leaves);
+      gx = (int)capped_blocks((long long)h.m * residue_k(h.m) / 16, leaves);
       gy = leaves;
       return plain;
     case CRT_RECON:

@@ -200,20 +200,21 @@ __global__ __launch_bounds__(T) void bb_pre_res_kernel(const BBPre *__restrict__
 }
 
 // ------------------------------------------------ residue pre of B fused with the split
-// thread: 2 consecutive positions of one leaf column (the pitch is even; rows
-// past m0 are zero).  The 16 FP64 inputs are scaled by their global columns'
+// thread: 2 consecutive positions of one leaf column (the pitch is even;
+// positions past m0 are zero).  The 16 FP64 inputs are scaled by their global columns'
 // exponents and truncated once, exactly as the separate split does; then for
 // every modulus they are reduced to symmetric residues and combined into all
 // 49 depth-2 operands.  Per position: 16 x 8 bytes in, 49 x nmod bytes out.
-// RAGGED: the pitch is larger than m0 (the row checks around the 16 loads cost
-// 13 % at n = 8192, so leaves without padding have their own instantiation).
+// RAGGED: the leaf is padded (the checks around the 16 loads cost 13 % at n =
+// 8192, so leaves without padding have their own instantiation).
 template <bool RAGGED>
 __global__ __launch_bounds__(T) void bb_split_b_kernel(const BBSplitB *__restrict__ P,
                                                        long long q,
                                                        const OzakiConsts *__restrict__ kc) {
   const int nmod = kc->nmod;
   const unsigned n2 = (unsigned)(q >> 1);
-  const unsigned m0 = (unsigned)P->m0, ld = residue_pitch(P->m0), mm0 = m0 * ld;
+  const unsigned m0 = (unsigned)P->m0, ld = RAGGED ? residue_pitch(P->m0) : m0;
+  const unsigned mm0 = RAGGED ? (unsigned)residue_area(P->m0) : m0 * m0;
   const int sub = P->sub;
   const long long qs = (long long)sub * sub;  // elements of an FP64 sub-block
   for (unsigned u = blockIdx.x * T + threadIdx.x; u < n2; u += gridDim.x * T) {
@@ -226,14 +227,15 @@ __global__ __launch_bounds__(T) void bb_split_b_kernel(const BBSplitB *__restric
     const double *src = P->B + (long long)L2 * m0 * m0 + (long long)lj * m0 + li;
     int sc[4];  // exponent of column half (a >> 1, b >> 1) as index 2 (a >> 1) + (b >> 1)
 #pragma unroll
-    for (int h = 0; h < 4; h++) sc[h] = P->sb[(h >> 1) * 2 * sub + (h & 1) * sub + cj];
+    for (int h = 0; h < 4; h++)
+      sc[h] = RAGGED && lj >= m0 ? 0 : P->sb[(h >> 1) * 2 * sub + (h & 1) * sub + cj];
     double x[16][2];
 #pragma unroll
     for (int k = 0; k < 16; k++) {
       v2du v = {0.0, 0.0};
-      if (!RAGGED || li + 1 < m0)
+      if (!RAGGED || (li + 1 < m0 && lj < m0))
         v = *reinterpret_cast<const v2du *>(src + k * qs);
-      else if (li < m0)
+      else if (li < m0 && lj < m0)
         v.x = src[k * qs];
       const int s = sc[2 * (k >> 3) + ((k & 3) >> 1)];
       x[k][0] = trunc(ldexp(v.x, s));
@@ -446,7 +448,7 @@ __global__ __launch_bounds__(T) void bb_post_crt_kernel(const BBPost *__restrict
 
   const int m0 = P->m0, sub = P->sub, nrec2 = P->nrec2, bs = P->bs;
   const int ld = residue_pitch(m0);
-  const long long mm0 = (long long)m0 * ld, qs = (long long)sub * sub;
+  const long long mm0 = residue_area(m0), qs = (long long)sub * sub;
   // lane -> one position pl (T is a multiple of PPOS) and outputs o = o0, o0 + T / PPOS, ...
   const int pl = threadIdx.x % PPOS, o0 = threadIdx.x / PPOS;
   const long long u = pos0 + pl;
@@ -454,7 +456,7 @@ __global__ __launch_bounds__(T) void bb_post_crt_kernel(const BBPost *__restrict
   // position u of a depth-2 sub-block: leaf L2 (quadtree of nrec2 levels), column-major leaf
   const long long L2 = u / mm0, e = u - L2 * mm0;
   const int li = (int)(e % ld), lj = (int)(e / ld);
-  if (li >= m0) return;  // the pitch's padding
+  if (li >= m0 || lj >= m0) return;  // the leaf's padding
   int bi, bj;
   leaf_coords((int)L2, nrec2, bi, bj);
   const long long dst_in_sub = L2 * m0 * m0 + leaf_elem_offset(m0, bs, li, lj);
@@ -511,7 +513,7 @@ hipError_t launch_bb_split_b(const BBSplitB *P, long long q, int m0, const Ozaki
                              hipStream_t s) {
   if (m0 <= 0 || q % residue_area(m0) || q >= (1LL << 31)) return hipErrorInvalidValue;
   const dim3 g(blocks_for(q / 2, 1));
-  if (residue_pitch(m0) != m0)
+  if (residue_area(m0) != (long long)m0 * m0)
     hipLaunchKernelGGL((bb_split_b_kernel<true>), g, dim3(T), 0, s, P, q, kc);
   else
     hipLaunchKernelGGL((bb_split_b_kernel<false>), g, dim3(T), 0, s, P, q, kc);

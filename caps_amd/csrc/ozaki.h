@@ -38,7 +38,8 @@ struct OzakiConsts {
   int nmod;
   int npieces;
   int m[OZ_MAX_MODULI];
-  int c14[OZ_MAX_MODULI];                  // 2^14 mod m_l, symmetric (|c14| <= m_l / 2)
+  unsigned dot16[OZ_MAX_MODULI];           // 1 | (2^16 mod m_l) << 16: halves of a sum (residue_of_sum)
+  int bias[OZ_MAX_MODULI];                 // least multiple of m_l >= 2^28: keeps sums positive
   int c22[OZ_MAX_MODULI];                  // round(2^22 / m_l): quotients of small sums (mod_k)
   double inv_m[OZ_MAX_MODULI];
   double w[OZ_MAX_MODULI][OZ_MAX_PIECES];  // CRT weight W_l in base 2^37 digits
@@ -49,13 +50,28 @@ struct OzakiConsts {
 };
 
 // Residue planes store a leaf of order m0 with rows (A side) or columns (B and
-// C side) of residue_pitch(m0) bytes, the bytes past m0 zero: 16-byte chunks
-// are aligned and wholly inside or outside the pitch for every leaf size, so
-// no kernel reads residues byte by byte, and zero k positions add nothing to
-// a product.
-__host__ __device__ constexpr int residue_pitch(int m0) { return (m0 + 15) & ~15; }
+// C side) at a pitch of residue_pitch(m0) bytes, of which the first
+// residue_k(m0) hold residues, zero past m0: 16-byte chunks are aligned and
+// wholly inside or outside for every leaf size, so no kernel reads residues
+// byte by byte, and zero k positions add nothing to a product.  Bytes past
+// residue_k, and past the rows in residue_area, are never part of a result.
+//
+// The pitch is the largest of the multiples of 128, 64, 32 and 16 that adds at
+// most 1/32, and a leaf fills whole 128-byte lines where that adds at most
+// 1/32: rows and planes that straddle lines cost the leaf GEMM and the passes
+// more than the padding.  Leaves of 750 (n = 3000, r = 2) at a pitch of 752:
+// 0.53 ms in the GEMM, 0.22 in B's split.
+__host__ __device__ constexpr int residue_k(int m0) { return (m0 + 15) & ~15; }
+__host__ __device__ constexpr int residue_pitch(int m0) {
+  for (int a = 128; a > 16; a /= 2) {
+    const int p = (m0 + a - 1) / a * a;
+    if (32LL * p <= 33LL * m0) return p;
+  }
+  return residue_k(m0);
+}
 __host__ __device__ constexpr long long residue_area(int m0) {
-  return (long long)m0 * residue_pitch(m0);
+  const long long a = (long long)m0 * residue_pitch(m0);
+  return a >= 4096 ? (a + 127) / 128 * 128 : a;
 }
 
 struct OzLeaf {
@@ -64,7 +80,7 @@ struct OzLeaf {
   double *C;
   int *ea;          // m row exponents of A
   int *eb;          // m column exponents of B
-  int8_t *ra;       // nmod planes of residue_area(m), row-major
+  int8_t *ra;       // nmod planes of residue_area(m), row-major leaf
   int8_t *rb;       // nmod planes, column-major
   int8_t *rc;       // nmod planes, column-major (product residues)
   double *pa;       // OZ_CHUNKS x m partial row sums of squares (A)

@@ -76,7 +76,7 @@ __global__ __launch_bounds__(T256) void oz_finalize_kernel(const OzLeaf *__restr
 
 // ------------------------------------------------------------------ split
 // A (column-major) -> nmod row-major INT8 planes; 64 x 64 tiles through LDS.
-// CHECK: m % 64 != 0; elements past m are zero, chunks past the pitch skipped.
+// CHECK: m % 64 != 0; elements past m are zero, chunks past residue_k skipped.
 template <bool CHECK>
 __global__ __launch_bounds__(T256) void oz_split_a_kernel(const OzLeaf *__restrict__ tab, int m,
                                                           int nmod,
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(T256) void oz_split_b_kernel(const OzLeaf *__restri
                                                           int nmod,
                                                           const OzakiConsts *__restrict__ kc) {
   const OzLeaf &L = tab[blockIdx.y];
-  const int c16 = residue_pitch(m) / 16;
+  const int ld = residue_pitch(m), c16 = residue_k(m) / 16;
   const long long total16 = (long long)m * c16;
   const long long plane = residue_area(m);
   for (long long u = (long long)blockIdx.x * T256 + threadIdx.x; u < total16;
@@ -150,7 +150,8 @@ __global__ __launch_bounds__(T256) void oz_split_b_kernel(const OzLeaf *__restri
           v |= (unsigned)(sym_residue(x[4 * q + b], mi, inv, c22) & 0xff) << (8 * b);
         w[q] = v;
       }
-      *reinterpret_cast<uint4 *>(L.rb + l * plane + 16 * u) = make_uint4(w[0], w[1], w[2], w[3]);
+      *reinterpret_cast<uint4 *>(L.rb + l * plane + (long long)j * ld + i0) =
+          make_uint4(w[0], w[1], w[2], w[3]);
     }
   }
 }
@@ -173,6 +174,17 @@ __device__ __forceinline__ void stage_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// a uniform pointer kept in scalar registers (buffer descriptors built from a
+// pointer the compiler thinks may vary per lane are used through per-lane
+// loops)
+template <typename P>
+__device__ __forceinline__ P *uniform_ptr(P *p) {
+  const unsigned long long v = reinterpret_cast<unsigned long long>(p);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+  return reinterpret_cast<P *>(((unsigned long long)hi << 32) | lo);
+}
+
 // a raw buffer of `bytes` (< 2^31) from p on
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const int8_t *p, long long bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(p), 0, (int)bytes, 0x00020000);
@@ -185,7 +197,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const int8_t *p, lo
 // the device idle in.  Several blocks share a CU (2 to 8), so one block's
 // epilogue, barriers and load latency run under the others' MFMAs.  Operands
 // go global -> LDS by buffer loads that write LDS directly, double-buffered;
-// rows past the leaf and 16-byte chunks past its pitch get an offset past the
+// rows past the leaf and 16-byte chunks past residue_k get an offset past the
 // buffer (the range check returns zeros).  LDS rows are 64 bytes; chunk c of
 // row r sits in slot c ^ ((r >> 2) & 3), so the 16 rows of one ds_read_b128
 // cycle cover the 64 banks once.  C leaves through LDS (columns of BT / 4 + 4
@@ -198,7 +210,7 @@ struct Mid {
   static constexpr int MT = WT / 16;      // MFMA tiles per wave dimension
   static constexpr int STAGE = BT * MBK;  // bytes of one operand's stage
   static constexpr int CP = BT / 4 + 4;   // words of a staged C column
-  static constexpr int OCC = BT == 64 ? 8 : (BT == 96 ? 5 : (BT == 128 ? 4 : (BT == 160 ? 3 : 2)));
+  static constexpr int OCC = BT == 64 ? 8 : (BT == 96 ? 6 : (BT == 128 ? 4 : (BT == 160 ? 3 : 2)));
   static_assert(BT * CP * 4 <= 4 * STAGE, "C is staged in the operands' LDS");
 };
 
@@ -222,13 +234,13 @@ __device__ __forceinline__ void mid_tile(const RGemm *__restrict__ tab, int m, i
   const int wm = wave & 1, wn = wave >> 1;
   const int l16 = lane & 15, lk = lane >> 4;
   const int m0 = m >> d, ld = residue_pitch(m0);
-  const int K = d == 0 ? ld : m, nk = (K + MBK - 1) / MBK;
+  const int K = d == 0 ? residue_k(m) : m, nk = (K + MBK - 1) / MBK;
   const int leaf = prob / nmod, l = prob - leaf * nmod;
-  const int8_t *Ap = tab[leaf].a + l * tab[leaf].sa;  // row-major
-  const int8_t *Bp = tab[leaf].b + l * tab[leaf].sb;  // column-major
-  int8_t *Cp = tab[leaf].c + l * tab[leaf].sc;
+  const int8_t *Ap = uniform_ptr(tab[leaf].a + l * tab[leaf].sa);  // row-major
+  const int8_t *Bp = uniform_ptr(tab[leaf].b + l * tab[leaf].sb);  // column-major
+  int8_t *Cp = uniform_ptr(tab[leaf].c + l * tab[leaf].sc);
   const int mi = kc->m[l];
-  const float mf = (float)mi, invf = 1.0f / mf;
+  const float invf = 1.0f / (float)mi;
   const int row0 = ti * BT, col0 = tj * BT;
   const long long mm0 = (long long)m0 * ld;
 
@@ -275,9 +287,9 @@ __device__ __forceinline__ void mid_tile(const RGemm *__restrict__ tab, int m, i
     }
   };
 
-  // small K: the sums start at 128 for the one-pass reduction res_byte128
+  // small K: the sums start at a positive bias for residue_of_sum
   const bool small_k = K <= 16384;
-  const int bias = small_k ? 128 : 0;
+  const int bias = small_k ? kc->bias[l] : 0;
   v4i acc[MT][MT];
 #pragma unroll
   for (int r = 0; r < MT; r++)
@@ -307,29 +319,35 @@ __device__ __forceinline__ void mid_tile(const RGemm *__restrict__ tab, int m, i
 
   // D layout: lane holds column (lane % 16), rows 4 * (lane / 16) + v
   unsigned *Cw = reinterpret_cast<unsigned *>(S);
-  const int c14m = kc->c14[l] - 16384;
-  const float cl = 0.5f - 128.0f * invf;
+  unsigned *Cl = Cw + (wn * WT + l16) * P::CP + wm * (WT / 4) + lk;
+  if (small_k) {
+    const unsigned dot16 = kc->dot16[l];
 #pragma unroll
-  for (int r = 0; r < MT; r++)
+    for (int r = 0; r < MT; r++)
 #pragma unroll
-    for (int c = 0; c < MT; c++) {
-      unsigned v = 0;
-      if (small_k) {
+      for (int c = 0; c < MT; c++) {
+        int e[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) v = res_byte128(acc[r][c][q], c14m, mf, invf, cl, q, v);
-        v ^= 0x80808080u;
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; q++) v |= (unsigned)(mod_i32(acc[r][c][q], mi, invf) & 0xff) << (8 * q);
+        for (int q = 0; q < 4; q++) e[q] = residue_of_sum(acc[r][c][q], dot16, invf, mi);
+        Cl[c * 16 * P::CP + r * 4] = pack4_lo(e[0], e[1], e[2], e[3]);
       }
-      Cw[(wn * WT + c * 16 + l16) * P::CP + wm * (WT / 4) + r * 4 + lk] = v;
-    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < MT; r++)
+#pragma unroll
+      for (int c = 0; c < MT; c++) {
+        int e[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) e[q] = mod_i32(acc[r][c][q], mi, invf);
+        Cl[c * 16 * P::CP + r * 4] = pack4_lo(e[0], e[1], e[2], e[3]);
+      }
+  }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   stage_barrier();
   int8_t *Ct = Cp + (d == 0 ? (long long)col0 * ld + row0
                             : quad_leaf(row0 / m0, col0 / m0, d) * mm0 +
                                   (long long)(col0 % m0) * ld + row0 % m0);
-  const int clim = m - col0, rlim = K - row0;  // rows: to the pitch (d = 0)
+  const int clim = m - col0, rlim = K - row0;  // rows: to residue_k (d = 0)
   for (int idx = tid; idx < BT * (BT / 16); idx += T256) {
     const int col = idx / (BT / 16), j = idx % (BT / 16);
     const v4i v = *reinterpret_cast<const v4i *>(Cw + col * P::CP + 4 * j);
@@ -435,17 +453,17 @@ __device__ __forceinline__ void stage_load(__amdgpu_buffer_rsrc_t ra, __amdgpu_b
 }
 
 // stage_load for plain operands (d = 0) of any order m, pitch ld: rows /
-// columns at or beyond m and 16-byte K chunks at or beyond ld read as zero
+// columns at or beyond m and 16-byte chunks at or beyond K read as zero
 // (their buffer offset is the plane size, past num_records: the buffer range
 // check returns zeros without a memory access)
 __device__ __forceinline__ void stage_load_edge(__amdgpu_buffer_rsrc_t ra,
                                                 __amdgpu_buffer_rsrc_t rb, int row0, int col0,
-                                                int k, int m, int ld, int8_t *As, int8_t *Bs,
+                                                int k, int m, int ld, int K, int8_t *As, int8_t *Bs,
                                                 int wave, int lane) {
   const int rl = lane >> 3;
   const int c = (lane & 7) ^ (((wave & 1) << 2) | (rl >> 1));
   const int oob = m * ld;
-  const bool kin = k + c * 16 < ld;
+  const bool kin = k + c * 16 < K;
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int r = j * 64 + wave * 8 + rl;
@@ -461,21 +479,11 @@ struct BigTile {
   const int8_t *Ap, *Bp;
   int8_t *Cp;
   __amdgpu_buffer_rsrc_t ra, rb;  // buffer descriptors of the operand planes
-  int mi, c14, c22, row0, col0, ti, tj;
+  int mi, bias, row0, col0, ti, tj;
+  unsigned dot16;
   float mf, invf;
   long long cseg;  // C segment stride (RGemm::cseg)
 };
-
-// a uniform pointer kept in scalar registers (buffer descriptors built from a
-// pointer the compiler thinks may vary per lane are used through per-lane
-// loops)
-template <typename P>
-__device__ __forceinline__ P *uniform_ptr(P *p) {
-  const unsigned long long v = reinterpret_cast<unsigned long long>(p);
-  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
-  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-  return reinterpret_cast<P *>(((unsigned long long)hi << 32) | lo);
-}
 
 __device__ __forceinline__ BigTile big_tile(const RGemm *__restrict__ tab, const TileMap &map,
                                             int tile, int nmod,
@@ -491,8 +499,8 @@ __device__ __forceinline__ BigTile big_tile(const RGemm *__restrict__ tab, const
   t.mi = kc->m[l];
   t.mf = (float)t.mi;
   t.invf = 1.0f / t.mf;
-  t.c14 = kc->c14[l];
-  t.c22 = kc->c22[l];
+  t.dot16 = kc->dot16[l];
+  t.bias = kc->bias[l];
   t.row0 = ti * JBM;
   t.col0 = tj * JBM;
   t.ti = ti;
@@ -503,11 +511,11 @@ __device__ __forceinline__ BigTile big_tile(const RGemm *__restrict__ tab, const
 }
 
 // SMALL_K: K = m <= 16384, so |sums| <= m 2^14 < 2^28 and the one-pass
-// exact reduction res_byte128 applies (sums start at 128); larger K takes the
-// general one
+// exact reduction residue_of_sum applies (sums start at a bias); larger K takes
+// the general one
 // EDGE: plain operands (d = 0) whose size m is not a multiple of 256: the last
 // tile row / column and K-step are partial, their missing elements read as
-// zero and the stores beyond m (rows: beyond ld) are skipped.
+// zero and the stores beyond m (rows: beyond residue_k) are skipped.
 template <bool SMALL_K, bool EDGE>
 __global__ __launch_bounds__(JT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
@@ -522,8 +530,7 @@ oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
   const int l16 = lane & 15, lk = lane >> 4;
   const int G = gridDim.x;
   const int ld = EDGE ? pitch : m0;
-  const int nk = ((EDGE ? ld : m) + JBK - 1) / JBK;
-  constexpr int bias = SMALL_K ? 128 : 0;
+  const int K = EDGE ? residue_k(m) : m, nk = (K + JBK - 1) / JBK;
   // read offsets (bytes) of this lane's row l16, chunk lk (kh = 0) and lk + 4 (kh = 1)
   const int s16 = jswz(l16);
   const int rd0 = l16 * JBK + ((lk ^ s16) << 4);
@@ -560,7 +567,7 @@ oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
   };
   auto load = [&](const BigTile &c, int k, int8_t *As, int8_t *Bs) {
     if (EDGE)
-      stage_load_edge(c.ra, c.rb, c.row0, c.col0, k, m, ld, As, Bs, wave, lane);
+      stage_load_edge(c.ra, c.rb, c.row0, c.col0, k, m, ld, K, As, Bs, wave, lane);
     else
       stage_load(c.ra, c.rb, (int)a_off(c.row0, k), (int)b_off(c.col0, k), ld, As, Bs, wave, lane);
   };
@@ -569,6 +576,7 @@ oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
   __syncthreads();
 
   for (int round = 0;; round++) {
+    const int bias = SMALL_K ? t.bias : 0;
     v4i acc[8][4];
 #pragma unroll
     for (int r = 0; r < 8; r++)
@@ -646,30 +654,17 @@ oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
       const int w = wm * 32 + r * 4 + lk;
       Ch[col * 64 + (w ^ (4 * l16))] = v;
     };
-    if constexpr (SMALL_K) {
-      const int c14m = t.c14 - 16384;
-      const float cl = 0.5f - 128.0f * t.invf;
 #pragma unroll
-      for (int r = 0; r < 8; r++)
+    for (int r = 0; r < 8; r++)
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-          unsigned v = 0;
+      for (int c = 0; c < 4; c++) {
+        int b[4];
 #pragma unroll
-          for (int q = 0; q < 4; q++) v = res_byte128(acc[r][c][q], c14m, t.mf, t.invf, cl, q, v);
-          put(r, c, v ^ 0x80808080u);
-        }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 8; r++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          unsigned v = 0;
-#pragma unroll
-          for (int q = 0; q < 4; q++)
-            v |= (unsigned)(mod_i32(acc[r][c][q], t.mi, t.invf) & 0xff) << (8 * q);
-          put(r, c, v);
-        }
-    }
+        for (int q = 0; q < 4; q++)
+          b[q] = SMALL_K ? residue_of_sum(acc[r][c][q], t.dot16, t.invf, t.mi)
+                         : mod_i32(acc[r][c][q], t.mi, t.invf);
+        put(r, c, pack4_lo(b[0], b[1], b[2], b[3]));
+      }
     // LDS writes done before the barrier; the next tile's first stage (in
     // A0 / B0) may still be loading
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -688,8 +683,8 @@ oz_igemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
       const int ccl = (pass * 32 + (tid >> 4)) & 127;  // pass < 4: A1, else B1
       const unsigned *Cs = reinterpret_cast<const unsigned *>(pass < 4 ? A1 : B1);
       const v4i v = *reinterpret_cast<const v4i *>(Cs + ccl * 64 + ((4 * j16) ^ (4 * (ccl & 15))));
-      // EDGE: ld % 16 == 0, so a 16-row chunk is wholly inside or outside
-      if (!EDGE || (t.col0 + pass * 32 + (tid >> 4) < m && t.row0 + 16 * j16 < ld))
+      // EDGE: K % 16 == 0, so a 16-row chunk is wholly inside or outside
+      if (!EDGE || (t.col0 + pass * 32 + (tid >> 4) < m && t.row0 + 16 * j16 < K))
         *(gv4i *)(Cl + pass * pstep) = v;
     }
     if (!has_next) break;
@@ -714,19 +709,19 @@ constexpr int IBM = 128, IBN = 128, IBK = 64;
 // global -> registers: 128 rows of A (k contiguous) and 128 columns of B
 // (k contiguous), 64 k each, 16 bytes per access.  Ab / Bb point at the
 // slice's first element, ld is the row (A) / column (B) stride.  CHECK: rows /
-// columns against m, 16-byte K chunks against ld; checks use the slice origin,
+// columns against m, 16-byte chunks against K; checks use the slice origin,
 // plain operands only.
 
 template <bool CHECK>
 __device__ __forceinline__ void gload_i8(const int8_t *__restrict__ Ab,
-                                         const int8_t *__restrict__ Bb, int ld, int m, int row0,
+                                         const int8_t *__restrict__ Bb, int ld, int m, int K, int row0,
                                          int col0, int k0, int tid, v4u (&ga)[2], v4u (&gb)[2]) {
 #pragma unroll
   for (int it = 0; it < 2; it++) {
     const int idx = tid + T256 * it;
     const int r = idx >> 2, kq = (idx & 3) * 16;
     const v4u z = {0u, 0u, 0u, 0u};
-    const bool kin = !CHECK || k0 + kq < ld;
+    const bool kin = !CHECK || k0 + kq < K;
     const long long off = (long long)r * ld + kq;
     ga[it] = kin && (!CHECK || row0 + r < m) ? *reinterpret_cast<const v4u *>(Ab + off) : z;
     gb[it] = kin && (!CHECK || col0 + r < m) ? *reinterpret_cast<const v4u *>(Bb + off) : z;
@@ -780,7 +775,7 @@ __global__ __launch_bounds__(T256) void oz_bgemm_kernel(const RGemm *__restrict_
   const int wm = wave & 1, wn = wave >> 1;
   const int l16 = lane & 15, lk = lane >> 4;
   const int G = gridDim.x;
-  const int K = CHECK ? ld : m, nk = (K + IBK - 1) / IBK;
+  const int K = CHECK ? residue_k(m) : m, nk = (K + IBK - 1) / IBK;
   const int fold_every = BFOLD / IBK;
 
   for (int round = 0; round * G < map.total; round++) {
@@ -810,13 +805,13 @@ __global__ __launch_bounds__(T256) void oz_bgemm_kernel(const RGemm *__restrict_
     auto b_at = [&](int k0) {
       return Bp + quad_leaf(k0 / m0, col0 / m0, d) * mm0 + (k0 % m0) + (long long)(col0 % m0) * ld;
     };
-    gload_i8<CHECK>(a_at(0), b_at(0), ld, m, row0, col0, 0, tid, ga, gb);
+    gload_i8<CHECK>(a_at(0), b_at(0), ld, m, K, row0, col0, 0, tid, ga, gb);
     lstore_bf(As[0], Bs[0], tid, ga, gb);
     __syncthreads();
     for (int kt = 0; kt < nk; kt++) {
       const int buf = kt & 1;
       if (kt + 1 < nk)
-        gload_i8<CHECK>(a_at((kt + 1) * IBK), b_at((kt + 1) * IBK), ld, m, row0, col0,
+        gload_i8<CHECK>(a_at((kt + 1) * IBK), b_at((kt + 1) * IBK), ld, m, K, row0, col0,
                         (kt + 1) * IBK, tid, ga, gb);
 #pragma unroll
       for (int kh = 0; kh < 2; kh++) {
@@ -836,7 +831,7 @@ __global__ __launch_bounds__(T256) void oz_bgemm_kernel(const RGemm *__restrict_
           for (int c = 0; c < 4; c++)
             acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r], b[c], acc[r][c], 0, 0, 0);
       }
-      if ((kt + 1) % fold_every == 0) {
+      if ((kt + 1) % fold_every == 0 && kt + 1 < nk) {
 #pragma unroll
         for (int r = 0; r < 4; r++)
 #pragma unroll
@@ -849,8 +844,7 @@ __global__ __launch_bounds__(T256) void oz_bgemm_kernel(const RGemm *__restrict_
     }
 
     // D layout: lane holds column (lane % 16), rows 4 * (lane / 16) + v.
-    // |acc| < 2^24 exact; a fold brings it to |x| <= 1.5 m, then the exact
-    // symmetric residue
+    // |acc| <= 2^23 + 1.5 m, exact
 #pragma unroll
     for (int r = 0; r < 4; r++)
 #pragma unroll
@@ -862,13 +856,10 @@ __global__ __launch_bounds__(T256) void oz_bgemm_kernel(const RGemm *__restrict_
         int res[4];
 #pragma unroll
         for (int q = 0; q < 4; q++)
-          res[q] = mod_k((int)fold_f32(acc[r][c][q], mf, invf), kc->c22[l], mi);  // |.| <= 1.5 m
-        // ld % 16 == 0: the 4 rows of the word are all inside or all outside
-        if (!CHECK || (col < m && row < ld)) {
-          unsigned v = 0;
-#pragma unroll
-          for (int q = 0; q < 4; q++) v |= (unsigned)(res[q] & 0xff) << (8 * q);
-          *(gu32 *)dst = v;
+          res[q] = residue_of_f32(acc[r][c][q], invf, mi);
+        // K % 16 == 0: the 4 rows of the word are all inside or all outside
+        if (!CHECK || (col < m && row < K)) {
+          *(gu32 *)dst = pack4_lo(res[0], res[1], res[2], res[3]);
         }
       }
   }
@@ -1008,7 +999,7 @@ oz_bgemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
       __builtin_amdgcn_sched_group_barrier(0x008, 28, 0);
-      if ((kt + 1) % fold_every == 0) {
+      if ((kt + 1) % fold_every == 0 && kt + 1 < nk) {
 #pragma unroll
         for (int r = 0; r < 8; r++)
 #pragma unroll
@@ -1030,7 +1021,6 @@ oz_bgemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
       gload(tn, 0, ga, gb);
     }
     // C through LDS (A1: columns 0..127, B1: 128..255, as in the INT8 kernel)
-    const int c22 = t.c22;
     unsigned *Ch = reinterpret_cast<unsigned *>(wn < 2 ? A1 : B1);
 #pragma unroll
     for (int r = 0; r < 8; r++)
@@ -1039,7 +1029,7 @@ oz_bgemm_big_kernel(const RGemm *__restrict__ tab, int m, int nmod,
         int res[4];
 #pragma unroll
         for (int q = 0; q < 4; q++)
-          res[q] = mod_k((int)fold_f32(acc[r][c][q], t.mf, t.invf), c22, t.mi);  // |.| <= 1.5 m
+          res[q] = residue_of_f32(acc[r][c][q], t.invf, t.mi);
         const int col = (wn & 1) * 64 + c * 16 + l16;
         const int w = wm * 32 + r * 4 + lk;
         Ch[col * 64 + (w ^ (4 * l16))] = pack4_lo(res[0], res[1], res[2], res[3]);
@@ -1168,24 +1158,24 @@ bool residue_gemm_segmented(int m, int levels, int tile, bool bf16, long long pr
 // as much as, at the tile's rate (POP/s over the device; the smaller tiles
 // load more operand bytes per product).  Both are fitted to launches of 686
 // products of orders 128 to 1000, in us with 256 / 192 / 160 / 128 / 96 / 64
-// tiles: order 128 26 25 18 14 24 19; 160 33 29 21 34 27 26; 320 120 88 67 77
-// 91 85; 384 127 107 123 97 120 135; 512 172 226 265 196 287 311; 640 421 475
-// 377 384 521 639; 750 572 676 708 769 936 1366; 1000 1177 1485 1608 1591 2359
-// 3097.  The 128 x 128 kernel these tiles replaced (registers between memory
+// tiles: order 128 25 20 16 14 19 18; 160 31 25 19 27 21 26; 320 114 72 61 66
+// 82 83; 384 121 94 108 89 111 136; 512 162 189 236 181 266 308; 640 397 414
+// 337 359 475 613; 750 484 502 557 575 707 1012; 1000 976 1202 1203 1135 1776
+// 2217.  The 128 x 128 kernel these tiles replaced (registers between memory
 // and LDS, two blocks per CU) took 122 at 320 and 395 at 640.
 double residue_tile_cost(int bt, double tiles, int K) {
   struct {
     int bt;
     double rate, epi;
-  } const t[] = {{256, 1.7, 230}, {192, 1.6, 390}, {160, 1.35, 250},
-                 {128, 1.1, 100}, {96, 1.0, 190},  {64, 0.57, 60}};
+  } const t[] = {{256, 2.1, 340},  {192, 1.87, 410}, {160, 1.55, 270},
+                 {128, 1.25, 110}, {96, 1.06, 160},  {64, 0.6, 60}};
   for (const auto &e : t)
     if (e.bt == bt) return ceil(tiles / device_cu_count()) * bt * bt * (K + e.epi) / e.rate;
   return INFINITY;
 }
 
 int residue_block_tile(int m, int levels, int tile, long long problems) {
-  const int m0 = m >> levels, K = levels > 0 ? m : residue_pitch(m);
+  const int m0 = m >> levels, K = levels > 0 ? m : residue_k(m);
   // the one-pass reduction of partial 256 tiles needs K <= 16384
   const bool big = tile == 0 && (m0 % JBM == 0 ? big_int8_gemm(m, levels, tile)
                                                : levels == 0 && K <= 16384);
@@ -1296,7 +1286,7 @@ hipError_t launch_ozaki_step(int step, const OzLeaf *tab, int count, int m, int 
         hipLaunchKernelGGL((oz_split_a_kernel<false>), ga, dim3(T256), 0, s, tab, m, nmod, kc);
       else
         hipLaunchKernelGGL((oz_split_a_kernel<true>), ga, dim3(T256), 0, s, tab, m, nmod, kc);
-      const long long u16 = residue_area(m) / 16;
+      const long long u16 = (long long)m * residue_k(m) / 16;
       long long blocks = (u16 + T256 - 1) / T256;
       long long cap = (long long)device_cu_count() * 8 / count;
       if (cap < 1) cap = 1;

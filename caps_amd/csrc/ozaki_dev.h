@@ -104,22 +104,33 @@ __device__ __forceinline__ int mod_small(int x, float mf, float inv) {
   return (int)fmaf(-rintf(xf * inv), mf, xf);
 }
 
-// byte q of a packed INT8 residue word from an INT32 product sum that started
-// at 128: xb = x + 128, |x| <= 2^28 (K <= 2^14 products of INT8 residues).
-//   y = xb + (xb >> 14) (c14 - 2^14) = (xb >> 14) c14 + (xb & 16383) = xb
-//   (mod m), |y| < 2^21.1, in one mad24 (c14m = c14 - 2^14);
-//   k = floor(y / m + 1/2 - 128 / m) from fma(y, 1/m, cl) in FP32, cl = 1/2 -
-//   128/m: the error (< 1.2e-3) is below the distance 1/(2m) of that argument
-//   to an integer for odd m, and every step is exact for m = 256;
-//   y - k m = r + 128, r = x mod m in [-m/2, m/2): a byte value in [0, 255]
-//   that cvt_pk_u8 converts and places at byte q of `word`.  XOR 0x80 per
-//   byte then gives the INT8 residue r.
-__device__ __forceinline__ unsigned res_byte128(int xb, int c14m, float mf, float inv, float cl,
-                                                int q, unsigned word) {
-  const int y = __mul24(xb >> 14, c14m) + xb;
-  const float yf = (float)y;
-  const float k = floorf(fmaf(yf, inv, cl));
-  return __builtin_amdgcn_cvt_pk_u8_f32(fmaf(-k, mf, yf), q, word);
+// added to a float |k| < 2^22, rounds it to the nearest integer, which is then
+// in the low 22 bits of the sum (0x4B400000 + k)
+constexpr float ROUND_MAGIC = 12582912.0f;  // 1.5 * 2^23
+
+// low byte: the symmetric residue modulo m of an INT32 product sum that started
+// at `bias` (a multiple of m, >= 2^28): xb = x + bias >= 0 for |x| <= 2^28 (K
+// <= 2^14 products of INT8 residues).
+//   y = lo16(xb) + hi16(xb) (2^16 mod m) = x (mod m), 0 <= y < 2^22, one
+//   dot product of 16-bit halves;
+//   k = round(y / m): y is exact in FP32 and the quotient's error below 1/(2m),
+//   its least distance to a half-integer for odd m (exact for m = 256), so one
+//   fma with ROUND_MAGIC leaves k in the low bits;
+//   y - k m in one mad24 of those bits (their 2^22 times m changes no low byte).
+// Four full-rate operations; checked for every y and modulus.
+__device__ __forceinline__ int residue_of_sum(int xb, unsigned dot16, float inv, int mi) {
+  typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+  const unsigned y = __builtin_amdgcn_udot2(__builtin_bit_cast(v2us, xb),
+                                            __builtin_bit_cast(v2us, dot16), 0u, false);
+  const float t = fmaf((float)y, inv, ROUND_MAGIC);
+  return __mul24((int)__float_as_uint(t), -mi) + (int)y;
+}
+
+// low byte: the symmetric residue modulo m of an FP32 integer |x| <= 2^23 +
+// 1.5 m (a folded sum and at most 512 products more), as above
+__device__ __forceinline__ int residue_of_f32(float x, float inv, int mi) {
+  const float t = fmaf(x, inv, ROUND_MAGIC);
+  return __mul24((int)__float_as_uint(t), -mi) + (int)x;
 }
 
 // symmetric residue of an INT32 product sum (|x| < 2^31) modulo mi

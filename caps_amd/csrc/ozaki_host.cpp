@@ -124,11 +124,8 @@ bool ozaki_make_consts(int nmod, OzakiConsts &k) {
   Big M(1);
   for (int l = 0; l < nmod; l++) {
     k.m[l] = mods[l];
-    {
-      int c = (1 << 14) % mods[l];
-      if (c > (mods[l] - 1) / 2) c -= mods[l];
-      k.c14[l] = c;
-    }
+    k.dot16[l] = 1u | ((unsigned)((1 << 16) % mods[l]) << 16);
+    k.bias[l] = ((1 << 28) + mods[l] - 1) / mods[l] * mods[l];
     k.c22[l] = ((1 << 23) / mods[l] + 1) >> 1;  // round(2^22 / m)
     k.inv_m[l] = 1.0 / (double)mods[l];
     M.mul((uint32_t)mods[l]);
