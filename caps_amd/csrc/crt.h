@@ -60,8 +60,7 @@ hipError_t launch_residue_ew(int op, const RPtrs *d_tab, int count, long long n,
 // ---- segmented launches over the items of an uneven batch (kernels.h VSeg)
 // the kernels of the scale, split and reconstruct steps
 enum CrtKernel : int {
-  CRT_ROWPART = 0,
-  CRT_COLPART = 1,
+  CRT_PARTIALS = 0,
   CRT_FINALIZE = 2,
   CRT_SPLIT_A = 3,
   CRT_SPLIT_B = 4,
@@ -78,9 +77,10 @@ hipError_t launch_residue_ew_multi(int op, const char *d_tables, const VSeg *d_s
                                    int blocks, bool vec4, const OzakiConsts *d_consts,
                                    hipStream_t s);
 
-// chunks of a leaf row used by the row-partials reduction
-inline int crt_row_chunks(int m) {
-  int c = m / 256;
+// chunks of a leaf row used by the row-partials reduction (each split once
+// more over the waves of a block); `pad` false: as counted without the pitch
+inline int crt_row_chunks(int m, bool pad = true) {
+  int c = pad ? (m + 127) / 128 : m / 256;
   return c < 1 ? 1 : (c > 8 ? 8 : c);
 }
 

@@ -12,42 +12,51 @@ namespace {
 constexpr int T = 256;
 
 // ------------------------------------------------------------------ scale
-// partial (e, s) of row i of A over columns [lj0, lj1) of leaf column block bj.
+// partials (e, s) of 64 rows of A over chunk by of a leaf column block: lane =
+// row, each of the 4 waves takes a quarter of the chunk's columns, wave 0
+// merges them (in wave order).  Bound by the read of A where the blocks fill
+// the device (n = 8192: 5.8 TB/s with the columns of B); a thread per row made
+// 20 blocks at n = 1280, each a chain of 40 loads: 37 -> 8.8 us (n = 3000:
+// 75 -> 36) for the rows of A and the columns of B together.
 // PLAIN: column-major leaves (bs == 1 or bs == m), 8 columns per step.
+typedef double2 RowLds[T / 64][64];
+
 template <bool PLAIN>
-__device__ __forceinline__ void rowpart_body(const CrtMats *__restrict__ M, int bx, int by) {
+__device__ __forceinline__ void rowpart_body(const CrtMats *__restrict__ M, int bx, int by,
+                                             RowLds &P) {
   const int n = M->n, m = M->m, nrec = M->nrec, bs = M->bs, ch = M->chunks;
-  const int i = bx * T + threadIdx.x;
-  if (i >= n) return;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int row = bx * 64 + lane, i = min(row, n - 1);
   const int c = by;  // bj * chunks + k
-  const int bj = c / ch, k = c - bj * ch;
-  const int per = (m + ch - 1) / ch;
-  const int lj0 = k * per, lj1 = min(m, lj0 + per);
+  const int bj = c / ch, k = (c - bj * ch) * (T / 64) + wv;
+  const int per = (m + ch * (T / 64) - 1) / (ch * (T / 64));
+  const int lj0 = min(m, k * per), lj1 = min(m, lj0 + per);
   int e = NOSCALE;
   double s = 0.0;
   if (PLAIN) {
-    const double *row = M->A + caps_elem_offset(n, nrec, bs, i, bj * m);  // (i, bj m)
+    const double *base = M->A + caps_elem_offset(n, nrec, bs, i, bj * m);  // (i, bj m)
     int lj = lj0;
     for (; lj + 8 <= lj1; lj += 8) {
       double v[8];
 #pragma unroll
-      for (int t = 0; t < 8; t++) v[t] = row[(long long)(lj + t) * m];
+      for (int t = 0; t < 8; t++) v[t] = base[(long long)(lj + t) * m];
       int e8;
       double s8;
       sq_block8(v, e8, s8);
       sq_merge(e, s, e8, s8);
     }
-    for (; lj < lj1; lj++) sq_acc(row[(long long)lj * m], e, s);
+    for (; lj < lj1; lj++) sq_acc(base[(long long)lj * m], e, s);
   } else {
     for (int lj = lj0; lj < lj1; lj++)
       sq_acc(M->A[caps_elem_offset(n, nrec, bs, i, bj * m + lj)], e, s);
   }
-  reinterpret_cast<double2 *>(M->pa)[(long long)c * n + i] = make_double2(s, (double)e);
-}
-
-template <bool PLAIN>
-__global__ __launch_bounds__(T) void crt_rowpart_kernel(const CrtMats *__restrict__ M) {
-  rowpart_body<PLAIN>(M, blockIdx.x, blockIdx.y);
+  P[wv][lane] = make_double2(s, (double)e);
+  __syncthreads();
+  if (wv == 0 && row < n) {
+#pragma unroll
+    for (int w = 1; w < T / 64; w++) sq_merge(e, s, (int)P[w][lane].y, P[w][lane].x);
+    reinterpret_cast<double2 *>(M->pa)[(long long)c * n + i] = make_double2(s, (double)e);
+  }
 }
 
 // partial of column j of B over leaf row block bi: one wave, fixed butterfly.
@@ -88,9 +97,40 @@ __device__ __forceinline__ void colpart_body(const CrtMats *__restrict__ M, int 
   if (lane == 0) reinterpret_cast<double2 *>(M->pb)[(long long)bi * n + j] = make_double2(s, (double)e);
 }
 
+// row partials of A (the first blocks: x over the rows, then the chunks) and
+// column partials of B in one launch: together they fill the device sooner
 template <bool PLAIN>
-__global__ __launch_bounds__(T) void crt_colpart_kernel(const CrtMats *__restrict__ M) {
-  colpart_body<PLAIN>(M, blockIdx.x);
+__device__ __forceinline__ void partials_body(const CrtMats *__restrict__ M, int bx, RowLds &P) {
+  const int gx = (M->n + 63) / 64, rows = gx * (M->chunks << M->nrec);
+  if (bx < rows)
+    rowpart_body<PLAIN>(M, bx % gx, bx / gx, P);
+  else
+    colpart_body<PLAIN>(M, bx - rows);
+}
+
+template <bool PLAIN>
+__global__ __launch_bounds__(T) void crt_partials_kernel(const CrtMats *__restrict__ M) {
+  __shared__ RowLds P;
+  partials_body<PLAIN>(M, blockIdx.x, P);
+}
+
+// merges `count` partials, one every n; 4 loads in flight
+__device__ __forceinline__ int merged_exponent(const double2 *p, int count, int n, double L) {
+  int e = NOSCALE;
+  double s = 0.0;
+  int c = 0;
+  for (; c + 4 <= count; c += 4) {
+    double2 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = p[(long long)(c + k) * n];
+#pragma unroll
+    for (int k = 0; k < 4; k++) sq_merge(e, s, (int)v[k].y, v[k].x);
+  }
+  for (; c < count; c++) {
+    const double2 v = p[(long long)c * n];
+    sq_merge(e, s, (int)v.y, v.x);
+  }
+  return scale_exponent(e, s, L);
 }
 
 __device__ __forceinline__ void finalize_body(const CrtMats *__restrict__ M,
@@ -99,22 +139,9 @@ __device__ __forceinline__ void finalize_body(const CrtMats *__restrict__ M,
   const int i = bx * T + threadIdx.x;
   if (i >= n) return;
   const int nblk = 1 << M->nrec;
-  const double2 *pa = reinterpret_cast<const double2 *>(M->pa);
-  const double2 *pb = reinterpret_cast<const double2 *>(M->pb);
-  int e = NOSCALE;
-  double s = 0.0;
-  for (int c = 0; c < nblk * M->chunks; c++) {
-    double2 v = pa[(long long)c * n + i];
-    sq_merge(e, s, (int)v.y, v.x);
-  }
-  M->sa[i] = scale_exponent(e, s, kc->L);
-  e = NOSCALE;
-  s = 0.0;
-  for (int b = 0; b < nblk; b++) {
-    double2 v = pb[(long long)b * n + i];
-    sq_merge(e, s, (int)v.y, v.x);
-  }
-  M->sb[i] = scale_exponent(e, s, kc->L);
+  M->sa[i] = merged_exponent(reinterpret_cast<const double2 *>(M->pa) + i, nblk * M->chunks, n,
+                             kc->L);
+  M->sb[i] = merged_exponent(reinterpret_cast<const double2 *>(M->pb) + i, nblk, n, kc->L);
 }
 
 __global__ __launch_bounds__(T) void crt_finalize_kernel(const CrtMats *__restrict__ M,
@@ -301,12 +328,12 @@ __global__ __launch_bounds__(T) void crt_multi_kernel(const char *__restrict__ b
                                                       const VSeg *__restrict__ segs, int nseg,
                                                       const OzakiConsts *__restrict__ kc) {
   __shared__ double Ts[K == CRT_SPLIT_A ? SPLIT_K : 1][K == CRT_SPLIT_A ? SPLIT_R : 1];
+  __shared__ double2 P[K == CRT_PARTIALS ? T / 64 : 1][K == CRT_PARTIALS ? 64 : 1];
   const VSeg &S = segs[vseg_find(segs, nseg, blockIdx.x)];
   const int l = blockIdx.x - S.blk0;
   const int bx = l % S.gx, by = l / S.gx;
   const CrtMats *M = reinterpret_cast<const CrtMats *>(base + S.arg);
-  if constexpr (K == CRT_ROWPART) rowpart_body<F>(M, bx, by);
-  if constexpr (K == CRT_COLPART) colpart_body<F>(M, bx);
+  if constexpr (K == CRT_PARTIALS) partials_body<F>(M, l, P);
   if constexpr (K == CRT_FINALIZE) finalize_body(M, kc, bx);
   if constexpr (K == CRT_SPLIT_A) split_a_body<F>(M, kc, bx, by, Ts);
   if constexpr (K == CRT_SPLIT_B) split_b_body<F>(M, kc, bx, by, S.gx);
@@ -465,12 +492,8 @@ bool crt_grid(int k, const CrtMats &h, int &gx, int &gy) {
   const bool plain = (h.bs == 1 || h.bs == h.m);
   gy = 1;
   switch (k) {
-    case CRT_ROWPART:
-      gx = (h.n + T - 1) / T;
-      gy = nblk * h.chunks;
-      return plain;
-    case CRT_COLPART:
-      gx = (int)(((long long)h.n * nblk + 3) / 4);
+    case CRT_PARTIALS:
+      gx = (h.n + 63) / 64 * nblk * h.chunks + (int)(((long long)h.n * nblk + 3) / 4);
       return plain;
     case CRT_FINALIZE:
       gx = (h.n + T - 1) / T;
@@ -496,8 +519,7 @@ hipError_t launch_crt_multi(int k, bool flag, int np, const char *base, const VS
                             int nseg, int blocks, const OzakiConsts *kc, hipStream_t s) {
   if (nseg <= 0 || blocks <= 0) return hipSuccess;
   switch (k) {
-    case CRT_ROWPART: return launch_crt_multi_f<CRT_ROWPART>(flag, np, base, segs, nseg, blocks, kc, s);
-    case CRT_COLPART: return launch_crt_multi_f<CRT_COLPART>(flag, np, base, segs, nseg, blocks, kc, s);
+    case CRT_PARTIALS: return launch_crt_multi_f<CRT_PARTIALS>(flag, np, base, segs, nseg, blocks, kc, s);
     case CRT_FINALIZE: return launch_crt_multi_f<CRT_FINALIZE>(false, np, base, segs, nseg, blocks, kc, s);
     case CRT_SPLIT_A: return launch_crt_multi_f<CRT_SPLIT_A>(flag, np, base, segs, nseg, blocks, kc, s);
     case CRT_SPLIT_B: return launch_crt_multi_f<CRT_SPLIT_B>(flag, np, base, segs, nseg, blocks, kc, s);
@@ -530,16 +552,11 @@ hipError_t launch_crt_step(int step, const CrtMats *M, const CrtMats &h, const O
   bool f;
   switch (step) {
     case 0: {
-      f = crt_grid(CRT_ROWPART, h, gx, gy);
+      f = crt_grid(CRT_PARTIALS, h, gx, gy);
       if (f)
-        hipLaunchKernelGGL((crt_rowpart_kernel<true>), dim3(gx, gy), dim3(T), 0, s, M);
+        hipLaunchKernelGGL((crt_partials_kernel<true>), dim3(gx), dim3(T), 0, s, M);
       else
-        hipLaunchKernelGGL((crt_rowpart_kernel<false>), dim3(gx, gy), dim3(T), 0, s, M);
-      f = crt_grid(CRT_COLPART, h, gx, gy);
-      if (f)
-        hipLaunchKernelGGL((crt_colpart_kernel<true>), dim3(gx), dim3(T), 0, s, M);
-      else
-        hipLaunchKernelGGL((crt_colpart_kernel<false>), dim3(gx), dim3(T), 0, s, M);
+        hipLaunchKernelGGL((crt_partials_kernel<false>), dim3(gx), dim3(T), 0, s, M);
       crt_grid(CRT_FINALIZE, h, gx, gy);
       hipLaunchKernelGGL(crt_finalize_kernel, dim3(gx), dim3(T), 0, s, M, kc);
       return hipGetLastError();

@@ -538,7 +538,7 @@ struct Builder {
       M.m = m;
       M.plane = n2;
       M.nmod = moduli;
-      M.chunks = crt_row_chunks(m);
+      M.chunks = crt_row_chunks(m, pad);
       const int nblk = 1 << d.nrec;
       M.sa = reinterpret_cast<int *>(base + alloc(sizeof(int) * n));
       M.sb = reinterpret_cast<int *>(base + alloc(sizeof(int) * n));
@@ -613,7 +613,7 @@ hipError_t run_one(const Plan &plan, const Step &st, hipStream_t s) {
                            plan.oz_moduli, kc, s, st.vec2 != 0);
     case STEP_BB_SPLIT_B:
       return launch_bb_split_b(reinterpret_cast<const BBSplitB *>(tb + st.table), st.n, st.bs,
-                               kc, s);
+                               plan.oz_moduli, kc, s);
     case STEP_BB_SPLIT_A:
       return launch_bb_split_a(reinterpret_cast<const BBSplitA *>(tb + st.table), st.n, st.bs,
                                kc, s);
@@ -742,7 +742,7 @@ MergeKey merge_key(const Plan &plan, const Step &st) {
       break;
     }
     case STEP_CRT_SCALE:
-      k = {STEP_MULTI_CRT, MERGE_CRT_SCALE, crt_grid(CRT_ROWPART, plan.crt_host[st.aux], gx, gy)};
+      k = {STEP_MULTI_CRT, MERGE_CRT_SCALE, crt_grid(CRT_PARTIALS, plan.crt_host[st.aux], gx, gy)};
       break;
     case STEP_CRT_SPLIT: {
       const CrtMats &h = plan.crt_host[st.aux];
@@ -799,8 +799,7 @@ void emit_merged(Plan &plan, const MergeKey &k, const std::vector<const Step *> 
                  int moduli) {
   if (k.kind == STEP_MULTI_CRT) {
     if (k.a == MERGE_CRT_SCALE) {
-      emit_crt(plan, heads, CRT_ROWPART, k.b);
-      emit_crt(plan, heads, CRT_COLPART, k.b);
+      emit_crt(plan, heads, CRT_PARTIALS, k.b);
       emit_crt(plan, heads, CRT_FINALIZE, false);
     } else if (k.a == MERGE_CRT_SPLIT) {
       emit_crt(plan, heads, CRT_SPLIT_A, k.b & 1);

@@ -78,7 +78,7 @@ struct BBSplitA {
 hipError_t launch_bb_pre(const BBPre *d_P, long long q, bool residue, int nmod,
                          const OzakiConsts *d_consts, hipStream_t s, bool a_only = false);
 // m0: host copy of the table's leaf size; q < 2^31
-hipError_t launch_bb_split_b(const BBSplitB *d_P, long long q, int m0,
+hipError_t launch_bb_split_b(const BBSplitB *d_P, long long q, int m0, int nmod,
                              const OzakiConsts *d_consts, hipStream_t s);
 // m0 % 128 == 0 (host copy of the table's m0), q < 2^31
 hipError_t launch_bb_split_a(const BBSplitA *d_P, long long q, int m0,
