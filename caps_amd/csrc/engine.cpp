@@ -28,6 +28,7 @@
 
 #include "crt.h"
 #include "fused2.h"
+#include "fused3.h"
 #include "ozaki.h"
 
 namespace caps {
@@ -384,6 +385,48 @@ struct Builder {
     return residue ? (q % 4 == 0) : (q % 2 == 0);
   }
 
+  // Can three FP64 'b' levels starting at `depth` run as fused passes?  (pad =
+  // false: as two and one, the size the fixed scratch's limit counts)
+  bool fusable3(size_t batch, int s, int nrec, int depth) const {
+    if (residue || !pad || !fuse || batch != 1 || nrec - cutoff < 3) return false;
+    for (int l = depth; l < depth + 3; l++)
+      if (pattern[l] != 'b' && pattern[l] != 'B') return false;
+    return b3_fits(area(s / 8));
+  }
+
+  // Three fused 'b' levels of one FP64 sub-problem (fused3.h)
+  void bfs3(const Prob &pb, int s, int nrec, int depth) {
+    const int sub = s / 8;
+    const long long q = area(sub), step = b3_step(q);
+    const size_t mark = top;
+    for (int l = 0; l < 3; l++) level_tag(depth + l);
+    plan.additions += (16 + 7 * 4 + 49) * 15LL * q;
+    // plain operands are quadrants, passed by pointer
+    const int quad[2][7] = {{0, 2, -1, -1, -1, -1, 3}, {0, 1, -1, -1, -1, 3, -1}};
+    const Mat in[2] = {pb.A, pb.B};
+    const Mat L[2] = {alloc_mats(B3_WRITTEN, step), alloc_mats(B3_WRITTEN, step)};
+    const Mat Q = alloc_mats(343, step);
+    std::vector<Prob> next(343);
+    int written[2] = {0, 0};
+    for (int t = 0; t < 343; t++) {
+      const int i = t / 49, j = t / 7 % 7, k = t % 7;
+      Mat op[2];
+      for (int side = 0; side < 2; side++)
+        op[side] = bb_plain(side, i) && bb_plain(side, j) && bb_plain(side, k)
+                       ? at(in[side], (16 * quad[side][i] + 4 * quad[side][j] + quad[side][k]) * q)
+                       : at(L[side], written[side]++ * step);
+      next[t] = {op[0], op[1], at(Q, t * step)};
+    }
+    if (written[0] != B3_WRITTEN || written[1] != B3_WRITTEN) broken = true;
+    const auto d = [](const Mat &m) { return reinterpret_cast<double *>(m.p); };
+    const B3Pre pre{{d(pb.A), d(pb.B)}, {d(L[0]), d(L[1])}, step};
+    push(STEP_B3_PRE, 0, 1, q, 0, add_table(&pre, sizeof(pre)));
+    rec(next, sub, nrec - 3, depth + 3);
+    const B3Post post{d(Q), step, d(pb.C)};
+    push(STEP_B3_POST, 0, 1, q, 0, add_table(&post, sizeof(post)));
+    top = mark;
+  }
+
   // Two fused 'b' levels for one sub-problem (fused2.h).  In residue mode at
   // the top, `crt` carries the reconstruction target and the combinations are
   // fused with it.
@@ -496,6 +539,10 @@ struct Builder {
   void rec(const std::vector<Prob> &batch, int s, int nrec, int depth) {
     if (nrec == cutoff) {
       leaf(batch, s);
+      return;
+    }
+    if (fusable3(batch.size(), s, nrec, depth)) {
+      bfs3(batch[0], s, nrec, depth);
       return;
     }
     if (!residue && fusable(batch.size(), s, nrec, depth) && aligned16(batch[0])) {
@@ -621,6 +668,10 @@ hipError_t run_one(const Plan &plan, const Step &st, hipStream_t s) {
     case STEP_BB_POST:
       return launch_bb_post(reinterpret_cast<const BBPost *>(tb + st.table), st.n, st.op != 0,
                             st.op ? ozaki_npieces(plan.oz_moduli) : 0, kc, s);
+    case STEP_B3_PRE:
+      return launch_b3_pre(reinterpret_cast<const B3Pre *>(tb + st.table), st.n, s);
+    case STEP_B3_POST:
+      return launch_b3_post(reinterpret_cast<const B3Post *>(tb + st.table), st.n, s);
     case STEP_CRT_SCALE:
     case STEP_CRT_SPLIT:
     case STEP_CRT_RECON:
@@ -652,6 +703,8 @@ int timer_of(const Step &st) {
   switch (st.kind) {
     case STEP_EW:
     case STEP_REW:
+    case STEP_B3_PRE:
+    case STEP_B3_POST:
     case STEP_BB_PRE: return CAPS_TIMER_ADD;
     case STEP_BB_POST: return CAPS_TIMER_RECON;
     case STEP_GEMM_F64:

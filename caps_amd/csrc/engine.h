@@ -56,6 +56,8 @@ enum StepKind : int {
   STEP_MULTI_RGEMM = 17, // INT8 residue leaf GEMMs, bs = block tile
   STEP_MULTI_CRT = 18,   // residue scale / split / reconstruct kernel op (CrtKernel), vec2 = flag
   STEP_BB_SPLIT_A = 19,  // residue mode: A's split fused with its two top 'b' levels, bs = m0
+  STEP_B3_PRE = 20,    // FP64: three 'b' levels of pre-additions in one pass
+  STEP_B3_POST = 21,   // FP64: three 'b' levels of combinations
 };
 
 struct Step {
