@@ -19,6 +19,7 @@
 
 #include "../../include/caps_amd.h"
 #include "engine.h"
+#include "hostcopy.h"
 #include "ozaki.h"
 #include "planner.h"
 #include "tune.h"
@@ -82,6 +83,7 @@ struct State {
   double *stage[3] = {nullptr, nullptr, nullptr};
   size_t stage_elems = 0;
   hipStream_t stage_stream = nullptr;
+  HostCopy host_copy;
   // caps_multiply_device_noalloc: the address of each device's scratch array,
   // and host-only plans (their tables are copied into the scratch per call)
   std::map<int, char *> scratch;
@@ -573,15 +575,15 @@ int caps_multiply(const double *A, const double *B, double *C, const caps_desc *
   rc = stage_locked(s, n2);
   if (rc) return rc;
   hipStream_t ss = s.stage_stream;
-  HIP_TRY(hipMemcpyAsync(s.stage[0], A, n2 * sizeof(double), hipMemcpyHostToDevice, ss));
-  HIP_TRY(hipMemcpyAsync(s.stage[1], B, n2 * sizeof(double), hipMemcpyHostToDevice, ss));
+  const HostRange in[2] = {{s.stage[0], const_cast<double *>(A), n2 * sizeof(double)},
+                           {s.stage[1], const_cast<double *>(B), n2 * sizeof(double)}};
+  HIP_TRY(s.host_copy.up(in, 2, ss));
   rc = multiply_device_locked(s, s.stage[0], s.stage[1], s.stage[2], desc, pattern, opts, ss);
   if (rc) {
     hipStreamSynchronize(ss);
     return rc;
   }
-  HIP_TRY(hipMemcpyAsync(C, s.stage[2], n2 * sizeof(double), hipMemcpyDeviceToHost, ss));
-  HIP_TRY(hipStreamSynchronize(ss));
+  HIP_TRY(s.host_copy.down({s.stage[2], C, n2 * sizeof(double)}, ss));
   return CAPS_OK;
 }
 
@@ -624,14 +626,14 @@ static int layout_host(const double *src, double *dst, const caps_desc *desc, bo
   rc = stage_locked(s, n2);
   if (rc) return rc;
   hipStream_t ss = s.stage_stream;
-  HIP_TRY(hipMemcpyAsync(s.stage[0], src, n2 * sizeof(double), hipMemcpyHostToDevice, ss));
+  const HostRange in{s.stage[0], const_cast<double *>(src), n2 * sizeof(double)};
+  HIP_TRY(s.host_copy.up(&in, 1, ss));
   hipError_t e = to_caps ? launch_to_caps(s.stage[0], s.stage[1], desc->lda, desc->nrec,
                                           desc->bs, ss)
                          : launch_from_caps(s.stage[0], s.stage[1], desc->lda, desc->nrec,
                                             desc->bs, ss);
   if (e != hipSuccess) return fail(CAPS_EHIP, "layout kernel: %s", hipGetErrorString(e));
-  HIP_TRY(hipMemcpyAsync(dst, s.stage[1], n2 * sizeof(double), hipMemcpyDeviceToHost, ss));
-  HIP_TRY(hipStreamSynchronize(ss));
+  HIP_TRY(s.host_copy.down({s.stage[1], dst, n2 * sizeof(double)}, ss));
   return CAPS_OK;
 }
 
@@ -937,6 +939,7 @@ int caps_release(void) {
       p = nullptr;
     }
   s.stage_elems = 0;
+  s.host_copy.release();
   return CAPS_OK;
 }
 
