@@ -31,6 +31,8 @@
 
 namespace caps {
 
+long long dgemm_full_tiles(int bt, long long total);
+
 namespace {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
@@ -263,21 +265,38 @@ __device__ __forceinline__ void dgemm_tile(const double *__restrict__ A,
     }
 }
 
-// One persistent launch over all tiles of all problems of one size.
+// One persistent launch over all tiles of all problems of one size: the first
+// `full` whole, the others as four tiles of half the size (dgemm_full_tiles),
+// starting with the blocks dispatched last.
 template <int BT, bool CHECK>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(Tile<BT>::OCC, Tile<BT>::OCC))) void
 dgemm_kernel(const GemmPtrs *__restrict__ tab, int m,
-                                                   TileMap map, int m0, int d) {
+                                                   TileMap map, int full, int m0, int d) {
   constexpr int STAGE = Tile<BT>::STAGE;
   __shared__ __attribute__((aligned(1024))) double S[4 * STAGE];
   const int G = gridDim.x;
-  for (int round = 0; round * G < map.total; round++) {
-    const int tile = round * G + xcd_tile(blockIdx.x, G);
-    if (tile >= map.total) break;
+  for (int round = 0; round * G < full; round++) {
+    const int tile = round_tile(round, blockIdx.x, G, full);
+    if (tile >= full) break;
     int prob, ti, tj;
     tile_coords(map, tile, prob, ti, tj);
     const GemmPtrs &P = tab[prob];
     dgemm_tile<BT, CHECK>(P.A, P.B, P.C, m, m0, d, ti, tj, S);
+  }
+  if constexpr (BT > 32) {
+    const int subs = 4 * (map.total - full);
+    const int last = (G / NXCD - 1 - (int)blockIdx.x / NXCD) * NXCD + (int)blockIdx.x % NXCD;
+    for (int round = 0; round * G < subs; round++) {
+      const int sub = round_tile(round, last, G, subs);
+      if (sub >= subs) break;
+      int prob, ti, tj;
+      tile_coords(map, full + (sub >> 2), prob, ti, tj);
+      ti = 2 * ti + (sub & 1);
+      tj = 2 * tj + ((sub >> 1) & 1);
+      if (CHECK && (ti * (BT / 2) >= m || tj * (BT / 2) >= m)) continue;
+      const GemmPtrs &P = tab[prob];
+      dgemm_tile<BT / 2, CHECK>(P.A, P.B, P.C, m, m0, d, ti, tj, S);
+    }
   }
 }
 
@@ -294,7 +313,7 @@ dgemm_multi_kernel(const char *__restrict__ base,
   __shared__ __attribute__((aligned(1024))) double S[4 * STAGE];
   const int G = gridDim.x;
   for (int round = 0; round * G < total; round++) {
-    const int tile = round * G + xcd_tile(blockIdx.x, G);
+    const int tile = round_tile(round, blockIdx.x, G, total);
     if (tile >= total) break;
     const VSeg &V = segs[vseg_find(segs, nseg, tile)];
     const int m = (int)V.n, d = V.aux & 255;
@@ -319,12 +338,15 @@ hipError_t launch_tile(const GemmPtrs *tab, int count, int m, int levels, hipStr
   if (!fast && levels > 0) return hipErrorInvalidValue;  // quadtree operands need whole tiles
   // persistent grid: as many blocks per CU as registers and LDS allow, a
   // multiple of the XCD count
-  const int G = persistent_grid(Tile<BT>::OCC, device_cu_count(), map.total);
+  const int full = (int)dgemm_full_tiles(BT, map.total);
+  const long long items = full + 4LL * (map.total - full);
+  const int G = persistent_grid(Tile<BT>::OCC, device_cu_count(),
+                                (int)(items < 0x7ffffff0LL ? items : 0x7ffffff0LL));
   if (fast)
-    hipLaunchKernelGGL((dgemm_kernel<BT, false>), dim3(G), dim3(NT), 0, s, tab, m, map, m0,
+    hipLaunchKernelGGL((dgemm_kernel<BT, false>), dim3(G), dim3(NT), 0, s, tab, m, map, full, m0,
                        levels);
   else
-    hipLaunchKernelGGL((dgemm_kernel<BT, true>), dim3(G), dim3(NT), 0, s, tab, m, map, m0,
+    hipLaunchKernelGGL((dgemm_kernel<BT, true>), dim3(G), dim3(NT), 0, s, tab, m, map, full, m0,
                        levels);
   return hipGetLastError();
 }
@@ -347,13 +369,28 @@ hipError_t launch_dgemm_batched(const GemmPtrs *tab, int count, int m, int level
 // ceil(tiles / CUs) tiles of bt^2 outputs.  The smaller tiles move more
 // operand bytes per product and run at 0.86 (64) and 0.6 (32) of the 128
 // tile's rate (49 products of 2048^3: 71.5, 60 and 41-49 TFLOP/s), but leave
-// less of the device idle.  Measured with 128 / 64 / 32 tiles (us): one product
+// less of the device idle.  Measured with 128 / 64 / 32 tiles, all whole (us): one product
 // of 512^3 72 / 25 / 15, of 1024^3 142 / 50 / 55; 49 of 256^3 46 / 44 / 53,
 // of 384^3 111 / 119 / 142, of 512^3 283 / 265 / 332, of 750^3 842 / 869 /
 // 1114; 343 of 49^3 26 / 13 / 13.
+static double tile_time(int bt) {
+  return bt * bt / (bt == 128 ? 1.0 : (bt == 64 ? 0.86 : 0.6));
+}
+
 double dgemm_tile_cost(int bt, double tiles) {
-  const double rate = bt == 128 ? 1.0 : (bt == 64 ? 0.86 : 0.6);
-  return ceil(tiles / device_cu_count()) * bt * bt / rate;
+  return ceil(tiles / device_cu_count()) * tile_time(bt);
+}
+
+// Tiles that run whole, of `total`: all, or as many as give each CU the same
+// number where the remaining ones take less time as tiles of half the size on
+// more CUs.  Measured with all tiles whole and with this rule (us, with the
+// last round spread over the XCDs): 49 products of 256^3 47 and 42, of 320^3
+// 97 and 67, of 512^3 261 and 239, of 750^3 858 and 786; 7 of 2048^3 2136 and
+// 1932.
+long long dgemm_full_tiles(int bt, long long total) {
+  const long long cus = device_cu_count(), left = total % cus;
+  if (bt == 32 || left == 0) return total;
+  return dgemm_tile_cost(bt / 2, 4.0 * left) < tile_time(bt) ? total - left : total;
 }
 
 int dgemm_block_tile(int m, int levels, int tile, long long count) {
@@ -366,7 +403,8 @@ int dgemm_block_tile(int m, int levels, int tile, long long count) {
   for (int bt = 128; bt >= 32; bt /= 2) {
     if (levels > 0 && m0 % bt != 0) continue;
     const double t = (m + bt - 1) / bt;
-    const double c = dgemm_tile_cost(bt, t * t * (double)count);
+    const double tiles = t * t * (double)count, full = (double)dgemm_full_tiles(bt, (long long)tiles);
+    const double c = dgemm_tile_cost(bt, full) + dgemm_tile_cost(bt / 2, 4 * (tiles - full));
     if (c < cost) {
       best = bt;
       cost = c;

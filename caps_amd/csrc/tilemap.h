@@ -47,6 +47,17 @@ __host__ __device__ __forceinline__ int xcd_tile(int b, int G) {
   return (b % NXCD) * (G / NXCD) + b / NXCD;
 }
 
+// Tile of block b in a round of a persistent grid; `total` or more: none.  The
+// last round's tiles go to all XCDs in equal ranges, and in each to the blocks
+// dispatched first, which lie on different CUs (with xcd_tile alone a last
+// round of G / 8 tiles would all run on XCD 0).
+__host__ __device__ __forceinline__ int round_tile(int round, int b, int G, int total) {
+  const int base = round * G, rem = total - base;
+  if (rem >= G) return base + xcd_tile(b, G);
+  const int per = (rem + NXCD - 1) / NXCD, j = b / NXCD, t = (b % NXCD) * per + j;
+  return j < per && t < rem ? base + t : total;
+}
+
 // Index, in CAPS quadrant order (11, 21, 12, 22 at each level), of leaf
 // (bi, bj) of a 2^d x 2^d quadtree of leaves.
 __device__ __forceinline__ long long quad_leaf(int bi, int bj, int d) {
