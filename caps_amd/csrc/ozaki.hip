@@ -364,7 +364,7 @@ oz_igemm_mid_kernel(const RGemm *__restrict__ tab, int m, int nmod,
   __shared__ __attribute__((aligned(1024))) int8_t S[4 * Mid<BT>::STAGE];
   const int G = gridDim.x;
   for (int round = 0; round * G < map.total; round++) {
-    const int tile = round * G + xcd_tile(blockIdx.x, G);
+    const int tile = round_tile(round, blockIdx.x, G, map.total);
     if (tile >= map.total) break;
     int prob, ti, tj;
     tile_coords(map, tile, prob, ti, tj);
@@ -382,7 +382,7 @@ oz_igemm_multi_kernel(const char *__restrict__ base, const VSeg *__restrict__ se
   __shared__ __attribute__((aligned(1024))) int8_t S[4 * Mid<BT>::STAGE];
   const int G = gridDim.x;
   for (int round = 0; round * G < total; round++) {
-    const int tile = round * G + xcd_tile(blockIdx.x, G);
+    const int tile = round_tile(round, blockIdx.x, G, total);
     if (tile >= total) break;
     const VSeg &V = segs[vseg_find(segs, nseg, tile)];
     const int local = tile - V.blk0, per = V.gx * V.gx;
@@ -779,7 +779,7 @@ __global__ __launch_bounds__(T256) void oz_bgemm_kernel(const RGemm *__restrict_
   const int fold_every = BFOLD / IBK;
 
   for (int round = 0; round * G < map.total; round++) {
-    const int tile = round * G + xcd_tile(blockIdx.x, G);
+    const int tile = round_tile(round, blockIdx.x, G, map.total);
     if (tile >= map.total) break;
     int prob, ti, tj;
     tile_coords(map, tile, prob, ti, tj);

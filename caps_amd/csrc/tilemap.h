@@ -50,7 +50,10 @@ __host__ __device__ __forceinline__ int xcd_tile(int b, int G) {
 // Tile of block b in a round of a persistent grid; `total` or more: none.  The
 // last round's tiles go to all XCDs in equal ranges, and in each to the blocks
 // dispatched first, which lie on different CUs (with xcd_tile alone a last
-// round of G / 8 tiles would all run on XCD 0).
+// round of G / 8 tiles would all run on XCD 0): for kernels with several blocks
+// per CU (686 INT8 products of 320^3 65 -> 58 us).  With one block per CU a round
+// takes as long either way and its tiles share more operands on one XCD (n = 3000
+// on 256 tiles 477 us, 490 spread).
 __host__ __device__ __forceinline__ int round_tile(int round, int b, int G, int total) {
   const int base = round * G, rem = total - base;
   if (rem >= G) return base + xcd_tile(b, G);
