@@ -28,7 +28,7 @@
 
 #include "crt.h"
 #include "fused2.h"
-#include "fused3.h"
+#include "fused_f64.h"
 #include "ozaki.h"
 
 namespace caps {
@@ -48,13 +48,13 @@ struct Builder {
   Plan &plan;
   char *base;  // workspace base (nullptr while sizing)
   size_t top = 0, peak = 0;
-  int bs = 1;
+  int leaf_bs = 1;  // block size of the leaves the steps see (1: column-major)
   int mode = CAPS_MODE_FP64;
   int moduli = 0;
   int cutoff = 0;  // layout levels below the Strassen recursion
   std::string pattern;
   std::string tags;      // the requested pattern (reported), when pattern differs
-  bool fuse = true;      // fuse two leading 'b' levels when the sizes allow
+  bool fuse = true;      // fuse consecutive 'b' levels when the sizes allow
   int tile = 0;          // leaf-GEMM block tile (0 default, 1 smaller)
   bool residue = false;  // matrices are nmod INT8 planes
   int m0 = 1;            // residue mode: the layout's leaf size
@@ -206,7 +206,7 @@ struct Builder {
     const size_t mark = top;
     std::vector<Prob> work = batch;
     // bs-blocked leaves of the layout (size m >> cutoff) need a reorder
-    const bool reorder = (bs != 1 && bs != (m >> cutoff));
+    const bool reorder = (leaf_bs != 1 && leaf_bs != (m >> cutoff));
     const long long mm = (long long)m * m;
     if (reorder) {
       Mat AA = alloc_mats(batch.size(), mm), BB = alloc_mats(batch.size(), mm),
@@ -222,7 +222,7 @@ struct Builder {
       for (size_t p = 0; p < batch.size(); p++)
         rr.push_back({reinterpret_cast<const double *>(batch[p].B.p),
                       reinterpret_cast<double *>(work[p].B.p)});
-      push(STEP_REORDER, 1, (int)rr.size(), m, bs,
+      push(STEP_REORDER, 1, (int)rr.size(), m, leaf_bs,
            add_table(rr.data(), rr.size() * sizeof(ReorderPtrs)));
     }
     if (mode == CAPS_MODE_FP64) {
@@ -240,7 +240,7 @@ struct Builder {
       for (size_t p = 0; p < batch.size(); p++)
         rc.push_back({reinterpret_cast<const double *>(work[p].C.p),
                       reinterpret_cast<double *>(batch[p].C.p)});
-      push(STEP_REORDER, 0, (int)rc.size(), m, bs,
+      push(STEP_REORDER, 0, (int)rc.size(), m, leaf_bs,
            add_table(rc.data(), rc.size() * sizeof(ReorderPtrs)));
     }
     top = mark;
@@ -370,66 +370,78 @@ struct Builder {
     top = mark;
   }
 
-  // the fused FP64 passes move 16-byte pairs
-  static bool aligned16(const Prob &p) {
-    return ((reinterpret_cast<uintptr_t>(p.A.p) | reinterpret_cast<uintptr_t>(p.B.p) |
-             reinterpret_cast<uintptr_t>(p.C.p)) & 15) == 0;
-  }
-
-  // Can two 'b' levels starting at `depth` run as fused passes?
+  // Can two residue 'b' levels starting at `depth` run as fused passes?
   bool fusable(size_t batch, int s, int nrec, int depth) const {
     if (!fuse || batch != 1 || nrec - cutoff < 2) return false;
     if (!(pattern[depth] == 'b' || pattern[depth] == 'B')) return false;
     if (!(pattern[depth + 1] == 'b' || pattern[depth + 1] == 'B')) return false;
     const long long q = area(s / 4);
-    return residue ? (q % 4 == 0) : (q % 2 == 0);
+    return residue && q % 4 == 0;
   }
 
-  // Can three FP64 'b' levels starting at `depth` run as fused passes?  (pad =
-  // false: as two and one, the size the fixed scratch's limit counts)
-  bool fusable3(size_t batch, int s, int nrec, int depth) const {
-    if (residue || !pad || !fuse || batch != 1 || nrec - cutoff < 3) return false;
-    for (int l = depth; l < depth + 3; l++)
-      if (pattern[l] != 'b' && pattern[l] != 'B') return false;
-    return b3_fits(area(s / 8));
+  // FP64 'b' levels starting at `depth` that run as fused passes: 3, 2 or 0.
+  // (pad = false: two, for even sub-blocks, the size the fixed scratch's limit
+  // counts)
+  int fusable_f64(const std::vector<Prob> &batch, int s, int nrec, int depth) const {
+    if (residue || !fuse || batch.size() != 1) return 0;
+    for (int levels = pad ? 3 : 2; levels >= 2; levels--) {
+      if (nrec - cutoff < levels) continue;
+      bool b = true;
+      for (int l = depth; l < depth + levels; l++) b = b && (pattern[l] == 'b' || pattern[l] == 'B');
+      const long long q = area(s >> levels);
+      if (b && fused_fits(q) && (pad || q % 2 == 0)) return levels;
+    }
+    return 0;
   }
 
-  // Three fused 'b' levels of one FP64 sub-problem (fused3.h)
-  void bfs3(const Prob &pb, int s, int nrec, int depth) {
-    const int sub = s / 8;
-    const long long q = area(sub), step = b3_step(q);
+  // Two or three fused 'b' levels of one FP64 sub-problem (fused_f64.h)
+  void fused_bfs(const Prob &pb, int s, int nrec, int depth, int levels) {
+    const int sub = s >> levels, products = fused_products(levels);
+    const long long q = area(sub), step = pad ? fused_step(q) : q;
     const size_t mark = top;
-    for (int l = 0; l < 3; l++) level_tag(depth + l);
-    plan.additions += (16 + 7 * 4 + 49) * 15LL * q;
+    // leaves in blocks become column-major here, once per position of A, B and
+    // C, and not once per leaf product
+    const bool blocked = pad && cutoff == 0 && leaf_bs != 1 && leaf_bs != m0;
+    const int written = fused_written(levels, blocked);
+    for (int l = 0, n = 1; l < levels; l++, n *= 7) {
+      level_tag(depth + l);
+      plan.additions += 15LL * n * area(s >> (l + 1));
+    }
     // plain operands are quadrants, passed by pointer
     const int quad[2][7] = {{0, 2, -1, -1, -1, -1, 3}, {0, 1, -1, -1, -1, 3, -1}};
     const Mat in[2] = {pb.A, pb.B};
-    const Mat L[2] = {alloc_mats(B3_WRITTEN, step), alloc_mats(B3_WRITTEN, step)};
-    const Mat Q = alloc_mats(343, step);
-    std::vector<Prob> next(343);
-    int written[2] = {0, 0};
-    for (int t = 0; t < 343; t++) {
-      const int i = t / 49, j = t / 7 % 7, k = t % 7;
+    const Mat L[2] = {alloc_mats(written, step), alloc_mats(written, step)};
+    const Mat Q = alloc_mats(products, step);
+    std::vector<Prob> next((size_t)products);
+    int k[2] = {0, 0};
+    for (int t = 0; t < products; t++) {
       Mat op[2];
-      for (int side = 0; side < 2; side++)
-        op[side] = bb_plain(side, i) && bb_plain(side, j) && bb_plain(side, k)
-                       ? at(in[side], (16 * quad[side][i] + 4 * quad[side][j] + quad[side][k]) * q)
-                       : at(L[side], written[side]++ * step);
-      next[t] = {op[0], op[1], at(Q, t * step)};
+      for (int side = 0; side < 2; side++) {
+        bool plain = !blocked;
+        int sb = 0;  // the sub-block a plain operand is
+        for (int n = products / 7; n > 0; n /= 7) {
+          plain = plain && bb_plain(side, t / n % 7);
+          sb = 4 * sb + quad[side][t / n % 7];
+        }
+        op[side] = plain ? at(in[side], sb * q) : at(L[side], k[side]++ * step);
+      }
+      next[(size_t)t] = {op[0], op[1], at(Q, t * step)};
     }
-    if (written[0] != B3_WRITTEN || written[1] != B3_WRITTEN) broken = true;
+    if (k[0] != written || k[1] != written) broken = true;
     const auto d = [](const Mat &m) { return reinterpret_cast<double *>(m.p); };
-    const B3Pre pre{{d(pb.A), d(pb.B)}, {d(L[0]), d(L[1])}, step};
-    push(STEP_B3_PRE, 0, 1, q, 0, add_table(&pre, sizeof(pre)));
-    rec(next, sub, nrec - 3, depth + 3);
-    const B3Post post{d(Q), step, d(pb.C)};
-    push(STEP_B3_POST, 0, 1, q, 0, add_table(&post, sizeof(post)));
+    const int lbs = blocked ? leaf_bs : 0;
+    const FusedPre pre{{d(pb.A), d(pb.B)}, {d(L[0]), d(L[1])}, step, m0, lbs};
+    push(STEP_FUSED_PRE, levels, 1, q, lbs, add_table(&pre, sizeof(pre)));
+    if (blocked) leaf_bs = 1;
+    rec(next, sub, nrec - levels, depth + levels);
+    if (blocked) leaf_bs = lbs;
+    const FusedPost post{d(Q), step, d(pb.C), m0, lbs};
+    push(STEP_FUSED_POST, levels, 1, q, lbs, add_table(&post, sizeof(post)));
     top = mark;
   }
 
-  // Two fused 'b' levels for one sub-problem (fused2.h).  In residue mode at
-  // the top, `crt` carries the reconstruction target and the combinations are
-  // fused with it.
+  // Two fused residue 'b' levels at the top (fused2.h): `crt` carries the
+  // reconstruction target, the combinations are fused with it.
   void bfs2(const Prob &pb, int s, int nrec, int depth, const CrtMats *crt) {
     const int sub = s / 4;
     const long long q = area(sub);
@@ -441,17 +453,17 @@ struct Builder {
     // plain sub-blocks passed by pointer: level-1 / level-2 operand -> quadrant
     const int quadA[7] = {0, 2, -1, -1, -1, -1, 3};  // T1 = A11, T2 = A12, T7 = A22
     const int quadB[7] = {0, 1, -1, -1, -1, 3, -1};  // S1 = B11, S2 = B21, S6 = B22
-    const bool fused_b = crt && crt->fused_b, fused_a = crt && crt->fused_a;
+    const bool fused_b = crt->fused_b, fused_a = crt->fused_a;
     Mat LA = alloc_mats(fused_a ? 49 : 40, q), LB = alloc_mats(fused_b ? 49 : 40, q),
         P2 = alloc_mats(49, q);
     // residue products written by the leaf GEMM itself (no level between) on
     // its 256-tile kernel: the 49 products of a modulus interleave in 128-byte
     // segments, so that the post-combination reads one contiguous 49 x 128
     // bytes per modulus for 128 positions
-    const bool seg = residue && nrec - 2 == cutoff && q % 128 == 0 &&
+    const bool seg = nrec - 2 == cutoff && q % 128 == 0 &&
                      residue_gemm_segmented(sub, cutoff, tile, mode == CAPS_MODE_CRT_BF16,
                                           49LL * moduli);
-    const long long pstep = seg ? 128 : q * es, cseg = seg ? 49 * 128 : 128;
+    const long long pstep = seg ? 128 : q, cseg = seg ? 49 * 128 : 128;
     // the kernels address the 40 written operands of a side as out + k * step
     // (k counts the non-plain (i, j) in order) and product (i, j) as
     // q + (7 i + j) * step
@@ -464,7 +476,7 @@ struct Builder {
     pre.out[1] = LB.p;
     pre.sout[0] = LA.ps;
     pre.sout[1] = LB.ps;
-    pre.step = q * es;
+    pre.step = q;
     std::vector<Prob> next(49);
     int ka = 0, kb = 0;
     for (int i = 0; i < 7; i++)
@@ -488,7 +500,7 @@ struct Builder {
         next[k] = {a, b, {P2.p + k * pstep, P2.ps}, cseg};
       }
     if (ka != (fused_a ? 0 : 40) || kb != (fused_b ? 0 : 40)) broken = true;
-    if (residue) ensure_consts();
+    ensure_consts();
     if (fused_b) {
       BBSplitB sp{};
       sp.B = crt->B;
@@ -511,7 +523,7 @@ struct Builder {
       sp.nrec2 = crt->nrec - 2;
       push(STEP_BB_SPLIT_A, 1, 1, q, crt->m, add_table(&sp, sizeof(sp)));
     } else {
-      push(STEP_BB_PRE, residue, 1, q, 0, add_table(&pre, sizeof(pre)), fused_b ? 1 : 0);
+      push(STEP_BB_PRE, 1, 1, q, 0, add_table(&pre, sizeof(pre)), fused_b ? 1 : 0);
     }
     rec(next, sub, nrec - 2, depth + 2);
     BBPost post{};
@@ -521,18 +533,14 @@ struct Builder {
     post.cseg = cseg;
     for (int k = 0; k < 49; k++)
       if (next[k].C.p != P2.p + k * pstep || next[k].C.ps != P2.ps) broken = true;
-    if (!residue) {
-      post.c = reinterpret_cast<double *>(pb.C.p);
-    } else {
-      post.out_c = crt->C;
-      post.sa = crt->sa;
-      post.sb = crt->sb;
-      post.sub = sub;
-      post.m0 = crt->m;
-      post.nrec2 = crt->nrec - 2;
-      post.bs = crt->bs;
-    }
-    push(STEP_BB_POST, residue, 1, q, 0, add_table(&post, sizeof(post)));
+    post.out_c = crt->C;
+    post.sa = crt->sa;
+    post.sb = crt->sb;
+    post.sub = sub;
+    post.m0 = crt->m;
+    post.nrec2 = crt->nrec - 2;
+    post.bs = crt->bs;
+    push(STEP_BB_POST, 1, 1, q, 0, add_table(&post, sizeof(post)));
     top = mark;
   }
 
@@ -541,12 +549,8 @@ struct Builder {
       leaf(batch, s);
       return;
     }
-    if (fusable3(batch.size(), s, nrec, depth)) {
-      bfs3(batch[0], s, nrec, depth);
-      return;
-    }
-    if (!residue && fusable(batch.size(), s, nrec, depth) && aligned16(batch[0])) {
-      bfs2(batch[0], s, nrec, depth, nullptr);
+    if (const int levels = fusable_f64(batch, s, nrec, depth)) {
+      fused_bfs(batch[0], s, nrec, depth, levels);
       return;
     }
     char c = pattern[depth];
@@ -656,7 +660,7 @@ hipError_t run_one(const Plan &plan, const Step &st, hipStream_t s) {
       return launch_residue_ew(st.op, reinterpret_cast<const RPtrs *>(tb + st.table), st.count,
                                st.n, plan.oz_moduli, st.vec2 != 0, kc, s);
     case STEP_BB_PRE:
-      return launch_bb_pre(reinterpret_cast<const BBPre *>(tb + st.table), st.n, st.op != 0,
+      return launch_bb_pre(reinterpret_cast<const BBPre *>(tb + st.table), st.n,
                            plan.oz_moduli, kc, s, st.vec2 != 0);
     case STEP_BB_SPLIT_B:
       return launch_bb_split_b(reinterpret_cast<const BBSplitB *>(tb + st.table), st.n, st.bs,
@@ -666,12 +670,14 @@ hipError_t run_one(const Plan &plan, const Step &st, hipStream_t s) {
                                kc, s);
 
     case STEP_BB_POST:
-      return launch_bb_post(reinterpret_cast<const BBPost *>(tb + st.table), st.n, st.op != 0,
-                            st.op ? ozaki_npieces(plan.oz_moduli) : 0, kc, s);
-    case STEP_B3_PRE:
-      return launch_b3_pre(reinterpret_cast<const B3Pre *>(tb + st.table), st.n, s);
-    case STEP_B3_POST:
-      return launch_b3_post(reinterpret_cast<const B3Post *>(tb + st.table), st.n, s);
+      return launch_bb_post(reinterpret_cast<const BBPost *>(tb + st.table), st.n,
+                            ozaki_npieces(plan.oz_moduli), kc, s);
+    case STEP_FUSED_PRE:
+      return launch_fused_pre(reinterpret_cast<const FusedPre *>(tb + st.table), st.op, st.n,
+                              st.bs != 0, s);
+    case STEP_FUSED_POST:
+      return launch_fused_post(reinterpret_cast<const FusedPost *>(tb + st.table), st.op, st.n,
+                               st.bs != 0, s);
     case STEP_CRT_SCALE:
     case STEP_CRT_SPLIT:
     case STEP_CRT_RECON:
@@ -699,12 +705,11 @@ hipError_t run_one(const Plan &plan, const Step &st, hipStream_t s) {
 }
 
 int timer_of(const Step &st) {
-  if (st.kind == STEP_BB_POST && st.op == 0) return CAPS_TIMER_ADD;
   switch (st.kind) {
     case STEP_EW:
     case STEP_REW:
-    case STEP_B3_PRE:
-    case STEP_B3_POST:
+    case STEP_FUSED_PRE:
+    case STEP_FUSED_POST:
     case STEP_BB_PRE: return CAPS_TIMER_ADD;
     case STEP_BB_POST: return CAPS_TIMER_RECON;
     case STEP_GEMM_F64:
@@ -739,7 +744,7 @@ int build_plan(Plan &plan, const double *A, const double *B, double *C, const ca
   plan.oz_moduli = 0;
   plan.crt_host.clear();
   Builder b{plan, reinterpret_cast<char *>(work_base)};
-  b.bs = d.bs;
+  b.leaf_bs = d.bs;
   b.mode = mode;
   b.moduli = moduli;
   b.cutoff = cutoff;
@@ -991,7 +996,7 @@ int build_batch_plan(Plan &plan, const std::vector<BatchItem> &items, int mode, 
                          std::vector<Step> *out, size_t &peak) {
     Builder b{into, base};
     b.out = out;
-    b.bs = g[0]->desc.bs;
+    b.leaf_bs = g[0]->desc.bs;
     b.mode = mode;
     b.moduli = moduli;
     b.cutoff = g[0]->cutoff;

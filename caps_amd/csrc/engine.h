@@ -44,8 +44,8 @@ enum StepKind : int {
   STEP_CRT_SCALE = 8,  // residue mode: scale exponents of the whole A and B
   STEP_CRT_SPLIT = 9,  // residue mode: A, B -> residue planes
   STEP_CRT_RECON = 10, // residue mode: C residues -> C
-  STEP_BB_PRE = 11,    // two 'b' levels of pre-additions in one pass (op = residue)
-  STEP_BB_POST = 12,   // two 'b' levels of combinations (residue: + reconstruction)
+  STEP_BB_PRE = 11,    // residue mode: two 'b' levels of pre-additions in one pass
+  STEP_BB_POST = 12,   // residue mode: two 'b' levels of combinations and the reconstruction
   STEP_BB_SPLIT_B = 13,  // residue mode: B's split fused with its two top 'b' levels, bs = m0
   // segmented launches (kernels.h VSeg) merging one step of several
   // problems of an uneven batch: table = segment array, count = segments,
@@ -56,8 +56,9 @@ enum StepKind : int {
   STEP_MULTI_RGEMM = 17, // INT8 residue leaf GEMMs, bs = block tile
   STEP_MULTI_CRT = 18,   // residue scale / split / reconstruct kernel op (CrtKernel), vec2 = flag
   STEP_BB_SPLIT_A = 19,  // residue mode: A's split fused with its two top 'b' levels, bs = m0
-  STEP_B3_PRE = 20,    // FP64: three 'b' levels of pre-additions in one pass
-  STEP_B3_POST = 21,   // FP64: three 'b' levels of combinations
+  STEP_FUSED_PRE = 20,   // FP64: op (2 or 3) 'b' levels of pre-additions in one pass, bs != 0:
+                         // leaves out of bs x bs blocks
+  STEP_FUSED_POST = 21,  // FP64: op 'b' levels of combinations, leaves back into blocks
 };
 
 struct Step {

@@ -1,4 +1,5 @@
-// Two consecutive batched Winograd levels in single passes (fused2.hip).
+// Two consecutive batched Winograd levels on residues in single passes
+// (fused2.hip; FP64: fused_f64.h).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -22,7 +23,7 @@ struct BBPre {
   void *out[2];           // the 40 written depth-2 operands (i, j) = operand j of level-1
                           // operand i, not plain, in (i, j) order, one every `step` bytes
   long long step;         // bytes between consecutive operands (q elements)
-  long long sin[2];       // residue mode: plane strides (bytes)
+  long long sin[2];       // plane strides (bytes)
   long long sout[2];
 };
 
@@ -30,14 +31,12 @@ struct BBPre {
 struct BBPost {
   const void *q;          // the 49 depth-2 products (i, j), product 7 i + j at (7 i + j) * step
   long long step;         // bytes
-  long long sq;           // residue mode: plane stride
-  // residue mode: position u of a product at (u >> 7) * cseg + (u & 127)
+  long long sq;           // plane stride
+  // position u of a product at (u >> 7) * cseg + (u & 127)
   // (128: plain planes; 49 * 128 with step = 128: the products interleaved
   // in 128-byte segments, as the 256-tile leaf GEMM writes them)
   long long cseg;
-  double *c;              // FP64 mode: C's 16 depth-2 sub-blocks at (4a + b) * q
-  // residue mode: reconstruct into FP64 C (CAPS layout) directly
-  double *out_c;
+  double *out_c;          // FP64 C (CAPS layout), reconstructed directly
   const int *sa, *sb;     // scale exponents of the global rows / columns
   int sub;                // depth-2 sub-block size (n / 4)
   int m0;                 // leaf size of the layout (products: pitch residue_pitch(m0))
@@ -72,10 +71,9 @@ struct BBSplitA {
   int nrec2;              // quadrant levels inside a depth-2 sub-block
 };
 
-// q: positions of a depth-2 sub-block (residue mode: with the leaves' pitch).
-// FP64: q % 2 == 0; residue: q % 4 == 0.  a_only (residue): side B is
-// produced by launch_bb_split_b instead.
-hipError_t launch_bb_pre(const BBPre *d_P, long long q, bool residue, int nmod,
+// q: positions of a depth-2 sub-block, with the leaves' pitch.
+// q % 4 == 0.  a_only: side B is produced by launch_bb_split_b instead.
+hipError_t launch_bb_pre(const BBPre *d_P, long long q, int nmod,
                          const OzakiConsts *d_consts, hipStream_t s, bool a_only = false);
 // m0: host copy of the table's leaf size; q < 2^31
 hipError_t launch_bb_split_b(const BBSplitB *d_P, long long q, int m0, int nmod,
@@ -83,7 +81,7 @@ hipError_t launch_bb_split_b(const BBSplitB *d_P, long long q, int m0, int nmod,
 // m0 % 128 == 0 (host copy of the table's m0), q < 2^31
 hipError_t launch_bb_split_a(const BBSplitA *d_P, long long q, int m0,
                              const OzakiConsts *d_consts, hipStream_t s);
-hipError_t launch_bb_post(const BBPost *d_P, long long q, bool residue, int npieces,
+hipError_t launch_bb_post(const BBPost *d_P, long long q, int npieces,
                           const OzakiConsts *d_consts, hipStream_t s);
 
 }  // namespace caps

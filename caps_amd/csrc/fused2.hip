@@ -1,4 +1,5 @@
-// Two consecutive batched ('b') Winograd levels fused into single passes.
+// Two consecutive batched ('b') Winograd levels on residues fused into single
+// passes (FP64: fused_f64.hip).
 //
 // Pre-additions: the 16 depth-2 sub-blocks of A (of B) at one position give
 // all 49 depth-2 operands T_j(T_i) (S_j(S_i)) at that position; one launch
@@ -7,13 +8,10 @@
 // by pointer).  Post-combinations: the 49 depth-2 products at one position
 // give C's 16 depth-2 sub-blocks.  The expression trees are exactly those of
 // two strassenBFS levels (multiply.cpp:272, 277, 195-210) applied one after
-// the other, so FP64 results are bit-identical to the unfused levels; on
-// residues every step is exact modulo m_l.
+// the other; every step is exact modulo m_l.
 //
-// HBM-bound: per position, FP64 pre reads 16 x 8 B and writes 40 x 8 B per
-// side; FP64 post reads 49 x 8 B and writes 16 x 8 B.  At the top of a
-// residue-domain multiply the splits of B and A are fused with their
-// pre-additions (16 FP64 values in, the residues of all 49 operands out; A's
+// HBM-bound.  At the top of a residue-domain multiply the splits of B and A are
+// fused with their pre-additions (16 FP64 values in, the residues of all 49 operands out; A's
 // transposed to row-major leaves on the way), and the residue post with the
 // CRT reconstruction: 49 x nmod bytes in, 16 FP64 results out (its VALU work,
 // about 4,900 lane instructions per position for 14 moduli, is close to its
@@ -56,96 +54,6 @@ __device__ __forceinline__ void level_ops(int side, const V (&q)[4], V (&o)[7]) 
     o[0] = q[0]; o[1] = q[2]; o[2] = y[0]; o[3] = y[1]; o[4] = y[2]; o[5] = y[3]; o[6] = q[3];
   } else {
     o[0] = q[0]; o[1] = q[1]; o[2] = y[4]; o[3] = y[5]; o[4] = y[6]; o[5] = q[3]; o[6] = y[7];
-  }
-}
-
-// ---------------------------------------------------------------- FP64 pre
-// thread: 2 consecutive positions, 16-byte loads and stores; grid.y: side
-__global__ __launch_bounds__(T) void bb_pre_f64_kernel(const BBPre *__restrict__ P, long long q) {
-  const int side = blockIdx.y;
-  const double *in = reinterpret_cast<const double *>(P->in[side]);
-  const long long n2 = q >> 1;
-  for (long long u = (long long)blockIdx.x * T + threadIdx.x; u < n2;
-       u += (long long)gridDim.x * T) {
-    double l1[2][7][4];  // [position][level-1 operand i][sub-position q2]
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-      double q0[4], q1[4];
-#pragma unroll
-      for (int a = 0; a < 4; a++) {
-        const double2 v = reinterpret_cast<const double2 *>(in + (4 * a + b) * q)[u];
-        q0[a] = v.x;
-        q1[a] = v.y;
-      }
-      double o0[7], o1[7];
-      level_ops(side, q0, o0);
-      level_ops(side, q1, o1);
-#pragma unroll
-      for (int i = 0; i < 7; i++) {
-        l1[0][i][b] = o0[i];
-        l1[1][i][b] = o1[i];
-      }
-    }
-    char *out = reinterpret_cast<char *>(P->out[side]);
-    int k = 0;  // index among the written operands (compile-time after unrolling)
-#pragma unroll
-    for (int i = 0; i < 7; i++) {
-      double q0[4] = {l1[0][i][0], l1[0][i][1], l1[0][i][2], l1[0][i][3]};
-      double q1[4] = {l1[1][i][0], l1[1][i][1], l1[1][i][2], l1[1][i][3]};
-      double o0[7], o1[7];
-      level_ops(side, q0, o0);
-      level_ops(side, q1, o1);
-#pragma unroll
-      for (int j = 0; j < 7; j++) {
-        if (bb_plain(side, i) && bb_plain(side, j)) continue;
-        reinterpret_cast<double2 *>(out + k * P->step)[u] = make_double2(o0[j], o1[j]);
-        k++;
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------- FP64 post
-// thread: 2 consecutive positions, 16-byte loads and stores
-__global__ __launch_bounds__(T) void bb_post_f64_kernel(const BBPost *__restrict__ P, long long q) {
-  const long long n2 = q >> 1;
-  for (long long u = (long long)blockIdx.x * T + threadIdx.x; u < n2;
-       u += (long long)gridDim.x * T) {
-    double l1[2][7][4];  // [position][product i of level 1][sub-position q2]
-#pragma unroll
-    for (int i = 0; i < 7; i++) {
-      double q0[7], q1[7], c0[4], c1[4];
-#pragma unroll
-      for (int j = 0; j < 7; j++) {
-        const double2 v =
-            reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(P->q) +
-                                              (7 * i + j) * P->step)[u];
-        q0[j] = v.x;
-        q1[j] = v.y;
-      }
-      Ew<EW_BFS_POST>::apply(q0, c0);  // C11 C21 C12 C22 of product i
-      Ew<EW_BFS_POST>::apply(q1, c1);
-#pragma unroll
-      for (int b = 0; b < 4; b++) {
-        l1[0][i][b] = c0[b];
-        l1[1][i][b] = c1[b];
-      }
-    }
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-      double q0[7], q1[7], c0[4], c1[4];
-#pragma unroll
-      for (int i = 0; i < 7; i++) {
-        q0[i] = l1[0][i][b];
-        q1[i] = l1[1][i][b];
-      }
-      Ew<EW_BFS_POST>::apply(q0, c0);
-      Ew<EW_BFS_POST>::apply(q1, c1);
-#pragma unroll
-      for (int a = 0; a < 4; a++)
-        reinterpret_cast<double2 *>(reinterpret_cast<double *>(P->c) + (4 * a + b) * q)[u] =
-            make_double2(c0[a], c1[a]);
-    }
   }
 }
 
@@ -510,18 +418,12 @@ unsigned blocks_for(long long units, int per_grid) {
 
 }  // namespace
 
-hipError_t launch_bb_pre(const BBPre *P, long long q, bool residue, int nmod,
-                         const OzakiConsts *kc, hipStream_t s, bool a_only) {
-  if (!residue) {
-    if (q % 2) return hipErrorInvalidValue;
-    dim3 g(blocks_for(q / 2, 2), 2);
-    hipLaunchKernelGGL(bb_pre_f64_kernel, g, dim3(T), 0, s, P, q);
-  } else {
-    if (q % 4 || q >= (1LL << 31)) return hipErrorInvalidValue;
-    dim3 g(blocks_for(q / 4, 2 * nmod), nmod);
-    hipLaunchKernelGGL(bb_pre_res_kernel<0>, g, dim3(T), 0, s, P, q, kc);
-    if (!a_only) hipLaunchKernelGGL(bb_pre_res_kernel<1>, g, dim3(T), 0, s, P, q, kc);
-  }
+hipError_t launch_bb_pre(const BBPre *P, long long q, int nmod, const OzakiConsts *kc,
+                         hipStream_t s, bool a_only) {
+  if (q % 4 || q >= (1LL << 31)) return hipErrorInvalidValue;
+  dim3 g(blocks_for(q / 4, 2 * nmod), nmod);
+  hipLaunchKernelGGL(bb_pre_res_kernel<0>, g, dim3(T), 0, s, P, q, kc);
+  if (!a_only) hipLaunchKernelGGL(bb_pre_res_kernel<1>, g, dim3(T), 0, s, P, q, kc);
   return hipGetLastError();
 }
 
@@ -552,20 +454,15 @@ hipError_t launch_bb_split_a(const BBSplitA *P, long long q, int m0, const Ozaki
   return hipGetLastError();
 }
 
-hipError_t launch_bb_post(const BBPost *P, long long q, bool residue, int npieces,
-                          const OzakiConsts *kc, hipStream_t s) {
-  if (!residue) {
-    if (q % 2) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(bb_post_f64_kernel, dim3(blocks_for(q / 2, 1)), dim3(T), 0, s, P, q);
-  } else {
-    if (q % 4) return hipErrorInvalidValue;
-    dim3 g((unsigned)((q + PPOS - 1) / PPOS));
-    switch (npieces) {
-      case 1:
-      case 2: hipLaunchKernelGGL((bb_post_crt_kernel<2>), g, dim3(T), 0, s, P, q, kc); break;
-      case 3: hipLaunchKernelGGL((bb_post_crt_kernel<3>), g, dim3(T), 0, s, P, q, kc); break;
-      default: hipLaunchKernelGGL((bb_post_crt_kernel<4>), g, dim3(T), 0, s, P, q, kc); break;
-    }
+hipError_t launch_bb_post(const BBPost *P, long long q, int npieces, const OzakiConsts *kc,
+                          hipStream_t s) {
+  if (q % 4) return hipErrorInvalidValue;
+  dim3 g((unsigned)((q + PPOS - 1) / PPOS));
+  switch (npieces) {
+    case 1:
+    case 2: hipLaunchKernelGGL((bb_post_crt_kernel<2>), g, dim3(T), 0, s, P, q, kc); break;
+    case 3: hipLaunchKernelGGL((bb_post_crt_kernel<3>), g, dim3(T), 0, s, P, q, kc); break;
+    default: hipLaunchKernelGGL((bb_post_crt_kernel<4>), g, dim3(T), 0, s, P, q, kc); break;
   }
   return hipGetLastError();
 }
