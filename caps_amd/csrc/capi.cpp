@@ -96,9 +96,21 @@ State &st() {
 }
 
 constexpr size_t MAX_PLANS = 24;
-// plans with more launches than this (deep 'd' recursions: 7^d leaf
-// products one after another) are launched directly instead of captured
+// Plans of few launches, and those with very many (deep 'd' recursions: 7^d
+// leaf products one after another), are launched directly, the others as a
+// captured graph.  A graph launch leaves the device idle for about 5 us more
+// than the launches it replaces and takes longer on the host (us per call,
+// graph and direct: n = 64 27.7 and 16.3, n = 1024 55.8 and 51.0, n = 2048 331
+// and 325), and its first call captures and instantiates it (n = 408 327 and
+// 222); over some tens of launches the two are level (32 uneven problems 1993
+// and 1983) and the graph spares the host.
+constexpr size_t MAX_DIRECT_STEPS = 16;
 constexpr size_t MAX_GRAPH_STEPS = 16384;
+
+bool by_graph(const Plan &p, const caps_opts *o) {
+  return !(o && (o->flags & (CAPS_FLAG_NO_GRAPH | CAPS_FLAG_TIMERS))) &&
+         p.steps.size() > MAX_DIRECT_STEPS && p.steps.size() <= MAX_GRAPH_STEPS;
+}
 
 int ensure_device_locked(State &s) {
   int dev = 0;
@@ -374,8 +386,7 @@ int multiply_device_locked(State &s, const double *dA, const double *dB, double 
                        plan);
   if (rc) return rc;
   const bool timed = opts && (opts->flags & CAPS_FLAG_TIMERS);
-  const bool use_graph = !timed && !(opts && (opts->flags & CAPS_FLAG_NO_GRAPH)) &&
-                         plan->steps.size() <= MAX_GRAPH_STEPS;
+  const bool use_graph = by_graph(*plan, opts);
   if (timed) {
     hipError_t e = run_steps_timed(*plan, stream, s.timers_ms, s.timed);
     if (e != hipSuccess) return fail(CAPS_EHIP, "timed launch: %s", hipGetErrorString(e));
@@ -769,8 +780,7 @@ int caps_multiply_batch_device(int count, const double *const *dA, const double 
         plan);
     if (rc) return rc;
   }
-  const bool use_graph = !(opts && (opts->flags & (CAPS_FLAG_NO_GRAPH | CAPS_FLAG_TIMERS))) &&
-                         plan->steps.size() <= MAX_GRAPH_STEPS;
+  const bool use_graph = by_graph(*plan, opts);
   if (opts && (opts->flags & CAPS_FLAG_TIMERS)) {
     hipError_t e = run_steps_timed(*plan, (hipStream_t)stream, s.timers_ms, s.timed);
     if (e != hipSuccess) return fail(CAPS_EHIP, "timed launch: %s", hipGetErrorString(e));

@@ -89,9 +89,10 @@ typedef struct caps_opts {
 } caps_opts;
 
 /* Re-use a captured hipGraph for repeated calls with the same pointers,
- * descriptor, pattern, options and stream (default on).  A cached plan owns
- * one device workspace and belongs to one stream: calls on different streams
- * never share a workspace, and calls on one stream run in stream order. */
+ * descriptor, pattern, options and stream (default on, for plans of more than
+ * a few launches: those are launched directly).  A cached plan owns one device
+ * workspace and belongs to one stream: calls on different streams never share
+ * a workspace, and calls on one stream run in stream order. */
 #define CAPS_FLAG_NO_GRAPH 1
 /* Force the reference's automatic rule when pattern == NULL (DFS at every
  * level on one process, multiply.cpp:43-66) instead of the planner's choice. */
