@@ -278,7 +278,7 @@ int get_plan_locked(State &s, const double *A, const double *B, double *C, const
                     hipStream_t stream, int tile, Plan *&out) {
   PlanKey key{A,  B,    C,             d,      pat,  mode, moduli, cutoff,
               fuse, std::string(), stream, tile,
-              batch_levels(d, pat, mode, moduli, cutoff, batch_limit_bytes(s))};
+              batch_levels(d, pat, mode, moduli, cutoff, batch_limit_bytes(s), BATCH_ANY_ALONE)};
   for (;;) {
     for (auto &p : s.plans)
       if (p->key == key) {
@@ -501,7 +501,8 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
   // hold this device's scratch addresses
   PlanKey key{dA, dB, dC, *desc, pat, mode, moduli, cutoff, fuse,
               "scratch of device " + std::to_string(s.device), nullptr, tile,
-              batch_levels(*desc, pat, mode, moduli, cutoff, batch_limit_bytes(s))};
+              batch_levels(*desc, pat, mode, moduli, cutoff, batch_limit_bytes(s),
+                           BATCH_ANY_SHARED)};
   Plan *p = nullptr;
   for (auto &hp : s.host_plans)
     if (hp->key == key) {
@@ -751,7 +752,7 @@ int caps_multiply_batch_device(int count, const double *const *dA, const double 
     // recursive levels run batched within the item's share of the budget (the
     // key holds the pattern as run)
     items[i].pattern = batch_levels(descs[i], items[i].pattern, mode, moduli, cutoff,
-                                    (size_t)share * sizeof(double), count);
+                                    (size_t)share * sizeof(double), BATCH_ANY_SHARED, count);
     char buf[176];
     snprintf(buf, sizeof(buf), "%p %p %p %d %d %d %d %s;", (const void *)dA[i],
              (const void *)dB[i], (void *)dC[i], descs[i].lda, descs[i].nrec, descs[i].bs, cutoff,

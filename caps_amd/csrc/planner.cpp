@@ -73,17 +73,17 @@ double workspace_estimate(const caps_desc &d, const std::string &pattern, int mo
 // workspace at two half-size matrices.  On this device that leaves small
 // products alone on 256 CUs and costs 13 dependent launches per level, while
 // 288 GB hold far more than the operands; BFS and DFS steps evaluate the same
-// expression trees.  Measured (FP64): n = 4096 'ddd' 7.42 ms recursive, 2.26
-// ms with its two lower levels batched; n = 392 'bdd' 563 and 47 us.
+// expression trees.  Measured (FP64): n = 4096 'ddd' 7.42 ms recursive, 2.07
+// ms with its two lower levels batched, 1.78 with all three (2 GB); n = 392
+// 'bdd' 563 and 47 us.
 std::string batch_levels(const caps_desc &d, const std::string &pattern, int mode, int moduli,
-                         int cutoff, size_t limit_bytes, int items) {
+                         int cutoff, size_t limit_bytes, size_t any_bytes, int items) {
   std::string run = pattern;
   // a launch takes at most 65,535 leaves of the leaf-only split (grid.y)
   double batch = items;
   for (int l = 0; l < d.nrec - cutoff; l++)
     if (pattern[(size_t)l] == 'b' || pattern[(size_t)l] == 'B') batch *= 7;
-  // 64 MiB (a 4096th of the device) however small the operands are
-  const double extra = std::max(24.0 * d.lda * d.lda, (double)(64 << 20));
+  const double extra = std::max(24.0 * d.lda * d.lda, (double)any_bytes);
   const double limit = std::min(workspace_estimate(d, pattern, mode, moduli, cutoff) + extra,
                                 (double)limit_bytes);
   for (int l = d.nrec - cutoff - 1; l >= 0; l--) {

@@ -17,11 +17,16 @@ std::string choose_pattern(const caps_desc &d, int mode, int moduli, long long b
                            bool budget_set);
 
 // The pattern a plan runs for the requested one: recursive levels run batched,
-// the deepest first, while they add at most the operands' own bytes (or 64 MiB)
-// to the requested pattern's workspace, within limit_bytes.  The results do not
-// depend on it.  items: problems of the same shape planned together.
+// the deepest first, while they add at most the operands' own bytes (or
+// any_bytes) to the requested pattern's workspace, within limit_bytes.  The
+// results do not depend on it.  items: problems of the same shape planned
+// together.
 std::string batch_levels(const caps_desc &d, const std::string &pattern, int mode, int moduli,
-                         int cutoff, size_t limit_bytes, int items = 1);
+                         int cutoff, size_t limit_bytes, size_t any_bytes, int items = 1);
+// any_bytes of one multiply with a workspace of its own (a 72nd of the device),
+// and of a problem that shares the device with many or a scratch array
+constexpr size_t BATCH_ANY_ALONE = (size_t)4 << 30;
+constexpr size_t BATCH_ANY_SHARED = (size_t)64 << 20;
 
 // Leaf arithmetic when the caller asks for CAPS_MODE_AUTO.
 int choose_mode(const caps_desc &d);

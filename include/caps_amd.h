@@ -129,9 +129,9 @@ long long caps_num_entries(const caps_desc *desc);
  * A and B are only read; C is overwritten.  pattern: one char per recursion
  * level from [bBdDhH] ('b' = batched level, 'd'/'h' = recursive level), or
  * NULL for the planner's choice.  A recursive level whose batched form adds at
- * most the operands' own size (or 64 MiB) of workspace, within a budget set by
- * caps_set_available_memory, runs batched: the same bits, reported as
- * requested.  opts may be NULL (FP64 mode).
+ * most the operands' own size (or 4 GiB; in a batch or the scratch array 64
+ * MiB) of workspace, within a budget set by caps_set_available_memory, runs
+ * batched: the same bits, reported as requested.  opts may be NULL (FP64 mode).
  * multiply.h:13 / multiply.cpp:9-25. */
 int caps_multiply(const double *A, const double *B, double *C,
                   const caps_desc *desc, const char *pattern,

@@ -54,3 +54,10 @@ def test_small_recursive_levels(n, r, bs, pattern, cutoff, mode):
     torch.cuda.synchronize()
     assert torch.equal(N, out[0][0]) and caps_amd.counters()["pattern"] == want
     caps_amd.release()
+
+
+@pytest.mark.parametrize("mode", [caps_amd.MODE_FP64, caps_amd.MODE_CRT_INT8])
+@pytest.mark.parametrize("n,r,bs,pattern", [(1536, 2, 3, "dd"), (2048, 3, 1, "ddd")])
+def test_levels_above_the_operands_size(n, r, bs, pattern, mode):
+    """More workspace than the operands' size, little for the device."""
+    test_small_recursive_levels(n, r, bs, pattern, 0, mode)
