@@ -55,6 +55,7 @@ struct Builder {
   std::string pattern;
   std::string tags;      // the requested pattern (reported), when pattern differs
   bool fuse = true;      // fuse consecutive 'b' levels when the sizes allow
+  bool shared = false;   // the plan holds other groups, whose steps may merge with these
   int tile = 0;          // leaf-GEMM block tile (0 default, 1 smaller)
   bool residue = false;  // matrices are nmod INT8 planes
   int m0 = 1;            // residue mode: the layout's leaf size
@@ -379,12 +380,13 @@ struct Builder {
     return residue && q % 4 == 0;
   }
 
-  // FP64 'b' levels starting at `depth` that run as fused passes: 3, 2 or 0.
+  // FP64 'b' levels starting at `depth` that run as fused passes: 3, 2, 1 or 0.
   // (pad = false: two, for even sub-blocks, the size the fixed scratch's limit
   // counts)
   int fusable_f64(const std::vector<Prob> &batch, int s, int nrec, int depth) const {
     if (residue || !fuse || batch.size() != 1) return 0;
-    for (int levels = pad ? 3 : 2; levels >= 2; levels--) {
+    // (in a batch a level alone joins the other groups' in one launch instead)
+    for (int levels = pad ? 3 : 2; levels >= (pad && !shared ? 1 : 2); levels--) {
       if (nrec - cutoff < levels) continue;
       bool b = true;
       for (int l = depth; l < depth + levels; l++) b = b && (pattern[l] == 'b' || pattern[l] == 'B');
@@ -394,7 +396,7 @@ struct Builder {
     return 0;
   }
 
-  // Two or three fused 'b' levels of one FP64 sub-problem (fused_f64.h)
+  // One to three fused 'b' levels of one FP64 sub-problem (fused_f64.h)
   void fused_bfs(const Prob &pb, int s, int nrec, int depth, int levels) {
     const int sub = s >> levels, products = fused_products(levels);
     const long long q = area(sub), step = pad ? fused_step(q) : q;
@@ -1006,6 +1008,7 @@ int build_batch_plan(Plan &plan, const std::vector<BatchItem> &items, int mode, 
     b.planes = b.residue ? moduli : 1;
     b.m0 = g[0]->desc.lda >> g[0]->desc.nrec;
     b.fuse = true;
+    b.shared = true;
     b.tile = tile;
     if (b.residue) {
       b.crt_group(g);

@@ -56,7 +56,7 @@ enum StepKind : int {
   STEP_MULTI_RGEMM = 17, // INT8 residue leaf GEMMs, bs = block tile
   STEP_MULTI_CRT = 18,   // residue scale / split / reconstruct kernel op (CrtKernel), vec2 = flag
   STEP_BB_SPLIT_A = 19,  // residue mode: A's split fused with its two top 'b' levels, bs = m0
-  STEP_FUSED_PRE = 20,   // FP64: op (2 or 3) 'b' levels of pre-additions in one pass, bs != 0:
+  STEP_FUSED_PRE = 20,   // FP64: op (1 to 3) 'b' levels of pre-additions in one pass, bs != 0:
                          // leaves out of bs x bs blocks
   STEP_FUSED_POST = 21,  // FP64: op 'b' levels of combinations, leaves back into blocks
 };

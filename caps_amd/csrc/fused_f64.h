@@ -1,4 +1,4 @@
-// Two or three consecutive batched Winograd levels of an FP64 product in single
+// One to three consecutive batched Winograd levels of an FP64 product in single
 // passes (fused_f64.hip).  With L levels a matrix has 4^L sub-blocks of q
 // elements, numbered by their quadrants from the outermost level on ((a, b) at
 // (4 a + b) * q, (a, b, c) at (16 a + 4 b + c) * q), and 7^L operands a side,
@@ -26,9 +26,9 @@ struct FusedPost {
   int m, bs;        // as in FusedPre: products column-major, C blocked
 };
 
-constexpr int fused_products(int levels) { return levels == 2 ? 49 : 343; }
+constexpr int fused_products(int levels) { return levels == 1 ? 7 : (levels == 2 ? 49 : 343); }
 constexpr int fused_written(int levels, bool all) {
-  return fused_products(levels) - (all ? 0 : (levels == 2 ? 9 : 27));
+  return fused_products(levels) - (all ? 0 : (levels == 1 ? 3 : (levels == 2 ? 9 : 27)));
 }
 
 // operands and products lie on whole 128-byte lines (none has two writers), an

@@ -1,4 +1,4 @@
-// Two or three Winograd levels of an FP64 product per pass (fused_f64.h): the
+// One to three Winograd levels of an FP64 product per pass (fused_f64.h): the
 // operands of a level are never written for the next one to read.  Per element
 // of A or B a pass over three levels moves 1 + 316/64 elements where passes over
 // two and one move 3.5 + 6.1, and back 343/64 + 1 where those move 8.4 + 4.1.
@@ -119,7 +119,12 @@ __device__ __forceinline__ unsigned blocked_offset(unsigned p, int m, int bs) {
 template <int SIDE, int LEVELS, bool ALL>
 __device__ __forceinline__ void pre_all(gcdouble *in, gdouble *out, long long q, long long step,
                                         unsigned u0, unsigned u) {
-  if constexpr (LEVELS == 2) {
+  if constexpr (LEVELS == 1) {
+    double x[4];
+#pragma unroll
+    for (int a = 0; a < 4; a++) x[a] = *at(in + a * q, u0);
+    store_k<SIDE, !ALL, 0, 0>(x, out, step, u);
+  } else if constexpr (LEVELS == 2) {
     double x[4][4];
     load_quad(in, 0, q, u0, x);
     store_jk<SIDE, !ALL, 0>(x, out, step, u);
@@ -251,6 +256,15 @@ __global__ __launch_bounds__(T, 2) void fused_post_kernel(const FusedPost *__res
   gcdouble *in = (gcdouble *)P->q;
   gdouble *out = (gdouble *)P->c;
   const long long step = P->step;
+  if constexpr (LEVELS == 1) {
+    double v[7], c[4];
+#pragma unroll
+    for (int k = 0; k < 7; k++) v[k] = __builtin_nontemporal_load(at(in + k * step, u));
+    combine(v, c);
+#pragma unroll
+    for (int a = 0; a < 4; a++) *at(out + a * q, u0) = c[a];
+    return;
+  }
   double w[4][4], y[4][4], z[4][4], r[4][4];
   product(in, 0, step, u, w);
   if constexpr (LEVELS == 2) {
@@ -336,7 +350,7 @@ hipError_t launch_pre(const FusedPre *P, long long q, hipStream_t s) {
   const unsigned b256 = (unsigned)((q + 255) / 256), b64 = (unsigned)((q + 63) / 64);
   if (b256 >= cus)
     hipLaunchKernelGGL((fused_pre_kernel<256, LEVELS, ALL>), dim3(b256, 2), dim3(256), 0, s, P, q);
-  else if (LEVELS == 2 || b64 >= cus)
+  else if (LEVELS < 3 || b64 >= cus)
     hipLaunchKernelGGL((fused_pre_kernel<64, LEVELS, ALL>), dim3(b64, 2), dim3(64), 0, s, P, q);
   else
     hipLaunchKernelGGL((fused_pre_split_kernel<64, ALL>), dim3(b64, 14), dim3(64), 0, s, P, q);
@@ -350,7 +364,7 @@ hipError_t launch_post(const FusedPost *P, long long q, hipStream_t s) {
   if (b256 >= cus)
     hipLaunchKernelGGL((fused_post_kernel<256, LEVELS, BLOCKED>), dim3(b256), dim3(256), 0, s, P,
                        q);
-  else if (LEVELS == 2 || b64 >= cus)
+  else if (LEVELS < 3 || b64 >= cus)
     hipLaunchKernelGGL((fused_post_kernel<64, LEVELS, BLOCKED>), dim3(b64), dim3(64), 0, s, P, q);
   else
     hipLaunchKernelGGL((fused_post_split_kernel<64, BLOCKED>), dim3(b64, 16), dim3(64), 0, s, P,
@@ -362,14 +376,16 @@ hipError_t launch_post(const FusedPost *P, long long q, hipStream_t s) {
 
 hipError_t launch_fused_pre(const FusedPre *P, int levels, long long q, bool blocked,
                             hipStream_t s) {
-  if (!fused_fits(q) || levels < 2 || levels > 3) return hipErrorInvalidValue;
+  if (!fused_fits(q) || levels < 1 || levels > 3) return hipErrorInvalidValue;
+  if (levels == 1) return blocked ? launch_pre<1, true>(P, q, s) : launch_pre<1, false>(P, q, s);
   if (levels == 2) return blocked ? launch_pre<2, true>(P, q, s) : launch_pre<2, false>(P, q, s);
   return blocked ? launch_pre<3, true>(P, q, s) : launch_pre<3, false>(P, q, s);
 }
 
 hipError_t launch_fused_post(const FusedPost *P, int levels, long long q, bool blocked,
                              hipStream_t s) {
-  if (!fused_fits(q) || levels < 2 || levels > 3) return hipErrorInvalidValue;
+  if (!fused_fits(q) || levels < 1 || levels > 3) return hipErrorInvalidValue;
+  if (levels == 1) return blocked ? launch_post<1, true>(P, q, s) : launch_post<1, false>(P, q, s);
   if (levels == 2) return blocked ? launch_post<2, true>(P, q, s) : launch_post<2, false>(P, q, s);
   return blocked ? launch_post<3, true>(P, q, s) : launch_post<3, false>(P, q, s);
 }

@@ -1,4 +1,4 @@
-"""Two and three batched FP64 levels in single passes: the bits of the level-by-level
+"""One to three batched FP64 levels in single passes: the bits of the level-by-level
 run (FLAG_NO_FUSION, the same expression trees) at odd and even leaf sizes, with
 one position and with partly filled blocks, on both sides of the order from
 which a thread takes all of a side, nested and below other levels, at operands
@@ -35,6 +35,12 @@ def test_bits_of_the_level_by_level_run(m, pattern, bs, offset):
     (130, "bb", 5, 0), (257, "bb", 1, 0), (258, "bb", 3, 1), (35, "dbb", 5, 0)])
 def test_two_levels_give_them_too(m, pattern, bs, offset):
     """Also at odd sizes and 8-byte alignment, plain and blocked leaves."""
+    _same_bits(m, pattern, bs, offset)
+
+
+@pytest.mark.parametrize("m,pattern,bs,offset", [
+    (1, "b", 1, 0), (9, "b", 1, 1), (49, "b", 7, 0), (300, "b", 4, 1), (513, "b", 1, 0)])
+def test_one_level_gives_them(m, pattern, bs, offset):
     _same_bits(m, pattern, bs, offset)
 
 
