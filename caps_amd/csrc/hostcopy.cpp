@@ -1,7 +1,10 @@
 #include "hostcopy.h"
 
+#include <emmintrin.h>
+
 #include <algorithm>
 #include <atomic>
+#include <cstdint>
 #include <cstring>
 #include <memory>
 #include <new>
@@ -22,9 +25,39 @@ constexpr size_t PIECE = CHUNK / PIECES;
 // with the calling thread: more than four gain nothing (memory bound)
 constexpr int MAX_HELPERS = 3;
 constexpr size_t BYTES_PER_HELPER = 2 * CHUNK;
+// What a helper reads stays in its core's caches too: a caller that refills
+// operands of 10 or 26 MB after the call then takes 8 and 18 ms, 2.4 and 6.6 if
+// it read them itself, which up to there is as quick (n = 800 550 and 564 us, n =
+// 1280 1098 and 1041).  From 32 MiB on little of them is left in those caches
+// (36 MB: 11.5 and 10.2 ms) and helpers pay (n = 1536 2042 -> 1379 us, n = 2048
+// 3475 -> 2634).
+constexpr size_t UP_HELPER_BYTES = (size_t)32 << 20;
 // smaller copies are the runtime's: it is as quick or quicker below (a multiply
 // of host arrays of 0.5 MiB 114 us against 137, of 1.25 MiB 229 against 205)
 constexpr size_t DIRECT_BYTES = (size_t)1 << 20;
+
+// memcpy past the caches: what a helper writes would else stay in its core's
+// caches, and the caller's next pass over the array would fetch it from there
+void stream_copy(char *dst, const char *src, size_t n) {
+  const size_t head = std::min(n, (size_t)(-reinterpret_cast<uintptr_t>(dst) & 15));
+  memcpy(dst, src, head);
+  dst += head;
+  src += head;
+  n -= head;
+  for (; n >= 64; n -= 64, dst += 64, src += 64) {
+    _mm_prefetch(src + 512, _MM_HINT_NTA);
+    const __m128i a = _mm_loadu_si128(reinterpret_cast<const __m128i *>(src));
+    const __m128i b = _mm_loadu_si128(reinterpret_cast<const __m128i *>(src + 16));
+    const __m128i c = _mm_loadu_si128(reinterpret_cast<const __m128i *>(src + 32));
+    const __m128i d = _mm_loadu_si128(reinterpret_cast<const __m128i *>(src + 48));
+    _mm_stream_si128(reinterpret_cast<__m128i *>(dst), a);
+    _mm_stream_si128(reinterpret_cast<__m128i *>(dst + 16), b);
+    _mm_stream_si128(reinterpret_cast<__m128i *>(dst + 32), c);
+    _mm_stream_si128(reinterpret_cast<__m128i *>(dst + 48), d);
+  }
+  memcpy(dst, src, n);
+  _mm_sfence();  // the stores are visible before the piece counts as done
+}
 
 struct Chunk {
   char *dev, *host;
@@ -103,9 +136,9 @@ class Pieces {
       const size_t n = std::min(PIECE, k.bytes - off);
       char *slot = ring_ + (size_t)(c % slots_) * CHUNK + off;
       if (up_)
-        memcpy(slot, k.host + off, n);
+        stream_copy(slot, k.host + off, n);
       else
-        memcpy(k.host + off, slot, n);
+        stream_copy(k.host + off, slot, n);
     }
     done_[c].fetch_add(1, std::memory_order_release);
   }
@@ -177,7 +210,9 @@ hipError_t HostCopy::send(const HostRange *r, int count, hipStream_t s) try {
   const bool two = n > 1;
   Pieces pieces(chunks, ring_, SLOTS, true);
   pieces.set_avail(std::min(n, SLOTS));
-  pieces.start_helpers();
+  size_t bytes = 0;
+  for (const Chunk &c : chunks) bytes += c.bytes;
+  if (bytes >= UP_HELPER_BYTES) pieces.start_helpers();
   int issued = 0, retired = 0;  // chunks given to the DMA, chunks it is done with
   while (issued < n) {
     if (pieces.done(issued)) {

@@ -4,8 +4,9 @@
 // The runtime's own copy of pageable memory runs at 33 GB/s up and 18 GB/s
 // down here (32 MiB), the DMA engines at 56 GB/s from pinned memory, one CPU
 // thread's memcpy at 28-33 GB/s and four at 107 GB/s.  So a copy is cut into
-// chunks: a few threads move pieces between the caller's memory and the ring
-// while two streams move whole chunks between the ring and the device.
+// chunks: the calling thread, with a few helpers where they are worth it, moves
+// pieces between the caller's memory and the ring while two streams move whole
+// chunks between the ring and the device.
 #pragma once
 #include <hip/hip_runtime.h>
 
