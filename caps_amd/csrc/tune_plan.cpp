@@ -65,8 +65,9 @@ std::vector<caps_candidate> enumerate_candidates(const caps_desc &d, int mask) {
     for (int cutoff = 0; cutoff <= d.nrec; cutoff++) {
       if (cutoff > 0 && (ms.mode == CAPS_MODE_OZAKI_INT8 || m0 % 128 != 0 || !plain_leaf)) break;
       const int L = d.nrec - cutoff;
-      // leaf-GEMM block tiles: FP64 128 or 64; INT8 residue products 256 or
-      // 128 where the layout leaf allows the 256 tiles; BF16 one tile
+      // leaf-GEMM block tiles: the default choice or the smaller one (FP64 64;
+      // INT8 residue products below 256 where the layout leaf is a multiple of
+      // 256); BF16 one tile
       int tiles = 1;
       if (ms.mode == CAPS_MODE_FP64) tiles = 2;
       if ((ms.mode == CAPS_MODE_CRT_INT8 || ms.mode == CAPS_MODE_OZAKI_INT8) && m0 % 256 == 0)
@@ -103,8 +104,8 @@ void candidate_features(const caps_desc &d, const caps_candidate &c, double spre
          : c.mode == CAPS_MODE_OZAKI_INT8 ? 2.f
          : c.mode == CAPS_MODE_CRT_BF16   ? 3.f
                                           : 0.f;
-  // power-of-two alignment of the layout's leaf, log2(gcd(leaf, 256)) / 8: it
-  // picks the leaf GEMM's path (256 tiles, 128 tiles, edge-checked variants)
+  // power-of-two alignment of the layout's leaf, log2(gcd(leaf, 256)) / 8: the
+  // leaf GEMM pads to tiles, checks edges and pitches rows by it
   const int leaf = d.lda >> d.nrec;
   int a = 0;
   while (a < 8 && leaf > 0 && (leaf >> a) % 2 == 0) a++;
