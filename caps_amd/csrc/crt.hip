@@ -174,13 +174,24 @@ __device__ __forceinline__ void split_a_body(const CrtMats *__restrict__ M,
   const long long plane = M->plane;
   const int tk = (m + SPLIT_K - 1) / SPLIT_K;
   const int r0 = (bx / tk) * SPLIT_R, k0 = (bx % tk) * SPLIT_K;
-  for (int idx = threadIdx.x; idx < SPLIT_R * SPLIT_K; idx += T) {
-    const int r = idx & 31, c = idx >> 5;
-    const int li = r0 + r, lj = k0 + c;
-    double v = 0.0;
-    if (li < m && lj < m)
-      v = A[PLAIN ? li + (long long)lj * m : leaf_elem_offset(m, bs, li, lj)];
-    T2[c][r ^ tswz(c)] = v;
+  // a thread's 16 elements: one row, every 8th column.  Elements outside are
+  // read at the leaf's first one and dropped, so that all loads go out before a
+  // wait (a branch around each: 13.6 against 9.3 us at n = 640, 57 against 50 at
+  // n = 3000)
+  constexpr int NV = SPLIT_R * SPLIT_K / T, DC = T / SPLIT_R;
+  const int tr = threadIdx.x % SPLIT_R, tc = threadIdx.x / SPLIT_R;
+  double v[NV];
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const int ti = r0 + tr, tj = k0 + tc + DC * i;
+    const bool in = ti < m && tj < m;
+    v[i] = A[!in ? 0 : (PLAIN ? ti + (long long)tj * m : leaf_elem_offset(m, bs, ti, tj))];
+    v[i] = in ? v[i] : 0.0;
+  }
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const int c = tc + DC * i;
+    T2[c][tr ^ tswz(c)] = v[i];
   }
   __syncthreads();
   const int r = threadIdx.x >> 3, kq = (threadIdx.x & 7) * 16;
