@@ -579,7 +579,8 @@ struct Builder {
     // leaves to row-major on the way.
     const bool top2 = items.size() == 1 && fusable(1, n, d.nrec, 0) && (d.bs == 1 || d.bs == m);
     const bool fused_b = top2 && (pad || m % 2 == 0);
-    const bool fused_a = fused_b && m % 128 == 0;
+    const bool fused_a =
+        fused_b && m % 128 == 0 && (!pad || bb_split_a_pays((long long)(n / 4) * (n / 4)));
     for (const BatchItem *it : items) {
       CrtMats M{};
       M.A = it->A;

@@ -78,6 +78,8 @@ hipError_t launch_bb_pre(const BBPre *d_P, long long q, int nmod,
 // m0: host copy of the table's leaf size; q < 2^31
 hipError_t launch_bb_split_b(const BBSplitB *d_P, long long q, int m0, int nmod,
                              const OzakiConsts *d_consts, hipStream_t s);
+// does A's fused split take less time than its split and pre-additions do?
+bool bb_split_a_pays(long long q);
 // m0 % 128 == 0 (host copy of the table's m0), q < 2^31
 hipError_t launch_bb_split_a(const BBSplitA *d_P, long long q, int m0,
                              const OzakiConsts *d_consts, hipStream_t s);
