@@ -231,9 +231,15 @@ size_t batch_limit_bytes(const State &s) {
   return s.budget_set ? (size_t)s.available_doubles * sizeof(double) : ~(size_t)0;
 }
 
-// allocate, build and upload a plan whose builder is `build(plan, work)`
+// the part of a plan's key that its batched levels depend on
+long long key_budget(const State &s, const std::string &pattern) {
+  return s.budget_set && has_recursive_level(pattern) ? s.available_doubles : 0;
+}
+
+// allocate, build and upload a plan whose builder is `build(plan, work)`;
+// optional: other plans stay, CAPS_ENOMEM where it does not fit beside them
 template <typename F>
-int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out) {
+int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out, bool optional = false) {
   evict_locked(s, MAX_PLANS - 1);
   auto plan = std::make_unique<Plan>();
   plan->key = key;
@@ -243,8 +249,10 @@ int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out) {
     size_t freeb = 0, totalb = 0;
     HIP_TRY(hipMemGetInfo(&freeb, &totalb));
     if (need > freeb) {
-      evict_locked(s, 0);
-      HIP_TRY(hipMemGetInfo(&freeb, &totalb));
+      if (!optional) {
+        evict_locked(s, 0);
+        HIP_TRY(hipMemGetInfo(&freeb, &totalb));
+      }
       if (need > freeb)
         return fail(CAPS_ENOMEM, "plan needs %.1f MiB of device workspace, %.1f MiB free",
                     need / 1048576.0, freeb / 1048576.0);
@@ -276,27 +284,32 @@ int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out) {
 int get_plan_locked(State &s, const double *A, const double *B, double *C, const caps_desc &d,
                     const std::string &pat, int mode, int moduli, int cutoff, bool fuse,
                     hipStream_t stream, int tile, Plan *&out) {
-  PlanKey key{A,  B,    C,             d,      pat,  mode, moduli, cutoff,
-              fuse, std::string(), stream, tile,
-              batch_levels(d, pat, mode, moduli, cutoff, batch_limit_bytes(s), BATCH_ANY_ALONE)};
-  for (;;) {
-    for (auto &p : s.plans)
-      if (p->key == key) {
-        out = p.get();
-        p->last_use = ++s.clock;
-        return CAPS_OK;
-      }
-    int rc = make_plan_locked(
+  PlanKey key{A,    B,      C,    d,  pat, mode, moduli, cutoff, fuse, std::string(),
+              stream, tile, key_budget(s, pat)};
+  for (auto &p : s.plans)
+    if (p->key == key) {
+      out = p.get();
+      p->last_use = ++s.clock;
+      return CAPS_OK;
+    }
+  const auto make = [&](const std::string &run) {
+    return make_plan_locked(
         s, key,
         [&](Plan &pl, void *work) {
           return build_plan(pl, A, B, C, d, pat, mode, moduli, cutoff, work, fuse, tile, true,
-                            key.run);
+                            run);
         },
-        out);
-    // no memory for more batched levels than asked for: exactly those
-    if (rc != CAPS_ENOMEM || key.run == pat) return rc;
-    key.run = pat;
+        out, run != pat);
+  };
+  // what a plan runs is decided once, when it is built: later calls find it
+  // whatever memory is free then
+  const std::string run =
+      batch_levels(d, pat, mode, moduli, cutoff, batch_limit_bytes(s), BATCH_ANY_ALONE);
+  if (run != pat) {
+    const int rc = make(run);
+    if (rc != CAPS_ENOMEM) return rc;  // no memory for it: exactly the levels asked for
   }
+  return make(pat);
 }
 
 int capture_graph(Plan &p) {
@@ -500,9 +513,7 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
   // host-only plans, one per (buffers, shape, options, device): their tables
   // hold this device's scratch addresses
   PlanKey key{dA, dB, dC, *desc, pat, mode, moduli, cutoff, fuse,
-              "scratch of device " + std::to_string(s.device), nullptr, tile,
-              batch_levels(*desc, pat, mode, moduli, cutoff, batch_limit_bytes(s),
-                           BATCH_ANY_SHARED)};
+              "scratch of device " + std::to_string(s.device), nullptr, tile, key_budget(s, pat)};
   Plan *p = nullptr;
   for (auto &hp : s.host_plans)
     if (hp->key == key) {
@@ -529,7 +540,8 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
                   need / 1048576.0, CAPS_NOALLOC_SCRATCH_MIB);
     // as run, with the residue pitch: where that does not fit, the requested
     // levels, then levels recursively from the bottom up (the same bits)
-    std::string run = key.run;
+    std::string run = batch_levels(*desc, pat, mode, moduli, cutoff, batch_limit_bytes(s),
+                                   BATCH_ANY_SHARED);
     for (size_t l = pat.size() + 1;; l--) {
       if (size_of(run, true, toff, need) != CAPS_OK)
         return fail(CAPS_EINVAL, "internal: plan layout check failed");
@@ -765,7 +777,7 @@ int caps_multiply_batch_device(int count, const double *const *dA, const double 
   const bool merge = !(opts && (opts[0].flags & CAPS_FLAG_NO_FUSION));
   const size_t merge_budget = merge ? planner_budget_bytes(s.available_doubles, s.budget_set) : 0;
   PlanKey pk{nullptr, nullptr, nullptr, descs[0], std::string(), mode, moduli, 0, merge, key,
-             stream, tile, std::string()};
+             stream, tile, 0};
   Plan *plan = nullptr;
   for (auto &p : s.plans)
     if (p->key == pk) {

@@ -37,7 +37,7 @@ bool PlanKey::operator==(const PlanKey &o) const {
   return A == o.A && B == o.B && C == o.C && memcmp(&desc, &o.desc, sizeof(desc)) == 0 &&
          pattern == o.pattern && mode == o.mode && moduli == o.moduli && cutoff == o.cutoff &&
          fuse == o.fuse && batch == o.batch && stream == o.stream && tile == o.tile &&
-         run == o.run;
+         budget == o.budget;
 }
 
 namespace {

@@ -86,7 +86,7 @@ struct PlanKey {
   std::string batch;  // batched plans: every item's pointers, descriptor and pattern
   const void *stream;
   int tile;           // leaf-GEMM block tile: 0 default, 1 the smaller one
-  std::string run;    // the pattern the plan runs (batch_levels of `pattern`)
+  long long budget;   // doubles that limited batch_levels, 0: none set or no recursive level
   bool operator==(const PlanKey &o) const;
 };
 

@@ -23,6 +23,9 @@ std::string choose_pattern(const caps_desc &d, int mode, int moduli, long long b
 // together.
 std::string batch_levels(const caps_desc &d, const std::string &pattern, int mode, int moduli,
                          int cutoff, size_t limit_bytes, size_t any_bytes, int items = 1);
+inline bool has_recursive_level(const std::string &pattern) {
+  return pattern.find_first_not_of("bB") != std::string::npos;
+}
 // any_bytes of one multiply with a workspace of its own (a 72nd of the device),
 // and of a problem that shares the device with many or a scratch array
 constexpr size_t BATCH_ANY_ALONE = (size_t)4 << 30;
