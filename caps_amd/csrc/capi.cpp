@@ -236,6 +236,14 @@ long long key_budget(const State &s, const std::string &pattern) {
   return s.budget_set && has_recursive_level(pattern) ? s.available_doubles : 0;
 }
 
+// hipMalloc whose failure the caller handles or reports: it is not left as the
+// last error, which the next launch would return
+hipError_t try_malloc(void **p, size_t bytes) {
+  const hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
 // allocate, build and upload a plan whose builder is `build(plan, work)`;
 // optional: other plans stay, CAPS_ENOMEM where it does not fit beside them
 template <typename F>
@@ -257,7 +265,7 @@ int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out, bool opt
         return fail(CAPS_ENOMEM, "plan needs %.1f MiB of device workspace, %.1f MiB free",
                     need / 1048576.0, freeb / 1048576.0);
     }
-    hipError_t e = hipMalloc(&plan->d_work, need);
+    hipError_t e = try_malloc(&plan->d_work, need);
     if (e != hipSuccess)
       return fail(CAPS_ENOMEM, "hipMalloc(%zu) for workspace: %s", need, hipGetErrorString(e));
   }
@@ -266,7 +274,7 @@ int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out, bool opt
     return fail(CAPS_EINVAL, "internal: plan layout check failed");
   }
   if (!plan->host_tables.empty()) {
-    hipError_t e = hipMalloc(&plan->d_tables, plan->host_tables.size());
+    hipError_t e = try_malloc(&plan->d_tables, plan->host_tables.size());
     if (e == hipSuccess)
       e = hipMemcpy(plan->d_tables, plan->host_tables.data(), plan->host_tables.size(),
                     hipMemcpyHostToDevice);
@@ -307,7 +315,7 @@ int get_plan_locked(State &s, const double *A, const double *B, double *C, const
       batch_levels(d, pat, mode, moduli, cutoff, batch_limit_bytes(s), BATCH_ANY_ALONE);
   if (run != pat) {
     const int rc = make(run);
-    if (rc != CAPS_ENOMEM) return rc;  // no memory for it: exactly the levels asked for
+    if (rc == CAPS_OK) return rc;  // else exactly the levels asked for
   }
   return make(pat);
 }
@@ -431,7 +439,7 @@ int stage_locked(State &s, size_t elems) {
     }
   s.stage_elems = 0;
   for (auto &p : s.stage) {
-    hipError_t e = hipMalloc(&p, elems * sizeof(double));
+    hipError_t e = try_malloc((void **)&p, elems * sizeof(double));
     if (e != hipSuccess) return fail(CAPS_ENOMEM, "staging hipMalloc: %s", hipGetErrorString(e));
   }
   if (!s.stage_stream) HIP_TRY(hipStreamCreateWithFlags(&s.stage_stream, hipStreamNonBlocking));

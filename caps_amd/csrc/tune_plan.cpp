@@ -222,8 +222,10 @@ int caps_autotune(const double *dA, const double *dB, double *dC, const caps_des
   if (cands.empty()) return set_error(CAPS_EUNSUPPORTED, "caps_autotune: no candidate");
   const size_t n2 = (size_t)desc->lda * desc->lda;
   double *ref = nullptr;
-  if (hipMalloc(&ref, n2 * sizeof(double)) != hipSuccess)
+  if (hipMalloc(&ref, n2 * sizeof(double)) != hipSuccess) {
+    (void)hipGetLastError();  // not the next launch's error
     return set_error(CAPS_ENOMEM, "caps_autotune: reference buffer");
+  }
   rc = caps_reference_product(dA, dB, ref, desc, stream);
   int found = -1;
   int measured = 0;

@@ -18,3 +18,28 @@ for _ in range(3):
     assert call(1024, 2, "bb", at=2) == 0 and call(1024, 1, "d", at=3) == 0
 assert (count("malloc"), count("free"), count("device_sync")) == before
 """)
+
+
+def test_failed_allocation_leaves_no_error():
+    """A workspace that hipMalloc refuses, whatever hipMemGetInfo said, is
+    replaced by the requested levels' one; the refusal is not the next launch's
+    error, nor the next call's after CAPS_ENOMEM."""
+    run("""
+fake.fake_set_malloc_limit(1 * GiB)  # batched: 1.9 GiB
+assert call(4096, 3, "ddd") == 0, error()
+assert peak_bytes() < 100 * MiB
+assert call(8192, 2, "bb", at=2) == 3  # CAPS_ENOMEM
+assert call(1024, 2, "bb", at=3) == 0, error()
+import numpy as np
+fake.fake_set_malloc_limit(8 * MiB)
+a = np.zeros(1536 * 1536)
+d = caps_amd.MatDescriptor.one_device(1536, 2, 1)
+p = a.ctypes.data
+assert lib.caps_multiply(p, p, p, ctypes.byref(d), None, None) == 3  # its staging
+fake.fake_set_malloc_limit(1 * GiB)
+assert call(512, 2, "bb", at=4) == 0, error()
+fake.fake_set_malloc_limit(8)  # tables alone (no level, no workspace)
+assert call(256, 0, None, at=5) != 0
+fake.fake_set_malloc_limit(1 * GiB)
+assert call(256, 2, "bb", at=6) == 0, error()
+""")
