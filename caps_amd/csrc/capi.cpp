@@ -744,13 +744,11 @@ int caps_multiply_batch_device(int count, const double *const *dA, const double 
     }
   }
   std::vector<BatchItem> items((size_t)count);
-  // items of one group are batched together: each NULL-pattern item gets an
-  // equal share of the budget
-  const long long share =
-      (long long)(planner_budget_bytes(s.available_doubles, s.budget_set) / sizeof(double)) /
-      count;
+  // the key has the patterns as asked for (* for NULL): the plan is found again
+  // whatever memory is free then
   std::string key;
   key.reserve((size_t)count * 64);
+  long long budget = 0;
   for (int i = 0; i < count; i++) {
     rc = check_desc(&descs[i]);
     if (rc) return rc;
@@ -765,27 +763,25 @@ int caps_multiply_batch_device(int count, const double *const *dA, const double 
     items[i].C = dC[i];
     items[i].desc = descs[i];
     items[i].cutoff = cutoff;
-    caps_opts o{mode, moduli, 0, cutoff};
-    rc = resolve_pattern(descs[i], patterns ? patterns[i] : nullptr, &o, items[i].pattern, mode,
-                         moduli, share > 0 ? share : 1, true);
-    if (rc) return rc;
-    // recursive levels run batched within the item's share of the budget (the
-    // key holds the pattern as run)
-    items[i].pattern = batch_levels(descs[i], items[i].pattern, mode, moduli, cutoff,
-                                    (size_t)share * sizeof(double), BATCH_ANY_SHARED, count);
+    std::string pat = "*";
+    if (patterns && patterns[i]) {
+      rc = resolve_pattern(descs[i], patterns[i], nullptr, pat, mode, moduli, 0, false);
+      if (rc) return rc;
+    }
+    items[i].pattern = pat;
+    if (key_budget(s, pat)) budget = s.available_doubles;
     char buf[176];
     snprintf(buf, sizeof(buf), "%p %p %p %d %d %d %d %s;", (const void *)dA[i],
              (const void *)dB[i], (void *)dC[i], descs[i].lda, descs[i].nrec, descs[i].bs, cutoff,
-             items[i].pattern.c_str());
+             pat.c_str());
     key += buf;
   }
   const int tile = (opts && (opts[0].flags & CAPS_FLAG_SMALL_TILE)) ? 1 : 0;
   // merged groups (segmented launches) unless CAPS_FLAG_NO_FUSION, within the
   // memory budget
   const bool merge = !(opts && (opts[0].flags & CAPS_FLAG_NO_FUSION));
-  const size_t merge_budget = merge ? planner_budget_bytes(s.available_doubles, s.budget_set) : 0;
   PlanKey pk{nullptr, nullptr, nullptr, descs[0], std::string(), mode, moduli, 0, merge, key,
-             stream, tile, 0};
+             stream, tile, budget};
   Plan *plan = nullptr;
   for (auto &p : s.plans)
     if (p->key == pk) {
@@ -793,12 +789,30 @@ int caps_multiply_batch_device(int count, const double *const *dA, const double 
       p->last_use = ++s.clock;
     }
   if (!plan) {
-    rc = make_plan_locked(
-        s, pk,
-        [&](Plan &pl, void *work) {
-          return build_batch_plan(pl, items, mode, moduli, work, tile, merge_budget);
-        },
-        plan);
+    const size_t budget_bytes = planner_budget_bytes(s.available_doubles, s.budget_set);
+    // items of one group are batched together: each gets an equal share of the
+    // budget, for its NULL pattern and for recursive levels that run batched
+    const long long share = std::max(1LL, (long long)(budget_bytes / sizeof(double)) / count);
+    std::vector<BatchItem> run = items;
+    bool wider = false;
+    for (int i = 0; i < count; i++) {
+      BatchItem &it = items[(size_t)i];
+      if (it.pattern == "*") it.pattern = choose_pattern(it.desc, mode, moduli, share, true);
+      run[(size_t)i].pattern =
+          batch_levels(it.desc, it.pattern, mode, moduli, it.cutoff,
+                       (size_t)share * sizeof(double), BATCH_ANY_SHARED, count);
+      wider = wider || run[(size_t)i].pattern != it.pattern;
+    }
+    const auto make = [&](const std::vector<BatchItem> &b, bool optional) {
+      return make_plan_locked(
+          s, pk,
+          [&](Plan &pl, void *work) {
+            return build_batch_plan(pl, b, mode, moduli, work, tile, merge ? budget_bytes : 0);
+          },
+          plan, optional);
+    };
+    rc = wider ? make(run, true) : CAPS_ENOMEM;
+    if (rc) rc = make(items, false);  // exactly the levels asked for
     if (rc) return rc;
   }
   const bool use_graph = by_graph(*plan, opts);

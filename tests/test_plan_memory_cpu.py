@@ -43,3 +43,25 @@ assert call(256, 0, None, at=5) != 0
 fake.fake_set_malloc_limit(1 * GiB)
 assert call(256, 2, "bb", at=6) == 0, error()
 """)
+
+
+def test_batch_plan_is_found_whatever_is_free():
+    """The identical batched call finds its plan though the plan's own workspace,
+    or another allocator, changed what is free."""
+    run("""
+for at, shapes, mode in ((1, [(2048, 2, "dd")] * 512, CRT), (2, [(1024, 2, None)] * 16, FP64),
+                         (3, [(1024, 2, "bd"), (640, 1, None), (768, 1, "d")], FP64)):
+    fake.fake_set_free(280 * GiB)
+    assert batch(shapes, mode, at) == 0, error()
+    before = count("malloc"), count("free")
+    for left in (None, 200 * MiB, 0):
+        if left is not None:
+            fake.fake_set_free(left)
+        assert batch(shapes, mode, at) == 0, error()
+        assert (count("malloc"), count("free")) == before, (at, left)
+fake.fake_set_free(280 * GiB)
+assert batch([(1024, 2, "dd")] * 4, at=4) == 0
+wide = peak_bytes()
+caps_amd.set_available_memory(1)  # a budget gives the recursive plan
+assert batch([(1024, 2, "dd")] * 4, at=4) == 0 and peak_bytes() < wide
+""")
