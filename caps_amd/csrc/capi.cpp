@@ -226,9 +226,11 @@ int check_cutoff(const caps_desc &d, int mode, int cutoff) {
   return CAPS_OK;
 }
 
-// the workspace limit of batch_levels: the caller's budget when one is set
-size_t batch_limit_bytes(const State &s) {
-  return s.budget_set ? (size_t)s.available_doubles * sizeof(double) : ~(size_t)0;
+// what cached plans leave of BATCH_ANY_PLANS
+size_t extra_left(const State &s) {
+  size_t used = 0;
+  for (const auto &p : s.plans) used += p->batched_extra;
+  return used < BATCH_ANY_PLANS ? BATCH_ANY_PLANS - used : 0;
 }
 
 // the part of a plan's key that its batched levels depend on
@@ -245,19 +247,21 @@ hipError_t try_malloc(void **p, size_t bytes) {
 }
 
 // allocate, build and upload a plan whose builder is `build(plan, work)`;
-// optional: other plans stay, CAPS_ENOMEM where it does not fit beside them
+// extra != 0: a plan wider than asked for by so many bytes, with which other
+// plans stay (CAPS_ENOMEM where it does not fit beside them)
 template <typename F>
-int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out, bool optional = false) {
+int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out, size_t extra = 0) {
   evict_locked(s, MAX_PLANS - 1);
   auto plan = std::make_unique<Plan>();
   plan->key = key;
+  plan->batched_extra = extra;
   if (build(*plan, nullptr) != CAPS_OK) return fail(CAPS_EINVAL, "internal: plan layout check failed");
   const size_t need = plan->work_bytes;
   if (need) {
     size_t freeb = 0, totalb = 0;
     HIP_TRY(hipMemGetInfo(&freeb, &totalb));
     if (need > freeb) {
-      if (!optional) {
+      if (extra == 0) {
         evict_locked(s, 0);
         HIP_TRY(hipMemGetInfo(&freeb, &totalb));
       }
@@ -307,12 +311,16 @@ int get_plan_locked(State &s, const double *A, const double *B, double *C, const
           return build_plan(pl, A, B, C, d, pat, mode, moduli, cutoff, work, fuse, tile, true,
                             run);
         },
-        out, run != pat);
+        out, batched_extra(d, pat, run, mode, moduli, cutoff));
   };
   // what a plan runs is decided once, when it is built: later calls find it
   // whatever memory is free then
   const std::string run =
-      batch_levels(d, pat, mode, moduli, cutoff, batch_limit_bytes(s), BATCH_ANY_ALONE);
+      has_recursive_level(pat)
+          ? batch_levels(d, pat, mode, moduli, cutoff,
+                         planner_budget_bytes(s.available_doubles, s.budget_set), BATCH_ANY_ALONE,
+                         extra_left(s))
+          : pat;
   if (run != pat) {
     const int rc = make(run);
     if (rc == CAPS_OK) return rc;  // else exactly the levels asked for
@@ -548,8 +556,10 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
                   need / 1048576.0, CAPS_NOALLOC_SCRATCH_MIB);
     // as run, with the residue pitch: where that does not fit, the requested
     // levels, then levels recursively from the bottom up (the same bits)
-    std::string run = batch_levels(*desc, pat, mode, moduli, cutoff, batch_limit_bytes(s),
-                                   BATCH_ANY_SHARED);
+    const size_t limit =
+        s.budget_set ? (size_t)s.available_doubles * sizeof(double) : ~(size_t)0;
+    std::string run =
+        batch_levels(*desc, pat, mode, moduli, cutoff, limit, BATCH_ANY_SHARED, ~(size_t)0);
     for (size_t l = pat.size() + 1;; l--) {
       if (size_of(run, true, toff, need) != CAPS_OK)
         return fail(CAPS_EINVAL, "internal: plan layout check failed");
@@ -794,25 +804,26 @@ int caps_multiply_batch_device(int count, const double *const *dA, const double 
     // budget, for its NULL pattern and for recursive levels that run batched
     const long long share = std::max(1LL, (long long)(budget_bytes / sizeof(double)) / count);
     std::vector<BatchItem> run = items;
-    bool wider = false;
+    size_t extra = 0;
     for (int i = 0; i < count; i++) {
       BatchItem &it = items[(size_t)i];
       if (it.pattern == "*") it.pattern = choose_pattern(it.desc, mode, moduli, share, true);
       run[(size_t)i].pattern =
           batch_levels(it.desc, it.pattern, mode, moduli, it.cutoff,
-                       (size_t)share * sizeof(double), BATCH_ANY_SHARED, count);
-      wider = wider || run[(size_t)i].pattern != it.pattern;
+                       (size_t)share * sizeof(double), BATCH_ANY_SHARED,
+                       extra_left(s) / (size_t)count, count);
+      extra += batched_extra(it.desc, it.pattern, run[(size_t)i].pattern, mode, moduli, it.cutoff);
     }
-    const auto make = [&](const std::vector<BatchItem> &b, bool optional) {
+    const auto make = [&](const std::vector<BatchItem> &b, size_t more) {
       return make_plan_locked(
           s, pk,
           [&](Plan &pl, void *work) {
             return build_batch_plan(pl, b, mode, moduli, work, tile, merge ? budget_bytes : 0);
           },
-          plan, optional);
+          plan, more);
     };
-    rc = wider ? make(run, true) : CAPS_ENOMEM;
-    if (rc) rc = make(items, false);  // exactly the levels asked for
+    rc = extra ? make(run, extra) : CAPS_ENOMEM;
+    if (rc) rc = make(items, 0);  // exactly the levels asked for
     if (rc) return rc;
   }
   const bool use_graph = by_graph(*plan, opts);

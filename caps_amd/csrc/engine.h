@@ -97,6 +97,7 @@ struct Plan {
   void *d_tables = nullptr;
   void *d_work = nullptr;
   size_t work_bytes = 0;
+  size_t batched_extra = 0;  // of it, for recursive levels that run batched
   hipGraphExec_t graph = nullptr;
   hipStream_t capture_stream = nullptr;
   long long additions = 0, multiplications = 0, leaves = 0;

@@ -77,13 +77,15 @@ double workspace_estimate(const caps_desc &d, const std::string &pattern, int mo
 // ms with its two lower levels batched, 1.78 with all three (2 GB); n = 392
 // 'bdd' 563 and 47 us.
 std::string batch_levels(const caps_desc &d, const std::string &pattern, int mode, int moduli,
-                         int cutoff, size_t limit_bytes, size_t any_bytes, int items) {
+                         int cutoff, size_t limit_bytes, size_t any_bytes, size_t extra_bytes,
+                         int items) {
   std::string run = pattern;
   // a launch takes at most 65,535 leaves of the leaf-only split (grid.y)
   double batch = items;
   for (int l = 0; l < d.nrec - cutoff; l++)
     if (pattern[(size_t)l] == 'b' || pattern[(size_t)l] == 'B') batch *= 7;
-  const double extra = std::max(24.0 * d.lda * d.lda, (double)any_bytes);
+  const double extra =
+      std::min(std::max(24.0 * d.lda * d.lda, (double)any_bytes), (double)extra_bytes);
   const double limit = std::min(workspace_estimate(d, pattern, mode, moduli, cutoff) + extra,
                                 (double)limit_bytes);
   for (int l = d.nrec - cutoff - 1; l >= 0; l--) {
@@ -95,6 +97,12 @@ std::string batch_levels(const caps_desc &d, const std::string &pattern, int mod
     batch *= 7;
   }
   return run;
+}
+
+size_t batched_extra(const caps_desc &d, const std::string &pattern, const std::string &run,
+                     int mode, int moduli, int cutoff) {
+  return (size_t)(workspace_estimate(d, run, mode, moduli, cutoff) -
+                  workspace_estimate(d, pattern, mode, moduli, cutoff));
 }
 
 int choose_mode(const caps_desc &) { return CAPS_MODE_FP64; }

@@ -18,11 +18,16 @@ std::string choose_pattern(const caps_desc &d, int mode, int moduli, long long b
 
 // The pattern a plan runs for the requested one: recursive levels run batched,
 // the deepest first, while they add at most the operands' own bytes (or
-// any_bytes) to the requested pattern's workspace, within limit_bytes.  The
-// results do not depend on it.  items: problems of the same shape planned
-// together.
+// any_bytes) to the requested pattern's workspace, but not more than
+// extra_bytes, within limit_bytes.  The results do not depend on it.  items:
+// problems of the same shape planned together.
 std::string batch_levels(const caps_desc &d, const std::string &pattern, int mode, int moduli,
-                         int cutoff, size_t limit_bytes, size_t any_bytes, int items = 1);
+                         int cutoff, size_t limit_bytes, size_t any_bytes, size_t extra_bytes,
+                         int items = 1);
+// the workspace that running `run` adds to the requested pattern's, as
+// batch_levels estimates it
+size_t batched_extra(const caps_desc &d, const std::string &pattern, const std::string &run,
+                     int mode, int moduli, int cutoff);
 inline bool has_recursive_level(const std::string &pattern) {
   return pattern.find_first_not_of("bB") != std::string::npos;
 }
@@ -30,6 +35,10 @@ inline bool has_recursive_level(const std::string &pattern) {
 // and of a problem that shares the device with many or a scratch array
 constexpr size_t BATCH_ANY_ALONE = (size_t)4 << 30;
 constexpr size_t BATCH_ANY_SHARED = (size_t)64 << 20;
+// what all cached plans together may add (a ninth of the device): 24 plans kept,
+// each with 4 GiB, would hold a third of it for callers who asked for the
+// smallest workspace
+constexpr size_t BATCH_ANY_PLANS = (size_t)32 << 30;
 
 // Leaf arithmetic when the caller asks for CAPS_MODE_AUTO.
 int choose_mode(const caps_desc &d);

@@ -130,8 +130,11 @@ long long caps_num_entries(const caps_desc *desc);
  * level from [bBdDhH] ('b' = batched level, 'd'/'h' = recursive level), or
  * NULL for the planner's choice.  A recursive level whose batched form adds at
  * most the operands' own size (or 4 GiB; in a batch or the scratch array 64
- * MiB) of workspace, within a budget set by caps_set_available_memory, runs
- * batched: the same bits, reported as requested.  opts may be NULL (FP64 mode).
+ * MiB) of workspace, within a budget set by caps_set_available_memory or, with
+ * none, half of the free device memory, runs batched: the same bits, reported as
+ * requested.  All cached plans together add at most 32 GiB so, and what a plan
+ * runs is decided when it is built.  A small budget keeps every level recursive.
+ * opts may be NULL (FP64 mode).
  * multiply.h:13 / multiply.cpp:9-25. */
 int caps_multiply(const double *A, const double *B, double *C,
                   const caps_desc *desc, const char *pattern,

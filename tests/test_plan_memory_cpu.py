@@ -9,7 +9,7 @@ def test_low_memory_keeps_the_cache():
     requested levels is built once and found again, and no other plan goes."""
     run("""
 assert call(1024, 2, "bb", at=2) == 0 and call(1024, 1, "d", at=3) == 0
-fake.fake_set_free(1 * GiB)  # batched: 1.9 GiB
+fake.fake_set_free(150 * MiB)  # batched: 1.9 GiB, as asked for 84 MiB
 assert call(4096, 3, "ddd") == 0, error()
 assert peak_bytes() < 100 * MiB and reported() == "DFS,DFS,DFS,"
 before = count("malloc"), count("free"), count("device_sync")
@@ -64,4 +64,29 @@ assert batch([(1024, 2, "dd")] * 4, at=4) == 0
 wide = peak_bytes()
 caps_amd.set_available_memory(1)  # a budget gives the recursive plan
 assert batch([(1024, 2, "dd")] * 4, at=4) == 0 and peak_bytes() < wide
+""")
+
+
+def test_recursive_levels_leave_memory_free():
+    """Without a budget the batched form of recursive levels takes at most half
+    of the free memory, and all plans' together 32 GiB more than the levels
+    asked for would."""
+    run("""
+fake.fake_set_free(3 * GiB)
+assert call(4096, 3, "ddd") == 0, error()
+assert fake.fake_free() >= 3 * GiB // 2
+caps_amd.release()
+fake.fake_set_free(256 * GiB)
+caps_amd.set_available_memory(1)
+assert call(4096, 3, "ddd") == 0, error()
+asked = 256 * GiB - fake.fake_free()
+caps_amd.release()
+caps_amd.set_available_memory(0)
+assert fake.fake_free() == 256 * GiB
+extra = []
+for at in range(1, 25):
+    assert call(4096, 3, "ddd", at=at) == 0, error()
+    extra.append(256 * GiB - fake.fake_free() - at * asked)
+assert max(extra) <= 32 * GiB and extra[0] > 1 * GiB, extra
+assert extra[4] > 4.9 * extra[0]  # the first plans have all of theirs
 """)
