@@ -247,16 +247,20 @@ hipError_t try_malloc(void **p, size_t bytes) {
 }
 
 // allocate, build and upload a plan whose builder is `build(plan, work)`;
-// extra != 0: a plan wider than asked for by so many bytes, with which other
-// plans stay (CAPS_ENOMEM where it does not fit beside them)
+// extra != 0: a plan wider than asked for by so many bytes, for which other
+// plans stay (CAPS_ENOMEM where it does not fit beside them or within `limit`)
 template <typename F>
-int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out, size_t extra = 0) {
+int make_plan_locked(State &s, const PlanKey &key, F build, Plan *&out, size_t extra = 0,
+                     size_t limit = 0) {
   evict_locked(s, MAX_PLANS - 1);
   auto plan = std::make_unique<Plan>();
   plan->key = key;
   plan->batched_extra = extra;
   if (build(*plan, nullptr) != CAPS_OK) return fail(CAPS_EINVAL, "internal: plan layout check failed");
   const size_t need = plan->work_bytes;
+  if (extra != 0 && need > limit)
+    return fail(CAPS_ENOMEM, "plan needs %.1f MiB of device workspace, limit %.1f MiB",
+                need / 1048576.0, limit / 1048576.0);
   if (need) {
     size_t freeb = 0, totalb = 0;
     HIP_TRY(hipMemGetInfo(&freeb, &totalb));
@@ -304,6 +308,7 @@ int get_plan_locked(State &s, const double *A, const double *B, double *C, const
       p->last_use = ++s.clock;
       return CAPS_OK;
     }
+  const size_t limit = planner_budget_bytes(s.available_doubles, s.budget_set);
   const auto make = [&](const std::string &run) {
     return make_plan_locked(
         s, key,
@@ -311,20 +316,14 @@ int get_plan_locked(State &s, const double *A, const double *B, double *C, const
           return build_plan(pl, A, B, C, d, pat, mode, moduli, cutoff, work, fuse, tile, true,
                             run);
         },
-        out, batched_extra(d, pat, run, mode, moduli, cutoff));
+        out, batched_extra(d, pat, run, mode, moduli, cutoff), limit);
   };
   // what a plan runs is decided once, when it is built: later calls find it
   // whatever memory is free then
-  const std::string run =
-      has_recursive_level(pat)
-          ? batch_levels(d, pat, mode, moduli, cutoff,
-                         planner_budget_bytes(s.available_doubles, s.budget_set), BATCH_ANY_ALONE,
-                         extra_left(s))
-          : pat;
-  if (run != pat) {
-    const int rc = make(run);
-    if (rc == CAPS_OK) return rc;  // else exactly the levels asked for
-  }
+  for (std::string run =
+           batch_levels(d, pat, mode, moduli, cutoff, limit, BATCH_ANY_ALONE, extra_left(s));
+       run != pat; run = drop_batched_level(pat, run))
+    if (make(run) == CAPS_OK) return CAPS_OK;
   return make(pat);
 }
 
@@ -554,22 +553,23 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
                   "plan needs %.1f MiB of tables and workspace; caps_multiply_device_noalloc "
                   "has %d MiB of scratch",
                   need / 1048576.0, CAPS_NOALLOC_SCRATCH_MIB);
-    // as run, with the residue pitch: where that does not fit, the requested
-    // levels, then levels recursively from the bottom up (the same bits)
+    // as run, with the residue pitch: where that does not fit, fewer levels
+    // batched, then levels recursively from the bottom up (the same bits)
     const size_t limit =
         s.budget_set ? (size_t)s.available_doubles * sizeof(double) : ~(size_t)0;
     std::string run =
         batch_levels(*desc, pat, mode, moduli, cutoff, limit, BATCH_ANY_SHARED, ~(size_t)0);
-    for (size_t l = pat.size() + 1;; l--) {
+    for (size_t l = pat.size();;) {
       if (size_of(run, true, toff, need) != CAPS_OK)
         return fail(CAPS_EINVAL, "internal: plan layout check failed");
-      if (need <= SCRATCH_BYTES) break;
-      if (l == 0)
+      const bool wider = l == pat.size() && run != pat;
+      if (need <= SCRATCH_BYTES && !(wider && plan->work_bytes > limit)) break;
+      if (wider)
+        run = drop_batched_level(pat, run);
+      else if (l == 0)
         return fail(CAPS_ENOMEM, "plan needs %.1f MiB of padded workspace", need / 1048576.0);
-      if (l > pat.size())
-        run = pat;
       else
-        run[l - 1] = 'd';
+        run[--l] = 'd';
     }
     if (build_plan(*plan, dA, dB, dC, *desc, pat, mode, moduli, cutoff, base + toff, fuse, tile,
                    true, run) != CAPS_OK ||
@@ -820,7 +820,7 @@ int caps_multiply_batch_device(int count, const double *const *dA, const double 
           [&](Plan &pl, void *work) {
             return build_batch_plan(pl, b, mode, moduli, work, tile, merge ? budget_bytes : 0);
           },
-          plan, more);
+          plan, more, budget_bytes);
     };
     rc = extra ? make(run, extra) : CAPS_ENOMEM;
     if (rc) rc = make(items, 0);  // exactly the levels asked for

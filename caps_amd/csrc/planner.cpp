@@ -99,6 +99,16 @@ std::string batch_levels(const caps_desc &d, const std::string &pattern, int mod
   return run;
 }
 
+std::string drop_batched_level(const std::string &pattern, const std::string &run) {
+  std::string r = run;  // the last one that batch_levels took: the outermost
+  for (size_t l = 0; l < r.size(); l++)
+    if (r[l] != pattern[l]) {
+      r[l] = pattern[l];
+      break;
+    }
+  return r;
+}
+
 size_t batched_extra(const caps_desc &d, const std::string &pattern, const std::string &run,
                      int mode, int moduli, int cutoff) {
   return (size_t)(workspace_estimate(d, run, mode, moduli, cutoff) -

@@ -20,10 +20,13 @@ std::string choose_pattern(const caps_desc &d, int mode, int moduli, long long b
 // the deepest first, while they add at most the operands' own bytes (or
 // any_bytes) to the requested pattern's workspace, but not more than
 // extra_bytes, within limit_bytes.  The results do not depend on it.  items:
-// problems of the same shape planned together.
+// problems of the same shape planned together.  An estimate (partials, exponents
+// and alignment come on top): a plan that turns out larger than its limit is
+// built again with drop_batched_level, one level less.
 std::string batch_levels(const caps_desc &d, const std::string &pattern, int mode, int moduli,
                          int cutoff, size_t limit_bytes, size_t any_bytes, size_t extra_bytes,
                          int items = 1);
+std::string drop_batched_level(const std::string &pattern, const std::string &run);
 // the workspace that running `run` adds to the requested pattern's, as
 // batch_levels estimates it
 size_t batched_extra(const caps_desc &d, const std::string &pattern, const std::string &run,

@@ -22,12 +22,12 @@ assert (count("malloc"), count("free"), count("device_sync")) == before
 
 def test_failed_allocation_leaves_no_error():
     """A workspace that hipMalloc refuses, whatever hipMemGetInfo said, is
-    replaced by the requested levels' one; the refusal is not the next launch's
+    replaced by a smaller one; the refusal is not the next launch's
     error, nor the next call's after CAPS_ENOMEM."""
     run("""
 fake.fake_set_malloc_limit(1 * GiB)  # batched: 1.9 GiB
 assert call(4096, 3, "ddd") == 0, error()
-assert peak_bytes() < 100 * MiB
+assert peak_bytes() < 1 * GiB
 assert call(8192, 2, "bb", at=2) == 3  # CAPS_ENOMEM
 assert call(1024, 2, "bb", at=3) == 0, error()
 import numpy as np
@@ -89,4 +89,36 @@ for at in range(1, 25):
     extra.append(256 * GiB - fake.fake_free() - at * asked)
 assert max(extra) <= 32 * GiB and extra[0] > 1 * GiB, extra
 assert extra[4] > 4.9 * extra[0]  # the first plans have all of theirs
+""")
+
+
+def test_batched_levels_keep_within_a_budget():
+    """A plan is never larger than the caller's budget where the levels asked
+    for fit it, whatever else a level needs (partials, exponents, alignment)."""
+    run("""
+for n, r, pattern, mode in ((512, 5, "ddddd", LEAF), (256, 5, "ddddd", CRT), (392, 3, "ddd", FP64),
+                            (544, 5, "ddddd", CRT), (272, 4, "dddd", LEAF), (1000, 3, "dbd", CRT)):
+    def peak(budget, at, entry=None):
+        caps_amd.set_available_memory(budget)
+        assert call(n, r, pattern, mode, at=at, entry=entry) == 0, error()
+        return peak_bytes()
+    for entry in (None, lib.caps_multiply_device_noalloc):
+        lo, hi = peak(1, 1, entry), peak(1 << 36, 2, entry)
+        assert lo < hi
+        for k in range(20):
+            budget = int(lo * (1.02 * hi / lo) ** (k / 19) / 8) + 1
+            assert peak(budget, 3 + k, entry) <= 8 * budget, (n, r, mode, budget)
+        caps_amd.release()
+for count_, n, r in ((3, 256, 4), (8, 544, 5)):
+    shapes = [(n, r, "d" * r)] * count_
+    def peak(budget, at):
+        caps_amd.set_available_memory(budget)
+        assert batch(shapes, CRT, at) == 0, error()
+        return peak_bytes()
+    lo, hi = peak(1, 1), peak(1 << 36, 2)
+    assert lo < hi
+    for k in range(20):
+        budget = int(lo * (1.02 * hi / lo) ** (k / 19) / 8) + 1
+        assert peak(budget, 3 + k) <= 8 * budget, (n, r, budget)
+    caps_amd.release()
 """)
