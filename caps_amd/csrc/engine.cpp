@@ -252,7 +252,7 @@ struct Builder {
   void ozaki_leaf_steps(const std::vector<Prob> &work, int m) {
     const int nmod = moduli;
     const size_t nb = work.size();
-    const size_t plane = (size_t)residue_area(m);  // bytes per INT8 plane
+    const size_t plane = pad ? (size_t)residue_area(m) : (size_t)m * m;  // bytes per INT8 plane
     ensure_consts();
     const size_t ex_bytes = (size_t)m * sizeof(int);
     const size_t pa_bytes = (size_t)OZ_CHUNKS * m * 2 * sizeof(double);
