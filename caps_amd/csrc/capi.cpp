@@ -31,10 +31,12 @@
 //
 // CAPS_NOALLOC_SCRATCH_MIB limits a plan's tables and workspace counted
 // without the padding of residue leaves to a 16-byte pitch.  A plan that passes
-// and does not fit with it runs fewer levels batched; recursive at every level,
-// the largest padded plan is 344 MiB (order 2176, 6 levels, 13 moduli).  Module
-// load clears the array (0.38 ms per MiB), so it is no larger than that needs.
-constexpr size_t SCRATCH_BYTES = (size_t)(CAPS_NOALLOC_SCRATCH_MIB + 96) << 20;
+// and does not fit with it gets its tables in parts, each copied before its
+// steps, or runs fewer levels batched.  Recursive at every level, the largest
+// padded workspace is 331.5 MiB (order 2176, 6 levels, 14 moduli), and no table
+// is larger than a few KB.  Module load clears the array (0.38 ms per MiB), so it
+// is no larger than that needs.
+constexpr size_t SCRATCH_BYTES = (size_t)(CAPS_NOALLOC_SCRATCH_MIB + 80) << 20;
 static __device__ __align__(256) char scratch[SCRATCH_BYTES];
 
 namespace caps {
@@ -554,7 +556,14 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
                   "has %d MiB of scratch",
                   need / 1048576.0, CAPS_NOALLOC_SCRATCH_MIB);
     // as run, with the residue pitch: where that does not fit, fewer levels
-    // batched, then levels recursively from the bottom up (the same bits)
+    // batched, the tables in parts, then levels recursively from the bottom up
+    // (the same bits)
+    auto parts_fit = [&] {
+      if (plan->work_bytes >= SCRATCH_BYTES) return false;
+      toff = SCRATCH_BYTES - plan->work_bytes;
+      return split_tables(*plan, toff);
+    };
+    bool whole = true;
     const size_t limit =
         s.budget_set ? (size_t)s.available_doubles * sizeof(double) : ~(size_t)0;
     std::string run =
@@ -563,7 +572,8 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
       if (size_of(run, true, toff, need) != CAPS_OK)
         return fail(CAPS_EINVAL, "internal: plan layout check failed");
       const bool wider = l == pat.size() && run != pat;
-      if (need <= SCRATCH_BYTES && !(wider && plan->work_bytes > limit)) break;
+      whole = need <= SCRATCH_BYTES;
+      if (wider ? whole && plan->work_bytes <= limit : whole || parts_fit()) break;
       if (wider)
         run = drop_batched_level(pat, run);
       else if (l == 0)
@@ -573,8 +583,10 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
     }
     if (build_plan(*plan, dA, dB, dC, *desc, pat, mode, moduli, cutoff, base + toff, fuse, tile,
                    true, run) != CAPS_OK ||
-        (plan->host_tables.size() + 255) / 256 * 256 != toff)
+        toff + plan->work_bytes > SCRATCH_BYTES || (!whole && !split_tables(*plan, toff)) ||
+        (whole && plan->host_tables.size() > toff))
       return fail(CAPS_EINVAL, "internal: plan layout check failed");
+    if (whole) plan->parts = {{0, 0, plan->host_tables.size()}};
     plan->d_tables = base;
     plan->d_work = base + toff;
     plan->last_use = ++s.clock;
@@ -591,11 +603,15 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
     s.host_plans.push_back(std::move(plan));
   }
   // the tables go to the front of the scratch in stream order (a pageable
-  // source is read before the call returns), then the steps run eagerly
-  HIP_TRY(hipMemcpyAsync(base, p->host_tables.data(), p->host_tables.size(),
-                         hipMemcpyHostToDevice, hs));
-  hipError_t e = run_steps(*p, hs);
-  if (e != hipSuccess) return fail(CAPS_EHIP, "kernel launch: %s", hipGetErrorString(e));
+  // source is read before the call returns), then their steps run eagerly
+  for (size_t i = 0; i < p->parts.size(); i++) {
+    const TablePart &t = p->parts[i];
+    HIP_TRY(hipMemcpyAsync(base, p->host_tables.data() + t.offset, t.bytes,
+                           hipMemcpyHostToDevice, hs));
+    hipError_t e = run_steps(*p, hs, t.first_step,
+                             i + 1 < p->parts.size() ? p->parts[i + 1].first_step : ~(size_t)0);
+    if (e != hipSuccess) return fail(CAPS_EHIP, "kernel launch: %s", hipGetErrorString(e));
+  }
   s.additions += p->additions;
   s.multiplications += p->multiplications;
   s.leaves += p->leaves;

@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <map>
 
 #include "crt.h"
 #include "fused2.h"
@@ -746,6 +747,7 @@ int build_plan(Plan &plan, const double *A, const double *B, double *C, const ca
   plan.exec_pattern.clear();
   plan.oz_moduli = 0;
   plan.crt_host.clear();
+  plan.parts.clear();
   Builder b{plan, reinterpret_cast<char *>(work_base)};
   b.leaf_bs = d.bs;
   b.mode = mode;
@@ -1066,9 +1068,71 @@ size_t plan_workspace_bytes(const caps_desc &d, const std::string &pattern, int 
   return p.work_bytes;
 }
 
-hipError_t run_steps(const Plan &plan, hipStream_t s) {
-  for (const Step &st : plan.steps) {
-    hipError_t e = run_one(plan, st, s);
+size_t step_table_bytes(const Step &st) {
+  const size_t n = (size_t)st.count;
+  switch (st.kind) {
+    case STEP_EW: return n * sizeof(EwPtrs);
+    case STEP_REW: return n * sizeof(RPtrs);
+    case STEP_GEMM_F64: return n * sizeof(GemmPtrs);
+    case STEP_REORDER: return n * sizeof(ReorderPtrs);
+    case STEP_OZ_GEMM: return n * sizeof(RGemm);
+    case STEP_OZ_SCALE:
+    case STEP_OZ_SPLIT:
+    case STEP_OZ_RECON: return n * sizeof(OzLeaf);
+    case STEP_CRT_SCALE:
+    case STEP_CRT_SPLIT:
+    case STEP_CRT_RECON: return sizeof(CrtMats);
+    case STEP_BB_PRE: return sizeof(BBPre);
+    case STEP_BB_POST: return sizeof(BBPost);
+    case STEP_BB_SPLIT_A: return sizeof(BBSplitA);
+    case STEP_BB_SPLIT_B: return sizeof(BBSplitB);
+    case STEP_FUSED_PRE: return sizeof(FusedPre);
+    case STEP_FUSED_POST: return sizeof(FusedPost);
+  }
+  return 0;  // segmented steps of batches: no size of their own
+}
+
+bool split_tables(Plan &plan, size_t window) {
+  const size_t consts = plan.oz_moduli ? sizeof(OzakiConsts) : 0;
+  std::vector<unsigned char> out;
+  std::map<size_t, size_t> here;  // this part's tables: old offset -> new
+  size_t used = 0;                // bytes of this part
+  const auto take = [&](size_t src, size_t bytes) {
+    const size_t dst = (used + 63) / 64 * 64;
+    used = dst + bytes;
+    out.resize(plan.parts.back().offset + used);
+    if (bytes) memcpy(&out[plan.parts.back().offset + dst], &plan.host_tables[src], bytes);
+    return dst;
+  };
+  const auto open = [&](size_t step) {
+    if (!plan.parts.empty()) plan.parts.back().bytes = used;
+    plan.parts.push_back({step, (out.size() + 63) / 64 * 64, 0});
+    out.resize(plan.parts.back().offset);
+    here.clear();
+    used = 0;
+    take(plan.oz_const, consts);
+  };
+  plan.parts.clear();
+  for (size_t i = 0; i < plan.steps.size(); i++) {
+    Step &st = plan.steps[i];
+    const size_t bytes = step_table_bytes(st);
+    if (bytes == 0 || (consts + 63) / 64 * 64 + bytes > window) return false;
+    if (i == 0) open(0);
+    if (!here.count(st.table)) {
+      if ((used + 63) / 64 * 64 + bytes > window) open(i);
+      here[st.table] = take(st.table, bytes);
+    }
+    st.table = here[st.table];
+  }
+  if (!plan.parts.empty()) plan.parts.back().bytes = used;
+  plan.host_tables = std::move(out);
+  plan.oz_const = 0;
+  return true;
+}
+
+hipError_t run_steps(const Plan &plan, hipStream_t s, size_t first, size_t last) {
+  for (size_t i = first; i < std::min(last, plan.steps.size()); i++) {
+    hipError_t e = run_one(plan, plan.steps[i], s);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -90,6 +90,12 @@ struct PlanKey {
   bool operator==(const PlanKey &o) const;
 };
 
+// the tables of the steps from first_step on (to the next part's), which start
+// with the split-mode constants; the steps' offsets are from the part's start
+struct TablePart {
+  size_t first_step, offset, bytes;
+};
+
 struct Plan {
   PlanKey key;
   std::vector<Step> steps;
@@ -108,6 +114,8 @@ struct Plan {
   int oz_moduli = 0;
   // residue mode: host copies of the residue descriptions (Step.aux indexes)
   std::vector<CrtMats> crt_host;
+  // split_tables: host_tables in parts (empty: as a whole)
+  std::vector<TablePart> parts;
   // batched plans: the key of every item
   std::string batch_key;
 };
@@ -141,8 +149,18 @@ int build_plan(Plan &plan, const double *A, const double *B, double *C,
 int build_batch_plan(Plan &plan, const std::vector<BatchItem> &items, int mode, int moduli,
                      void *work_base, int tile = 0, size_t merge_budget = 0);
 
-// Enqueue every step of the plan on `s` (no graph).
-hipError_t run_steps(const Plan &plan, hipStream_t s);
+// Bytes of a step's table (not the segmented steps of batches).
+size_t step_table_bytes(const Step &st);
+
+// Lay host_tables out in parts of at most `window` bytes (Plan::parts), for a
+// plan whose tables do not fit the device memory they may take: each part is
+// copied to the window before its steps run.  False: some step's table does not
+// fit by itself.
+bool split_tables(Plan &plan, size_t window);
+
+// Enqueue the steps [first, last) of the plan on `s` (no graph).
+hipError_t run_steps(const Plan &plan, hipStream_t s, size_t first = 0,
+                     size_t last = ~(size_t)0);
 
 // Same, with a HIP event pair around every step; adds each step's elapsed
 // milliseconds to ms[timer of its kind] and counts launches in n[].  Waits
