@@ -799,9 +799,12 @@ MergeKey merge_key(const Plan &plan, const Step &st) {
       break;
     case STEP_OZ_GEMM: {
       // INT8 products below the 256 tiles share a launch by block tile (that
-      // of a launch which fills the device); those on 256 tiles keep their own
+      // of a launch which fills the device); those on 256 tiles keep their own,
+      // and so do products in interleaved segments (all of a step or none),
+      // which no other kernel writes
       const int bt = residue_block_tile((int)st.n, st.levels, st.tile, 1LL << 24);
-      if (st.bs == 0 && bt < 256) k = {STEP_MULTI_RGEMM, bt, 0};
+      const RGemm *g = reinterpret_cast<const RGemm *>(&plan.host_tables[st.table]);
+      if (st.bs == 0 && bt < 256 && g->cseg == 128) k = {STEP_MULTI_RGEMM, bt, 0};
       break;
     }
     case STEP_CRT_SCALE:
