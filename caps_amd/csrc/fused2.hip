@@ -447,10 +447,12 @@ hipError_t launch_bb_split_b(const BBSplitB *P, long long q, int m0, int nmod,
 
 // One block of the fused pass fills a CU and does its tile's moduli one after
 // another, so its time goes in rounds of a tile per CU, 75 to 100 us each for 14
-// moduli; the separate split and pre-additions take 0.48 us per tile.  Measured
-// (us, fused and separate): n = 512 74 and 14, 1024 74 and 21, 2048 87 and 62,
-// 2560 (200 tiles) 100 and 93, 3072 (288) 165 and 146, 3584 (392) 173 and 185,
-// 4096 (512) 193 and 245, 5120 (800) 362 and 383.
+// moduli; the separate split and pre-additions take 0.48 us per tile.  Measured,
+// the whole multiply (us, fused and separate): n = 2560 (200 tiles) 537 and 543,
+// 3072 (288) 824 and 813, 3584 (392) 1195 and 1238, 4096 (512) 1424 and 1503, 4608
+// (648) 2001 and 2081, 5120 (800) 2600 and 2685, 5632 (968) 3374 and 3484.  Below,
+// the passes by themselves: n = 512 74 and 14, 1024 74 and 21, 2048 (128) 87 and
+// 62; so timed, n = 2560 is 100 and 93, but its multiply is faster fused.
 bool bb_split_a_pays(long long q) {
   const long long tiles = q / (SA_R * SA_C), cus = device_cu_count();
   return tiles > 195 * ((tiles + cus - 1) / cus);
