@@ -690,7 +690,10 @@ static int layout_host(const double *src, double *dst, const caps_desc *desc, bo
                                           desc->bs, ss)
                          : launch_from_caps(s.stage[0], s.stage[1], desc->lda, desc->nrec,
                                             desc->bs, ss);
-  if (e != hipSuccess) return fail(CAPS_EHIP, "layout kernel: %s", hipGetErrorString(e));
+  if (e != hipSuccess) {
+    hipStreamSynchronize(ss);  // the pinned ring is the next call's
+    return fail(CAPS_EHIP, "layout kernel: %s", hipGetErrorString(e));
+  }
   HIP_TRY(s.host_copy.down({s.stage[1], dst, n2 * sizeof(double)}, ss));
   return CAPS_OK;
 }
