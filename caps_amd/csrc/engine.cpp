@@ -455,9 +455,9 @@ struct Builder {
     plan.additions += 15LL * 4 * e2 + 7LL * 15 * e2;
     // plain sub-blocks passed by pointer: level-1 / level-2 operand -> quadrant
     const int quadA[7] = {0, 2, -1, -1, -1, -1, 3};  // T1 = A11, T2 = A12, T7 = A22
-    const int quadB[7] = {0, 1, -1, -1, -1, 3, -1};  // S1 = B11, S2 = B21, S6 = B22
-    const bool fused_b = crt->fused_b, fused_a = crt->fused_a;
-    Mat LA = alloc_mats(fused_a ? 49 : 40, q), LB = alloc_mats(fused_b ? 49 : 40, q),
+    const bool fused_a = crt->fused_a;
+    // (fused_b does not hold only where pad = false counts sizes)
+    Mat LA = alloc_mats(fused_a ? 49 : 40, q), LB = alloc_mats(crt->fused_b ? 49 : 40, q),
         P2 = alloc_mats(49, q);
     // residue products written by the leaf GEMM itself (no level between) on
     // its 256-tile kernel: the 49 products of a modulus interleave in 128-byte
@@ -467,25 +467,15 @@ struct Builder {
                      residue_gemm_segmented(sub, cutoff, tile, mode == CAPS_MODE_CRT_BF16,
                                           49LL * moduli);
     const long long pstep = seg ? 128 : q, cseg = seg ? 49 * 128 : 128;
-    // the kernels address the 40 written operands of a side as out + k * step
-    // (k counts the non-plain (i, j) in order) and product (i, j) as
-    // q + (7 i + j) * step
-    BBPre pre{};
-    pre.in[0] = pb.A.p;
-    pre.in[1] = pb.B.p;
-    pre.sin[0] = pb.A.ps;
-    pre.sin[1] = pb.B.ps;
-    pre.out[0] = LA.p;
-    pre.out[1] = LB.p;
-    pre.sout[0] = LA.ps;
-    pre.sout[1] = LB.ps;
-    pre.step = q;
+    // the kernels address A's 40 written operands as out + k * step (k counts
+    // the non-plain (i, j) in order) and product (i, j) as q + (7 i + j) * step
+    const BBPre pre{pb.A.p, LA.p, q, pb.A.ps, LA.ps};
     std::vector<Prob> next(49);
-    int ka = 0, kb = 0;
+    int ka = 0;
     for (int i = 0; i < 7; i++)
       for (int j = 0; j < 7; j++) {
         const int k = 7 * i + j;
-        Mat a, b;
+        Mat a;
         if (fused_a) {
           a = at(LA, (long long)k * q);
         } else if (bb_plain(0, i) && bb_plain(0, j)) {
@@ -493,18 +483,11 @@ struct Builder {
         } else {
           a = at(LA, (long long)ka++ * q);
         }
-        if (fused_b) {
-          b = at(LB, (long long)k * q);
-        } else if (bb_plain(1, i) && bb_plain(1, j)) {
-          b = at(pb.B, (4 * quadB[i] + quadB[j]) * q);
-        } else {
-          b = at(LB, (long long)kb++ * q);
-        }
-        next[k] = {a, b, {P2.p + k * pstep, P2.ps}, cseg};
+        next[k] = {a, at(LB, (long long)k * q), {P2.p + k * pstep, P2.ps}, cseg};
       }
-    if (ka != (fused_a ? 0 : 40) || kb != (fused_b ? 0 : 40)) broken = true;
+    if (ka != (fused_a ? 0 : 40)) broken = true;
     ensure_consts();
-    if (fused_b) {
+    if (crt->fused_b) {
       BBSplitB sp{};
       sp.B = crt->B;
       sp.out = reinterpret_cast<int8_t *>(LB.p);
@@ -526,7 +509,7 @@ struct Builder {
       sp.nrec2 = crt->nrec - 2;
       push(STEP_BB_SPLIT_A, 1, 1, q, crt->m, add_table(&sp, sizeof(sp)));
     } else {
-      push(STEP_BB_PRE, 1, 1, q, 0, add_table(&pre, sizeof(pre)), fused_b ? 1 : 0);
+      push(STEP_BB_PRE, 1, 1, q, 0, add_table(&pre, sizeof(pre)));
     }
     rec(next, sub, nrec - 2, depth + 2);
     BBPost post{};
@@ -665,7 +648,7 @@ hipError_t run_one(const Plan &plan, const Step &st, hipStream_t s) {
                                st.n, plan.oz_moduli, st.vec2 != 0, kc, s);
     case STEP_BB_PRE:
       return launch_bb_pre(reinterpret_cast<const BBPre *>(tb + st.table), st.n,
-                           plan.oz_moduli, kc, s, st.vec2 != 0);
+                           plan.oz_moduli, kc, s);
     case STEP_BB_SPLIT_B:
       return launch_bb_split_b(reinterpret_cast<const BBSplitB *>(tb + st.table), st.n, st.bs,
                                plan.oz_moduli, kc, s);

@@ -116,8 +116,6 @@ struct Plan {
   std::vector<CrtMats> crt_host;
   // split_tables: host_tables in parts (empty: as a whole)
   std::vector<TablePart> parts;
-  // batched plans: the key of every item
-  std::string batch_key;
 };
 
 // one independent multiply of a batched call

@@ -16,15 +16,16 @@ __host__ __device__ constexpr bool bb_plain(int side, int t) {
   return side == 0 ? (t == 0 || t == 1 || t == 6) : (t == 0 || t == 1 || t == 5);
 }
 
-// pre-additions of two 'b' levels for both operands of one sub-problem
+// pre-additions of two 'b' levels for A of one sub-problem (B's are fused with
+// its split: BBSplitB)
 struct BBPre {
-  const void *in[2];      // A (side 0) and B (side 1): 16 depth-2 sub-blocks of q elements,
-                          // sub-block (a, b) at element (4a + b) * q
-  void *out[2];           // the 40 written depth-2 operands (i, j) = operand j of level-1
+  const void *in;         // 16 depth-2 sub-blocks of q elements, sub-block (a, b) at element
+                          // (4a + b) * q
+  void *out;              // the 40 written depth-2 operands (i, j) = operand j of level-1
                           // operand i, not plain, in (i, j) order, one every `step` bytes
   long long step;         // bytes between consecutive operands (q elements)
-  long long sin[2];       // plane strides (bytes)
-  long long sout[2];
+  long long sin;          // plane strides (bytes)
+  long long sout;
 };
 
 // post-combinations of two 'b' levels for one sub-problem
@@ -72,9 +73,9 @@ struct BBSplitA {
 };
 
 // q: positions of a depth-2 sub-block, with the leaves' pitch.
-// q % 4 == 0.  a_only: side B is produced by launch_bb_split_b instead.
+// q % 4 == 0
 hipError_t launch_bb_pre(const BBPre *d_P, long long q, int nmod,
-                         const OzakiConsts *d_consts, hipStream_t s, bool a_only = false);
+                         const OzakiConsts *d_consts, hipStream_t s);
 // m0: host copy of the table's leaf size; q < 2^31
 hipError_t launch_bb_split_b(const BBSplitB *d_P, long long q, int m0, int nmod,
                              const OzakiConsts *d_consts, hipStream_t s);

@@ -2,10 +2,9 @@
 // passes (FP64: fused_f64.hip).
 //
 // Pre-additions: the 16 depth-2 sub-blocks of A (of B) at one position give
-// all 49 depth-2 operands T_j(T_i) (S_j(S_i)) at that position; one launch
+// all 49 depth-2 operands T_j(T_i) (S_j(S_i)) at that position; of A one launch
 // reads each input element once and writes the 40 operands that are not
-// plain sub-blocks (the 9 with i, j in {T1, T2, T7} / {S1, S2, S6} are passed
-// by pointer).  Post-combinations: the 49 depth-2 products at one position
+// plain sub-blocks (the 9 with i, j in {T1, T2, T7} are passed by pointer).  Post-combinations: the 49 depth-2 products at one position
 // give C's 16 depth-2 sub-blocks.  The expression trees are exactly those of
 // two strassenBFS levels (multiply.cpp:272, 277, 195-210) applied one after
 // the other; every step is exact modulo m_l.
@@ -58,17 +57,16 @@ __device__ __forceinline__ void level_ops(int side, const V (&q)[4], V (&o)[7]) 
 }
 
 // ---------------------------------------------------------------- residue pre
-// thread: 4 consecutive positions (one 4-byte word per operand); grid.y:
-// modulus; one instantiation per side.  Depth-2 values are sums of at most 16
+// A; thread: 4 consecutive positions (one 4-byte word per operand); grid.y:
+// modulus.  Depth-2 values are sums of at most 16
 // residues: |x| <= 2048, reduced by mod_k.  Offsets within a plane are 32-bit
 // (q < 2^31).
-template <int SIDE>
 __global__ __launch_bounds__(T) void bb_pre_res_kernel(const BBPre *__restrict__ P, long long q,
                                                        const OzakiConsts *__restrict__ kc) {
   const int l = blockIdx.y;
   const int mi = kc->m[l], c22 = kc->c22[l];
-  const char *in = reinterpret_cast<const char *>(P->in[SIDE]) + l * P->sin[SIDE];
-  char *obase = reinterpret_cast<char *>(P->out[SIDE]) + l * P->sout[SIDE];
+  const char *in = reinterpret_cast<const char *>(P->in) + l * P->sin;
+  char *obase = reinterpret_cast<char *>(P->out) + l * P->sout;
   const long long step = P->step;
   const unsigned qq = (unsigned)q, n4 = (unsigned)(q >> 2);
   for (unsigned u = blockIdx.x * T + threadIdx.x; u < n4; u += gridDim.x * T) {
@@ -85,7 +83,7 @@ __global__ __launch_bounds__(T) void bb_pre_res_kernel(const BBPre *__restrict__
         int qv[4], o[7];
 #pragma unroll
         for (int a = 0; a < 4; a++) qv[a] = (int)__builtin_amdgcn_sbfe(w[a][b], 8 * h, 8);
-        level_ops(SIDE, qv, o);
+        level_ops(0, qv, o);
 #pragma unroll
         for (int i = 0; i < 7; i++) l1[h][i][b] = o[i];
       }
@@ -94,10 +92,10 @@ __global__ __launch_bounds__(T) void bb_pre_res_kernel(const BBPre *__restrict__
     for (int i = 0; i < 7; i++) {
       int o[4][7];
 #pragma unroll
-      for (int h = 0; h < 4; h++) level_ops(SIDE, l1[h][i], o[h]);
+      for (int h = 0; h < 4; h++) level_ops(0, l1[h][i], o[h]);
 #pragma unroll
       for (int j = 0; j < 7; j++) {
-        if (bb_plain(SIDE, i) && bb_plain(SIDE, j)) continue;
+        if (bb_plain(0, i) && bb_plain(0, j)) continue;
         const unsigned v = pack4_lo(mod_k(o[0][j], c22, mi), mod_k(o[1][j], c22, mi),
                                     mod_k(o[2][j], c22, mi), mod_k(o[3][j], c22, mi));
         __builtin_nontemporal_store(v, (guint *)(obase + k * step + 4 * u));
@@ -419,11 +417,10 @@ unsigned blocks_for(long long units, int per_grid) {
 }  // namespace
 
 hipError_t launch_bb_pre(const BBPre *P, long long q, int nmod, const OzakiConsts *kc,
-                         hipStream_t s, bool a_only) {
+                         hipStream_t s) {
   if (q % 4 || q >= (1LL << 31)) return hipErrorInvalidValue;
   dim3 g(blocks_for(q / 4, 2 * nmod), nmod);
-  hipLaunchKernelGGL(bb_pre_res_kernel<0>, g, dim3(T), 0, s, P, q, kc);
-  if (!a_only) hipLaunchKernelGGL(bb_pre_res_kernel<1>, g, dim3(T), 0, s, P, q, kc);
+  hipLaunchKernelGGL(bb_pre_res_kernel, g, dim3(T), 0, s, P, q, kc);
   return hipGetLastError();
 }
 

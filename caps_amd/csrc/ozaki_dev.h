@@ -93,17 +93,6 @@ __device__ __forceinline__ int sym_residue(double x, int mi, double inv, int c22
   return mod_k((int)r, c22, mi);
 }
 
-// residue of a small integer (|x| < 2^22) modulo mi in [-mi/2, mi/2]: the
-// FP32 quotient estimate x * inv is within |x/mi| 2^-23 < 1 / (2 mi) of x / mi,
-// which is never a half-integer for odd mi (2x = odd * mi is impossible), so
-// rint finds the nearest integer; for mi = 256 (exact inverse) a tie gives
-// +-128, the same INT8 value after the wrap.  Every step is exact: integers
-// below 2^24 in FP32.
-__device__ __forceinline__ int mod_small(int x, float mf, float inv) {
-  const float xf = (float)x;
-  return (int)fmaf(-rintf(xf * inv), mf, xf);
-}
-
 // added to a float |k| < 2^22, rounds it to the nearest integer, which is then
 // in the low 22 bits of the sum (0x4B400000 + k)
 constexpr float ROUND_MAGIC = 12582912.0f;  // 1.5 * 2^23
