@@ -114,6 +114,18 @@ bool by_graph(const Plan &p, const caps_opts *o) {
          p.steps.size() > MAX_DIRECT_STEPS && p.steps.size() <= MAX_GRAPH_STEPS;
 }
 
+// is the caller recording `stream` into a graph of its own?  (The plan's kernels
+// go there: a graph launched there would record nothing.)
+bool under_capture(hipStream_t stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (!stream) return false;
+  if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return st == hipStreamCaptureStatusActive;
+}
+
 int ensure_device_locked(State &s) {
   int dev = 0;
   HIP_TRY(hipGetDevice(&dev));
@@ -146,14 +158,18 @@ void free_plan(Plan &p) {
   p.d_tables = p.d_work = nullptr;
 }
 
-void evict_locked(State &s, size_t keep) {
-  if (s.plans.size() <= keep) return;
+// frees the plans used longest ago, to `keep` of those that no caller's graph
+// holds; `all`: those too
+void evict_locked(State &s, size_t keep, bool all = false) {
+  const auto held = [&](const std::unique_ptr<Plan> &p) { return p->recorded && !all; };
+  const size_t n = (size_t)std::count_if(s.plans.begin(), s.plans.end(), held);
+  if (s.plans.size() - n <= keep) return;
   hipDeviceSynchronize();
   std::sort(s.plans.begin(), s.plans.end(),
-            [](const std::unique_ptr<Plan> &a, const std::unique_ptr<Plan> &b) {
-              return a->last_use > b->last_use;
+            [&](const std::unique_ptr<Plan> &a, const std::unique_ptr<Plan> &b) {
+              return held(a) != held(b) ? held(a) : a->last_use > b->last_use;
             });
-  while (s.plans.size() > keep) {
+  while (s.plans.size() - n > keep) {
     free_plan(*s.plans.back());
     s.plans.pop_back();
   }
@@ -416,7 +432,8 @@ int multiply_device_locked(State &s, const double *dA, const double *dB, double 
                        plan);
   if (rc) return rc;
   const bool timed = opts && (opts->flags & CAPS_FLAG_TIMERS);
-  const bool use_graph = by_graph(*plan, opts);
+  const bool recording = under_capture(stream), use_graph = !recording && by_graph(*plan, opts);
+  plan->recorded = plan->recorded || recording;
   if (timed) {
     hipError_t e = run_steps_timed(*plan, stream, s.timers_ms, s.timed);
     if (e != hipSuccess) return fail(CAPS_EHIP, "timed launch: %s", hipGetErrorString(e));
@@ -590,18 +607,21 @@ int caps_multiply_device_noalloc(const double *dA, const double *dB, double *dC,
     plan->d_tables = base;
     plan->d_work = base + toff;
     plan->last_use = ++s.clock;
-    // host memory only; keep the 16 most recent
-    if (s.host_plans.size() >= 16) {
+    // host memory only; keep the 16 most recent of those that no caller's graph
+    // reads
+    const auto held = [](const std::unique_ptr<Plan> &p) { return p->recorded; };
+    if (s.host_plans.size() - std::count_if(s.host_plans.begin(), s.host_plans.end(), held) >= 16) {
       auto oldest = std::min_element(
           s.host_plans.begin(), s.host_plans.end(),
-          [](const std::unique_ptr<Plan> &a, const std::unique_ptr<Plan> &b) {
-            return a->last_use < b->last_use;
+          [&](const std::unique_ptr<Plan> &a, const std::unique_ptr<Plan> &b) {
+            return held(a) != held(b) ? held(b) : a->last_use < b->last_use;
           });
       s.host_plans.erase(oldest);
     }
     p = plan.get();
     s.host_plans.push_back(std::move(plan));
   }
+  p->recorded = p->recorded || under_capture(hs);
   // the tables go to the front of the scratch in stream order (a pageable
   // source is read before the call returns), then their steps run eagerly
   for (size_t i = 0; i < p->parts.size(); i++) {
@@ -845,7 +865,9 @@ int caps_multiply_batch_device(int count, const double *const *dA, const double 
     if (rc) rc = make(items, 0);  // exactly the levels asked for
     if (rc) return rc;
   }
-  const bool use_graph = by_graph(*plan, opts);
+  const bool recording = under_capture((hipStream_t)stream);
+  const bool use_graph = !recording && by_graph(*plan, opts);
+  plan->recorded = plan->recorded || recording;
   if (opts && (opts->flags & CAPS_FLAG_TIMERS)) {
     hipError_t e = run_steps_timed(*plan, (hipStream_t)stream, s.timers_ms, s.timed);
     if (e != hipSuccess) return fail(CAPS_EHIP, "timed launch: %s", hipGetErrorString(e));
@@ -1006,7 +1028,7 @@ int caps_tune_load(const char *path) {
 int caps_release(void) {
   State &s = st();
   std::lock_guard<std::mutex> g(s.mu);
-  evict_locked(s, 0);
+  evict_locked(s, 0, true);
   s.host_plans.clear();
   for (auto &p : s.stage)
     if (p) {

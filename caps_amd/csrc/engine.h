@@ -109,6 +109,7 @@ struct Plan {
   long long additions = 0, multiplications = 0, leaves = 0;
   std::string exec_pattern;
   unsigned long long last_use = 0;
+  bool recorded = false;  // a caller's graph holds its tables and workspace
   // split-mode constants (moduli, CRT weights), device copy in d_tables
   size_t oz_const = 0;
   int oz_moduli = 0;

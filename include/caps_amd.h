@@ -92,7 +92,10 @@ typedef struct caps_opts {
  * descriptor, pattern, options and stream (default on, for plans of more than
  * a few launches: those are launched directly).  A cached plan owns one device
  * workspace and belongs to one stream: calls on different streams never share
- * a workspace, and calls on one stream run in stream order. */
+ * a workspace, and calls on one stream run in stream order.
+ * A call on a stream under capture (whose plan an earlier call there has built)
+ * records the plan's kernels, with its workspace: the plan is then kept until
+ * caps_release, and replays of that graph must not overlap other uses of it. */
 #define CAPS_FLAG_NO_GRAPH 1
 /* Force the reference's automatic rule when pattern == NULL (DFS at every
  * level on one process, multiply.cpp:43-66) instead of the planner's choice. */

@@ -27,12 +27,13 @@ def count(what):
     return fake.fake_count(what.encode())
 def opts(mode, moduli=0, flags=0, cutoff=0):
     return caps_amd.Options(mode, moduli, flags, cutoff)
-def call(n, r, pattern, mode=FP64, bs=1, moduli=0, flags=0, at=1, entry=None, cutoff=0):
+def call(n, r, pattern, mode=FP64, bs=1, moduli=0, flags=0, at=1, entry=None, cutoff=0,
+         stream=None):
     d, o = caps_amd.MatDescriptor.one_device(n, r, bs), opts(mode, moduli, flags, cutoff)
     p = [(at << 44) + (k << 40) for k in range(3)]
     f = entry or lib.caps_multiply_device
-    return f(*p, ctypes.byref(d), pattern.encode() if pattern else None, ctypes.byref(o), None)
-def batch(shapes, mode=FP64, at=1):
+    return f(*p, ctypes.byref(d), pattern.encode() if pattern else None, ctypes.byref(o), stream)
+def batch(shapes, mode=FP64, at=1, stream=None):
     k = len(shapes)
     ptr = [(ctypes.c_void_p * k)(*[(at << 44) + (s << 41) + (i << 32) for i in range(k)])
            for s in range(3)]
@@ -43,7 +44,7 @@ def batch(shapes, mode=FP64, at=1):
     return lib.caps_multiply_batch_device(k, *[ctypes.cast(x, ctypes.c_void_p) for x in ptr],
                                           ctypes.cast(descs, ctypes.c_void_p),
                                           ctypes.cast(pats, ctypes.c_void_p),
-                                          ctypes.cast(os_, ctypes.c_void_p), None)
+                                          ctypes.cast(os_, ctypes.c_void_p), stream)
 def error():
     return lib.caps_last_error().decode()
 def peak_bytes():

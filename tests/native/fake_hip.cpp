@@ -21,6 +21,10 @@ struct Fake {
   std::string fail_launch;           // kernels whose name contains it are not launched
   long long mallocs = 0, frees = 0, device_syncs = 0, stream_syncs = 0, copies = 0;
   long long copy_bytes = 0;
+  long long graph_launches = 0;
+  const void *copy_src = nullptr;    // of the last asynchronous copy
+  size_t copy_n = 0;
+  bool capturing = false;            // every stream but the default one
   std::map<const void *, std::string> names;
   std::vector<const void *> launched;
   dim3 grid, block;
@@ -50,6 +54,11 @@ void fake_set_free(size_t bytes) { f().free = bytes; }
 size_t fake_free() { return f().free; }
 void fake_set_malloc_limit(size_t bytes) { f().malloc_limit = bytes; }
 void fake_fail_launch(const char *name) { f().fail_launch = name; }
+const void *fake_copy_src(size_t *n) {
+  *n = f().copy_n;
+  return f().copy_src;
+}
+void fake_set_capturing(int yes) { f().capturing = yes != 0; }
 long long fake_count(const char *what) {
   const std::string w = what;
   if (w == "malloc") return f().mallocs;
@@ -57,6 +66,7 @@ long long fake_count(const char *what) {
   if (w == "device_sync") return f().device_syncs;
   if (w == "stream_sync") return f().stream_syncs;
   if (w == "copy") return f().copies;
+  if (w == "graph_launch") return f().graph_launches;
   if (w == "copy_bytes") return f().copy_bytes;
   long long n = 0;  // launches of kernels whose name contains it
   for (const void *k : f().launched) n += f().names[k].find(w) != std::string::npos;
@@ -131,8 +141,10 @@ hipError_t hipMemcpy(void *, const void *, size_t n, hipMemcpyKind) {
   f().copy_bytes += (long long)n;
   return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *, const void *, size_t n, hipMemcpyKind, hipStream_t) {
+hipError_t hipMemcpyAsync(void *, const void *src, size_t n, hipMemcpyKind, hipStream_t) {
   f().copies++;
+  f().copy_src = src;
+  f().copy_n = n;
   f().copy_bytes += (long long)n;
   return hipSuccess;
 }
@@ -196,6 +208,13 @@ hipError_t hipGraphInstantiate(hipGraphExec_t *g, hipGraph_t, hipGraphNode_t *, 
 }
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) {
+  f().graph_launches++;
+  return hipSuccess;
+}
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *st) {
+  *st = f().capturing && s ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
 
 }  // extern "C"

@@ -122,3 +122,54 @@ for count_, n, r in ((3, 256, 4), (8, 544, 5)):
         assert peak(budget, 3 + k) <= 8 * budget, (n, r, budget)
     caps_amd.release()
 """)
+
+
+def test_plans_recorded_into_a_graph_are_kept():
+    """A call on a stream under capture records its kernels, which hold the plan's
+    workspace and tables: that plan goes with release() alone, the others by age
+    as before."""
+    run("""
+S = 4096
+cases = [dict(n=512, r=2, pattern="bb"), dict(n=392, r=3, pattern="dbd", bs=7, flags=8)]
+caps_amd.set_available_memory(1)  # 'd' as asked: more than 16 launches
+for c in cases:
+    assert call(**c, stream=S) == 0, error()
+shapes = [(256, 1, "b"), (320, 1, "d")]
+assert batch(shapes, stream=S) == 0, error()
+fake.fake_set_capturing(1)
+for c in cases:
+    before = count("kernel"), count("graph_launch"), count("malloc")
+    assert call(**c, stream=S) == 0, error()
+    assert count("kernel") > before[0]
+    assert (count("graph_launch"), count("malloc")) == before[1:]
+assert batch(shapes, stream=S) == 0, error()
+fake.fake_set_capturing(0)
+held = 256 * GiB - fake.fake_free()
+for at in range(2, 62):  # 60 other plans
+    assert call(256, 2, "bb", at=at) == 0, error()
+mallocs = count("malloc")
+for c in cases:
+    assert call(**c, stream=S) == 0, error()
+assert batch(shapes, stream=S) == 0 and count("malloc") == mallocs
+for at in range(40, 62):  # the newest others are still there
+    assert call(256, 2, "bb", at=at) == 0 and count("malloc") == mallocs
+assert call(256, 2, "bb", at=2) == 0 and count("malloc") > mallocs
+fake.fake_set_free(1 * MiB)  # what is short of memory takes the others only
+assert call(4096, 2, "bb", at=70) == 3
+mallocs = count("malloc")
+assert call(**cases[0], stream=S) == 0 and count("malloc") == mallocs
+caps_amd.release()
+assert call(**cases[0], stream=S) == 0 and count("malloc") > mallocs
+# without allocation the graph holds the host's tables
+noalloc = lib.caps_multiply_device_noalloc
+fake.fake_copy_src.restype = ctypes.c_void_p
+fake.fake_set_capturing(1)
+assert call(512, 4, "dddd", stream=S, entry=noalloc) == 0, error()
+n = ctypes.c_size_t()
+src = fake.fake_copy_src(ctypes.byref(n))
+tables = ctypes.string_at(src, n.value)
+fake.fake_set_capturing(0)
+for at in range(2, 40):
+    assert call(512, 4, "dddd", at=at, stream=S, entry=noalloc) == 0, error()
+assert ctypes.string_at(src, n.value) == tables
+""")
